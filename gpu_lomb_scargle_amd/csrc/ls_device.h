@@ -12,6 +12,13 @@
 
 namespace lsamd {
 
+// Coarse-grid sweep, per object: the mode (0: direct) and the centre of its
+// time span.
+struct InterpObj {
+    double tc;
+    uint32_t mode, unused;
+};
+
 struct SweepArgs {
     const uint64_t *offsets;
     const uint32_t *order;
@@ -44,6 +51,14 @@ struct SweepArgs {
     uint4 *colfac;
     uint4 *rowfac;
     float *obj_ys;  // per object: y scale, weight scale
+    // coarse-grid sweep (null: every object direct): the objects' modes, the
+    // interpolation operands, workgroups per object, and the chunks to sweep
+    // again directly (bit c % 64 of word c / 64; null: the main pass)
+    const InterpObj *obj_ip;
+    uint4 *ip_tab;
+    uint32_t ip_items;
+    uint32_t cand_words, cand_split;  // words per object; workgroups per object of the direct passes
+    uint64_t *cand;
 };
 
 typedef void (*SweepFn)(SweepArgs);
@@ -249,40 +264,6 @@ __device__ __forceinline__ void block_top3(Peaks &L, double (*s_p)[kPeaks],
             L.i[1] = L.i[2];
             L.p[2] = 0.0;
             L.i[2] = 0u;
-        }
-    }
-}
-
-// Merge the lists of a whole workgroup; the result is valid in thread 0.
-template <int T>
-__device__ __forceinline__ void block_peaks(Peaks &L, double (*s_p)[kPeaks],
-                                            uint32_t (*s_i)[kPeaks]) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        double op[kPeaks];
-        uint32_t oi[kPeaks];
-#pragma unroll
-        for (int r = 0; r < kPeaks; ++r) {
-            op[r] = __shfl_xor(L.p[r], off, 64);
-            oi[r] = __shfl_xor(L.i[r], off, 64);
-        }
-#pragma unroll
-        for (int r = 0; r < kPeaks; ++r) peaks_insert(L, op[r], oi[r]);
-    }
-    if constexpr (T > 64) {
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        if (lane == 0) {
-#pragma unroll
-            for (int r = 0; r < kPeaks; ++r) {
-                s_p[wave][r] = L.p[r];
-                s_i[wave][r] = L.i[r];
-            }
-        }
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            for (int w = 1; w < T / 64; ++w)
-#pragma unroll
-                for (int r = 0; r < kPeaks; ++r) peaks_insert(L, s_p[w][r], s_i[w][r]);
         }
     }
 }

@@ -39,7 +39,7 @@ struct Workspace {
     size_t rec_t = 0;       // double[n]  split: t
     size_t rec_a = 0;       // float4[n]  split: {y or sqrt(w)(y-ybar), -sin step or sqrt(w), cos, sin step}
     size_t rec_n = 0;       // float[n]   split generalized: -sin step
-    size_t rec_r = 0;       // double2[n] split: {cos step, sin step}
+    size_t rec_r = 0;       // double2[n] split: {cos step, sin step}; coarse-grid sweep: {t - tc, 1/Phi}
     // per (object, chunk) peak partials
     size_t part_pow = 0;    // double[K*chunks*topk]
     size_t part_idx = 0;    // uint32[K*chunks*topk]
@@ -48,6 +48,12 @@ struct Workspace {
     size_t obj_ys = 0;      // float[2K]  matrix-core tile: power-of-two y and weight scales
     size_t colfac = 0;      // matrix-core tile: column-factor fragments, 8 (12 generalized) KiB per 16 observations
     size_t rowfac = 0;      // matrix-core tile: row-step phasors, 4 KiB per 16 observations
+    // coarse-grid sweep (interp): modes per object, interpolation operands,
+    // marked chunks
+    bool interp = false;
+    size_t obj_ip = 0;      // InterpObj[K]
+    size_t ip_tab = 0;
+    size_t cand = 0;        // uint64[K * ceil(chunks / 64)]
     uint32_t chunks = 0;
     uint32_t slices = 1;    // observation slices per (object, chunk)
     Tile tile{};

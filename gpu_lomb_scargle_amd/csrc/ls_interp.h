@@ -1,0 +1,71 @@
+// Modes of the coarse-grid sweep (ls_sweep_interp.hip), shared with the
+// statistics and record kernels that choose a mode per object (ls_sweep.hip).
+//
+// A mode has a coarse step of h bins and result rows of m coarse steps (h m
+// <= 32 bins, one lane each).  W = 8 taps at an oversampling of at least
+// kIpSigma = 1.95 keep the aliasing at 2e-8 and leave the rounding, which at
+// 1.95 is no larger than the direct sums': emulated over light curves of 30 to
+// 700 observations, worst power 7.3e-6 (bins of at least 1e-3 of the peak)
+// against 7.7e-6; W = 7 reaches 1.5e-5, an oversampling of 1.45 with W = 10
+// 2.5e-5 (the observations at the ends of the span carry weights 1/Phi of 18
+// there, 2.9 at 1.95).  h = 5 is the grid of ten bins per resolution element.
+#pragma once
+
+#include "ls_device.h"
+
+namespace lsamd {
+
+namespace {
+
+constexpr int kIpModes = 6;
+constexpr int kIpTaps = 8;
+constexpr double kIpSigma = 1.95, kIpSigmaGen = 2.4;
+constexpr int kIpFrags = 8;           // column-factor fragments per 16 observations
+constexpr float kIpMargin = 1e-4f;    // ten times the form's error bound
+__host__ __device__ constexpr int ip_step(int mode) {
+    return mode == 1 ? 4 : mode == 2 ? 5 : mode == 3 ? 6 : mode == 4 ? 8 : mode == 5 ? 10 : 16;
+}
+__host__ __device__ constexpr int ip_per_row(int mode) { return 32 / ip_step(mode); }
+// rows of a workgroup: m rows + W - 1 <= 2048 points, a multiple of 32 where that loses less than a tile
+__host__ __device__ constexpr int ip_rows(int mode) {
+    return mode == 1 ? 255 : mode == 2 ? 320 : mode == 3 ? 408 : mode == 4 ? 510 : mode == 5 ? 672 : 1020;
+}
+__host__ __device__ constexpr int ip_taps(int) { return kIpTaps; }
+__host__ __device__ constexpr double ip_beta(int mode) {
+    return 3.14159265358979323846 * ip_taps(mode) * (1.0 - 1.0 / (2.0 * kIpSigma));
+}
+constexpr uint32_t kIpLeastBins = 255 * 32;  // bins per workgroup, smallest mode
+// Objects up to here (at most two 16-observation blocks) keep the direct sums,
+// those of at most 16 observations their FP64 ones: with 18 observations and
+// weights over a factor of 400 the worst bin reached 1.4e-5 (direct 1.0e-5).
+constexpr uint32_t kIpLeastObs = 24;
+// Below these the direct sums are sooner done (FP32, top-1, ten bins per
+// resolution element; direct / coarse, us): 400 objects x 20,000 bins, 1.4e9
+// terms, 152 / 170 standard and 288 / 260 generalized; 100 x 80,000, 1.4e9:
+// 131 / 130; 100 x 200,000, 3.4e9: 252 / 177 and 440 / 235; 4 x 500,000, 0.3e9:
+// 56 / 75.  A call that may not look at how many objects it sweeps takes the
+// coarse grid from 2^18 bins on, where a few objects lose ~25 us by it.
+constexpr uint32_t kIpMinFreqs = 8192;  // bins a workgroup takes, smallest mode
+constexpr double kIpMinTerms = 1.5e9;
+constexpr uint32_t kIpAloneFreqs = 1u << 18;
+constexpr uint32_t kIpMaxFreqs = 1u << 29;   // byte offsets of an object's row in 32 bits
+
+// 1 / Phi(xi) of a mode's window, Phi(0) = 1, at xi = h df t' cycles per
+// coarse step, |xi| <= 1 / (2 kIpSigma): s = sqrt(beta^2 - (pi W xi)^2) >= 17,
+// where sinh s = e^s / 2 to FP64.
+__device__ __forceinline__ double ip_inv_window(int mode, double xi) {
+    const double beta = ip_beta(mode), u = 3.14159265358979323846 * ip_taps(mode) * xi;
+    const double s = sqrt(beta * beta - u * u);
+    return s / beta * exp(beta - s);
+}
+
+}  // namespace
+
+// Kernels of the coarse-grid sweep, [variant].
+struct InterpEntry {
+    SweepFn fac, sweep;
+    int threads;
+};
+extern const InterpEntry kInterp[2];
+
+}  // namespace lsamd

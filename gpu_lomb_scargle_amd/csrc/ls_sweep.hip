@@ -45,6 +45,7 @@
 #include <string>
 
 #include "ls_device.h"
+#include "ls_interp.h"
 
 namespace lsamd {
 
@@ -61,6 +62,12 @@ struct StatsArgs {
     int precenter;       // plain generalized: shift = sum(w y)/sum(w), w=1/sqrt(dy)
     int split_gen;       // split generalized constants
     double *obj_shift, *obj_scale, *obj_gen;
+    float *obj_ys;       // matrix-core tile: power-of-two scales of y and the weights (null: not needed)
+    const void *t;       // matrix-core tile (rec_t): its records, and the object's mode of the
+    double *rec_t;       // coarse-grid sweep (obj_ip, else null)
+    double2 *rec_r;
+    InterpObj *obj_ip;
+    double df_rev;
 };
 
 struct RecArgs {
@@ -83,6 +90,9 @@ struct ReduceArgs {
     uint32_t *peak_index;
     void *peak_power, *peak_period;
     double pmin, pstep;        // period of bin i = 2 pi / (pmin + i*pstep)
+    const InterpObj *obj_ip;   // coarse-grid sweep: only the marked chunks of such objects count
+    const uint64_t *cand;
+    uint32_t cand_words;
 };
 
 // ---------------------------------------------------------------------------
@@ -154,65 +164,109 @@ __global__ void k_obj_stats(StatsArgs a) {
     }
 }
 
-__device__ __forceinline__ double wave_sum64(double v) {
+// Sums and maxima over a workgroup of T threads (a wavefront butterfly, then
+// the wavefronts' values in order), the same in every thread.
+template <int T, typename Op>
+__device__ __forceinline__ double block_fold(double v, double *s, Op op) {
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+    for (int off = 32; off >= 1; off >>= 1) v = op(v, __shfl_xor(v, off, 64));
+    if constexpr (T > 64) {
+        __syncthreads();  // the previous fold's values are read
+        if ((threadIdx.x & 63u) == 0u) s[threadIdx.x >> 6] = v;
+        __syncthreads();
+        v = s[0];
+        for (int w = 1; w < T / 64; ++w) v = op(v, s[w]);
+    }
     return v;
 }
 
-// The same statistics for the split forms, one wavefront per object: sums in
-// lane-strided order with a butterfly reduction (the split forms are not
-// bit-matched to the CPU path, and an object's sums no longer wait on one
-// thread's sequential loop over its observations).
-template <typename R>
-__global__ __launch_bounds__(64) void k_obj_stats_wave(StatsArgs a) {
-    const uint32_t k = blockIdx.x;
-    const uint32_t lane = threadIdx.x;
+// The same statistics for the split forms, one workgroup of T threads per
+// object: sums in thread-strided order with a butterfly reduction (the split
+// forms are not bit-matched to the CPU path, and an object's sums no longer
+// wait on one thread's sequential loop over its observations).  A thread
+// loads its first kHeld observations once and makes every pass over them from
+// registers.  T = 64, or 512 for an object swept alone in observation slices
+// (3555 observations: statistics and records 27 us in 64- and 256-thread
+// kernels of their own).
+// For the matrix-core tile it also writes the records: the time in FP64 and,
+// for objects in coarse mode, the time from the middle of the span and the
+// window's weight there.
+template <typename R, int T>
+__global__ __launch_bounds__(T) void k_obj_stats_split(StatsArgs a) {
+    constexpr int kHeld = 4;
+    __shared__ double s_fold[T / 64];
+    const uint32_t k = blockIdx.x, tid = threadIdx.x;
     const uint64_t b = a.offsets[k], e = a.offsets[k + 1];
-    const R *y = static_cast<const R *>(a.y);
-    const R *dy = static_cast<const R *>(a.dy);
-    const double nd = (double)(e - b);
+    const uint64_t n = e - b;
+    const R *y = static_cast<const R *>(a.y) + b;
+    const R *dy = static_cast<const R *>(a.dy) + (a.split_gen ? b : 0);
+    const R *t = static_cast<const R *>(a.t) + b;
+    const double nd = (double)n;
+    R hy[kHeld] = {}, hd[kHeld] = {}, ht[kHeld] = {};
+#pragma unroll
+    for (int q = 0; q < kHeld; ++q) {
+        const uint64_t i = tid + (uint64_t)q * T;
+        if (i < n) {
+            hy[q] = y[i];
+            if (a.split_gen) hd[q] = dy[i];
+            if (a.rec_t) ht[q] = t[i];
+        }
+    }
+    // f(i, y, dy, t) for the thread's observations in order
+    auto each = [&](auto f) {
+#pragma unroll
+        for (int q = 0; q < kHeld; ++q) {
+            const uint64_t i = tid + (uint64_t)q * T;
+            if (i < n) f(i, (double)hy[q], (double)hd[q], (double)ht[q]);
+        }
+        for (uint64_t i = tid + (uint64_t)kHeld * T; i < n; i += T)
+            f(i, (double)y[i], a.split_gen ? (double)dy[i] : 0.0, a.rec_t ? (double)t[i] : 0.0);
+    };
+    auto sum = [&](double v) { return block_fold<T>(v, s_fold, [](double p, double q) { return p + q; }); };
+    auto most = [&](double v) { return block_fold<T>(v, s_fold, [](double p, double q) { return fmax(p, q); }); };
     double scale = 1.0;
     if (a.normalize) {  // 2/(N sigma^2), sigma^2 the population variance
         double s = 0.0;
-        for (uint64_t i = b + lane; i < e; i += 64) s += (double)y[i];
-        const double mean = wave_sum64(s) / nd;
+        each([&](uint64_t, double yi, double, double) { s += yi; });
+        const double mean = sum(s) / nd;
         double s2 = 0.0;
-        for (uint64_t i = b + lane; i < e; i += 64) s2 += ((double)y[i] - mean) * ((double)y[i] - mean);
-        const double sigma2 = wave_sum64(s2) / nd;
+        each([&](uint64_t, double yi, double, double) { s2 += (yi - mean) * (yi - mean); });
+        const double sigma2 = sum(s2) / nd;
         scale = 2.0 / (nd * sigma2);
     }
-    if (lane == 0) a.obj_scale[k] = scale;
+    if (tid == 0) a.obj_scale[k] = scale;
+    double W = 1.0, ybar = 0.0;
     if (a.split_gen) {  // as k_obj_stats
-        double W = 0.0, WY = 0.0;
-        for (uint64_t i = b + lane; i < e; i += 64) {
-            const double wi = 1.0 / ((double)dy[i] * (double)dy[i]);
+        W = 0.0;
+        double WY = 0.0;
+        each([&](uint64_t, double yi, double di, double) {
+            const double wi = 1.0 / (di * di);
             W += wi;
-            WY += wi * (double)y[i];
-        }
-        W = wave_sum64(W);
-        const double ybar = wave_sum64(WY) / W;
+            WY += wi * yi;
+        });
+        W = sum(W);
+        ybar = sum(WY) / W;
         double Wf = 0.0, Ys = 0.0, YYs = 0.0, Wd = 0.0, Yd = 0.0, YYd = 0.0;
-        for (uint64_t i = b + lane; i < e; i += 64) {
-            const double qi = sqrt(1.0 / ((double)dy[i] * (double)dy[i]) / W);
-            const double yc = (double)y[i] - ybar;
+        each([&](uint64_t, double yi, double di, double) {
+            const double qi = sqrt(1.0 / (di * di) / W);
+            const double yc = yi - ybar;
             const double q = (double)(float)qi;
             const float bq = (float)(qi * yc);
             Wf += q * q;
             Ys += (double)bq * q;
             YYs += q * q * yc * yc;
-            const double wn = 1.0 / ((double)dy[i] * (double)dy[i]) / W;
+            const double wn = 1.0 / (di * di) / W;
             Wd += wn;
             Yd += wn * yc;
             YYd += wn * yc * yc;
-        }
-        Wf = wave_sum64(Wf);
-        Ys = wave_sum64(Ys);
-        YYs = wave_sum64(YYs);
-        Wd = wave_sum64(Wd);
-        Yd = wave_sum64(Yd);
-        YYd = wave_sum64(YYd);
-        if (lane == 0) {
+        });
+        Wf = sum(Wf);
+        Ys = sum(Ys);
+        YYs = sum(YYs);
+        Wd = sum(Wd);
+        Yd = sum(Yd);
+        YYd = sum(YYd);
+        if (tid == 0) {
             const double Yb = Ys / Wf;
             a.obj_gen[kGen * k + 0] = Wf;
             a.obj_gen[kGen * k + 1] = Yb;
@@ -224,6 +278,60 @@ __global__ __launch_bounds__(64) void k_obj_stats_wave(StatsArgs a) {
             a.obj_gen[kGen * k + 7] = YYd / Wd - (Yd / Wd) * (Yd / Wd);
         }
     }
+    if (!a.rec_t) return;
+    {  // largest |y| (generalized: (w/W) |y - ybar|) and weight, as powers of two
+        const double iW = 1.0 / W;
+        double my = 0.0, mw = a.split_gen ? 0.0 : 1.0;
+        each([&](uint64_t, double yi, double di, double) {
+            double yv = yi;
+            if (a.split_gen) {
+                const double w = iW / (di * di);
+                yv = w * (yi - ybar);
+                mw = fmax(mw, w);
+            }
+            my = fmax(my, fabs(yv));
+        });
+        my = most(my);
+        mw = most(mw);
+        int ey = 0, ew = 0;
+        (void)frexp(my, &ey);  // my = f 2^ey, f in [0.5, 1)
+        (void)frexp(mw, &ew);
+        if (tid == 0) {
+            a.obj_ys[2 * k] = (float)(my > 0.0 ? ldexp(1.0, -ey) : 1.0);
+            a.obj_ys[2 * k + 1] = (float)(mw > 0.0 ? ldexp(1.0, -ew) : 1.0);
+        }
+    }
+    uint32_t mode = 0;
+    double tc = 0.0;
+    if (a.obj_ip) {  // the largest coarse step that oversamples the object's span enough
+        double lo = INFINITY, hi = -INFINITY;
+        each([&](uint64_t, double, double, double ti) {
+            lo = fmin(lo, ti);
+            hi = fmax(hi, ti);
+        });
+        lo = -most(-lo);
+        hi = most(hi);
+        const double cycles = (hi - lo) * a.df_rev * (a.split_gen ? kIpSigmaGen : kIpSigma);
+        if (n > kIpLeastObs && cycles > 0.0)
+            for (int q = 1; q <= kIpModes; ++q)
+                if (cycles * (double)ip_step(q) <= 1.0) mode = (uint32_t)q;
+        tc = 0.5 * (lo + hi);
+        if (tid == 0) {
+            InterpObj o;
+            o.tc = tc;
+            o.mode = mode;
+            o.unused = 0;
+            a.obj_ip[k] = o;
+        }
+    }
+    const double step = mode ? (double)ip_step((int)mode) * a.df_rev : 0.0;
+    each([&](uint64_t i, double, double, double ti) {
+        a.rec_t[b + i] = ti;
+        if (mode) {
+            const double tp = ti - tc;
+            a.rec_r[b + i] = make_double2(tp, ip_inv_window((int)mode, step * tp));
+        }
+    });
 }
 
 // ---------------------------------------------------------------------------
@@ -306,11 +414,31 @@ __global__ __launch_bounds__(64) void k_reduce_peaks(ReduceArgs a) {
     peaks_init(L);
     const uint64_t base = (uint64_t)k * a.chunks * kPeaks;
     const int nr = a.top_k == 1 ? 1 : kPeaks;  // top-1 sweeps write entry 0 of each slot
-    for (uint32_t c = threadIdx.x; c < a.chunks; c += 64)
+    const uint64_t *bits = a.obj_ip && a.obj_ip[k].mode ? a.cand + (uint64_t)k * a.cand_words : nullptr;
+    auto insert = [&](uint32_t c) {
         for (int r = 0; r < nr; ++r)
             peaks_insert(L, a.part_pow[base + (uint64_t)c * kPeaks + r],
                          a.part_idx[base + (uint64_t)c * kPeaks + r]);
-    block_peaks<64>(L, nullptr, nullptr);
+    };
+    if (bits) {
+        for (uint32_t w0 = 0; w0 < a.cand_words; w0 += 64) {  // a lane's word, the few set ones in turn
+            const uint32_t w = w0 + threadIdx.x;
+            const unsigned long long word = w < a.cand_words ? bits[w] : 0ull;
+            for (uint64_t some = __ballot(word != 0ull); some; some &= some - 1u) {
+                const int src = __builtin_ctzll(some);
+                const unsigned long long b = __shfl(word, src, 64);
+                if ((b >> threadIdx.x) & 1ull) insert(64u * (w0 + (uint32_t)src) + threadIdx.x);
+            }
+        }
+    } else {
+        for (uint32_t c = threadIdx.x; c < a.chunks; c += 64) insert(c);
+    }
+    Peaks W;
+    if (a.top_k == 1) block_best<64>(L.p[0], L.i[0], nullptr, nullptr);
+    else {
+        block_top3<64>(L, nullptr, nullptr, W);
+        L = W;
+    }
     if (threadIdx.x != 0) return;
     OUT *pp = static_cast<OUT *>(a.peak_power);
     OUT *pe = static_cast<OUT *>(a.peak_period);
@@ -471,6 +599,25 @@ int plan_workspace(const lsamd_sweep_args *a, Workspace *w) {
             w->part_sums = take(8 * base * sl * (size_t)ns * tile.fpt * tile.threads);
         }
     }
+    // The coarse-grid sweep: FP32 periodograms of the matrix-core tile.  An
+    // FP64 periodogram keeps the direct sums for every bin: interpolated
+    // powers differ from them by their rounding (1e-7), below the last places
+    // of an FP32 power but far above an FP64 one's.
+    // With obs_slices = 1 (the sub-sweeps of lsamd_batch_host) it looks at the
+    // call's type and grid alone, so that an object's result does not depend
+    // on what else is swept with it; with 0 small sweeps, which the direct
+    // sums' shorter chain of launches serves sooner, keep those.
+    const bool enough = a->obs_slices == 1 ? a->num_freqs >= kIpAloneFreqs
+                                           : a->num_freqs >= kIpMinFreqs &&
+                                                 (double)n * (double)a->num_freqs >= kIpMinTerms;
+    // (Its room does not depend on which outputs the arguments name.)
+    const bool room = te && te->prep && w->slices == 1 && enough && a->num_freqs < kIpMaxFreqs;
+    w->interp = room && a->dtype == LSAMD_F32 && a->pgram != nullptr;
+    if (room) {
+        w->obj_ip = take(sizeof(InterpObj) * K);
+        w->ip_tab = take((size_t)16 * 64 * 6 * kIpModes);
+        w->cand = take((size_t)8 * K * ((w->chunks + 63) / 64));
+    }
     w->queue = take(8 * kQueues);
     w->bytes = off + 256;
     return LSAMD_OK;
@@ -487,7 +634,10 @@ using namespace lsamd;
 // schedule's counter is cleared by a kernel), so no call depends on the
 // previous call's contents.
 namespace {
-constexpr size_t kStaticScratchBytes = LSAMD_STATIC_SCRATCH_BYTES;
+// 1 MiB beyond the documented size: what the coarse-grid sweep adds (its modes
+// and marks, under 1% of an object's tables and partials) refuses no call that
+// the documented size takes without it.
+constexpr size_t kStaticScratchBytes = LSAMD_STATIC_SCRATCH_BYTES + ((size_t)1 << 20);
 constexpr int kScratchDevices = 64;
 static __device__ __align__(256) unsigned char scratch[kStaticScratchBytes];
 std::atomic<void *> g_scratch_ptr[kScratchDevices];
@@ -601,13 +751,19 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
     const int T = w.tile.threads, M = w.tile.fpt;
 
     // 1. per-object statistics
+    const double dw = (a->max_freq - a->min_freq) / ((double)a->num_freqs * 1.0);
+    const bool mfma = te->prep != nullptr;
+    InterpObj *obj_ip = w.interp ? reinterpret_cast<InterpObj *>(ws + w.obj_ip) : nullptr;
     StatsArgs sa{a->offsets, a->y, a->dy, K, a->normalize && !gen, plain_pre ? 1 : 0,
-                 (split && gen) ? 1 : 0, obj_shift, obj_scale, obj_gen};
+                 (split && gen) ? 1 : 0, obj_shift, obj_scale, obj_gen,
+                 mfma ? reinterpret_cast<float *>(ws + w.obj_ys) : nullptr, a->t,
+                 mfma ? reinterpret_cast<double *>(ws + w.rec_t) : nullptr,
+                 mfma ? reinterpret_cast<double2 *>(ws + w.rec_r) : nullptr, obj_ip, dw * kInv2Pi};
     if (split) {
-        if (f64)
-            hipLaunchKernelGGL(k_obj_stats_wave<double>, dim3(K), dim3(64), 0, st, sa);
-        else
-            hipLaunchKernelGGL(k_obj_stats_wave<float>, dim3(K), dim3(64), 0, st, sa);
+        const bool wide = w.slices > 1;  // one long object alone
+        void (*fn)(StatsArgs) = wide ? (f64 ? k_obj_stats_split<double, 512> : k_obj_stats_split<float, 512>)
+                                     : (f64 ? k_obj_stats_split<double, 64> : k_obj_stats_split<float, 64>);
+        hipLaunchKernelGGL(fn, dim3(K), dim3(wide ? 512 : 64), 0, st, sa);
     } else {
         const dim3 sb(128), sg((K + 127) / 128);
         if (f64)
@@ -626,8 +782,9 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
     ra.obj_shift = obj_shift;
     ra.obj_gen = obj_gen;
     ra.precenter = plain_pre ? 1 : 0;
-    const double dw = (a->max_freq - a->min_freq) / ((double)a->num_freqs * 1.0);
-    if (split) {
+    if (mfma) {
+        // written with the statistics
+    } else if (split) {
         ra.rec_t = reinterpret_cast<double *>(ws + w.rec_t);
         ra.rec_a = reinterpret_cast<float4 *>(ws + w.rec_a);
         ra.rec_r = reinterpret_cast<double2 *>(ws + w.rec_r);
@@ -683,6 +840,13 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
     sw.rowfac = w.rowfac ? reinterpret_cast<uint4 *>(ws + w.rowfac) : nullptr;
     sw.obj_ys = w.obj_ys ? reinterpret_cast<float *>(ws + w.obj_ys) : nullptr;
 
+    if (w.interp) {
+        sw.obj_ip = obj_ip;
+        sw.ip_tab = reinterpret_cast<uint4 *>(ws + w.ip_tab);
+        sw.ip_items = (a->num_freqs + kIpLeastBins - 1) / kIpLeastBins;
+        sw.cand_words = (w.chunks + 63) / 64;
+    }
+
     const uint64_t items = (uint64_t)K * w.chunks * w.slices;
     sw.total_items = items;
     sw.queue = nullptr;
@@ -695,7 +859,7 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
     const uint64_t groups = (items + sw.group - 1) / sw.group;
     // about one object's groups per XCD run (grid schedule and persistent queues)
     sw.xcd_run = (uint32_t)std::max<uint64_t>(1, (uint64_t)w.chunks * w.slices / sw.group);
-    const bool persistent = a->schedule == LSAMD_SCHEDULE_PERSISTENT;
+    const bool persistent = a->schedule == LSAMD_SCHEDULE_PERSISTENT && !w.interp;
     uint32_t pgrid = 0;
     if (persistent) {
         sw.queue = reinterpret_cast<unsigned long long *>(ws + w.queue);
@@ -717,16 +881,45 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
         LS_HIP(timing_events(tm));
         LS_HIP(hipEventRecord(tm.ev[0], st));
     }
-    if (te->prep) {  // per-object set-up of the tile, inside the timed sweep
-        // wavefronts per object: enough for the mean object's 16-observation
-        // blocks, up to 256 (one object of many observations)
-        const uint64_t blocks = (a->num_obs / 16 + K - 1) / K + 1;
-        const uint32_t gy = (uint32_t)std::min<uint64_t>(256, blocks);
+    // wavefronts per object of its set-up: enough for the mean object's
+    // 16-observation blocks, up to 256 (one object of many observations)
+    const uint64_t blocks = (a->num_obs / 16 + K - 1) / K + 1;
+    const uint32_t gy = (uint32_t)std::min<uint64_t>(256, blocks);
+    if (w.interp) {
+        // The coarse-grid sweep, the marks of the chunks to sweep again and the
+        // direct tile's tables (which replace the coarse ones) in one launch,
+        // then the direct tile over those chunks and the objects in direct mode.
+        const InterpEntry &ip = kInterp[gen ? 1 : 0];
+        SweepArgs si = sw;
+        si.xcd_run = si.ip_items;
+        void *iargs[] = {&si};
+        LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(ip.fac), dim3(K + 3 * kIpModes, gy), dim3(64), iargs, 0,
+                               st));
+        const uint64_t ip_groups = (uint64_t)K * si.ip_items, most = 0xFFFFFFFFull / (uint64_t)ip.threads - 1;
+        for (uint64_t g = 0; g < ip_groups; g += most) {
+            si.item_base = g;
+            LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(ip.sweep),
+                                   dim3((uint32_t)std::min<uint64_t>(most, ip_groups - g)), dim3(ip.threads), iargs,
+                                   0, st));
+        }
+        SweepArgs sd = sw;
+        sd.cand = a->top_k > 0 ? reinterpret_cast<uint64_t *>(ws + w.cand) : nullptr;
+        sd.queue = nullptr;
+        // workgroups per object: ~16 rounds of the chip, or one per item
+        sd.cand_split = (uint32_t)std::min<uint64_t>(w.chunks, std::max<uint64_t>(1, 16384 / K));
+        sd.xcd_run = sd.cand_split;
+        void *dargs[] = {&sd};
+        LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->prep), dim3(K, gy + (sd.cand ? 1u : 0u)), dim3(64),
+                               dargs, 0, st));
+        LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->fn), dim3(K * sd.cand_split), dim3(T), dargs, 0,
+                               st));
+    } else if (te->prep) {  // per-object set-up of the tile, inside the timed sweep
         void *kargs[] = {&sw};
-        LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->prep), dim3(K, gy), dim3(64), kargs,
-                               0, st));
+        LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->prep), dim3(K, gy), dim3(64), kargs, 0, st));
     }
-    if (persistent) {
+    if (w.interp) {
+        // done
+    } else if (persistent) {
         sw.item_base = 0;
         void *kargs[] = {&sw};
         LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->fn), dim3(pgrid), dim3(T), kargs,
@@ -762,6 +955,9 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
         rd.top_k = a->top_k;
         rd.part_pow = sw.part_pow;
         rd.part_idx = sw.part_idx;
+        rd.obj_ip = obj_ip;
+        rd.cand = w.interp ? reinterpret_cast<const uint64_t *>(ws + w.cand) : nullptr;
+        rd.cand_words = sw.cand_words;
         rd.peak_index = a->peak_index;
         rd.peak_power = a->peak_power;
         rd.peak_period = a->peak_period;

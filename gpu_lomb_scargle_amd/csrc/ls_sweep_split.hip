@@ -2,165 +2,13 @@
 // rotation and FP32 partial sums folded into FP64, and the matrix-core
 // tiles), the observation-slice combiner, and their tile registry entries.
 
-#include "ls_device.h"
+#include "ls_split_device.h"
+
+#include "ls_interp.h"
 
 namespace lsamd {
 
 namespace {
-
-// ---------------------------------------------------------------------------
-// FP64 recomputation of ill-conditioned bins.  Every split-form power comes
-// from a 2x2 (standard) or centred 2x2 (generalized) least-squares system; its
-// relative error is the sums' relative error times a condition number that
-// the sums themselves give:
-//   standard:    k = (CC + SS)^2 / (4 D)                 (1 for balanced phases)
-//   generalized: k = (1 + C^2 + S^2) (CC + SS) / D      (centred CC, SS, CS;
-//                the 1 + C^2 + S^2 covers the centring CC = CCw - C^2)
-// with D = CC SS - CS^2.  The FP32 sums (split32) leave ~2.4e-7 k relative
-// (measured on the 1000-object generalized batch at the 1 cycle/day alias,
-// k ~ 110-230), the FP32-seeded FP64 sums (split) less.  Bins with
-// k > kCondMax (a few per 10^6 for nightly-sampled objects) and every bin of
-// objects of at most kSmallObs observations (5 points against the
-// generalized 3-parameter model can give k ~ 10^5) are computed again from
-// the caller's FP64 t, y, dy with FP64 phasors.
-// ---------------------------------------------------------------------------
-constexpr double kCondMax = 16.0;
-constexpr uint32_t kSmallObs = 16;
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
-// Lane src's v, in every lane (src the same in all lanes).
-__device__ __forceinline__ double lane_value(double v, int src) {
-    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, src);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), src);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
-// sin and cos of 2 pi r for |r| <= 1/2 revolution: the octant q = rint(4 r)
-// is taken off exactly, and x = 2 pi (r - q/4), |x| <= pi/4, goes through the
-// Taylor series of sin to x^17 and of cos to x^16 (the first omitted terms
-// are below 5e-17 and 2e-18), in Horner form.
-__device__ __forceinline__ void sincos_rev64(double r, double &s, double &c) {
-    const double q = __builtin_rint(4.0 * r);
-    const double x = (r - 0.25 * q) * kTwoPi, x2 = x * x;
-    double ps = -1.0 / 355687428096000.0;  // -1/17!
-    ps = fma(ps, x2, 1.0 / 1307674368000.0);
-    ps = fma(ps, x2, -1.0 / 6227020800.0);
-    ps = fma(ps, x2, 1.0 / 39916800.0);
-    ps = fma(ps, x2, -1.0 / 362880.0);
-    ps = fma(ps, x2, 1.0 / 5040.0);
-    ps = fma(ps, x2, -1.0 / 120.0);
-    ps = fma(ps, x2, 1.0 / 6.0);
-    const double sx = fma(-ps * x2, x, x);  // x - x^3/3! + ... - x^17/17!... with alternating signs
-    double pc = 1.0 / 20922789888000.0;     // 1/16!
-    pc = fma(pc, x2, -1.0 / 87178291200.0);
-    pc = fma(pc, x2, 1.0 / 479001600.0);
-    pc = fma(pc, x2, -1.0 / 3628800.0);
-    pc = fma(pc, x2, 1.0 / 40320.0);
-    pc = fma(pc, x2, -1.0 / 720.0);
-    pc = fma(pc, x2, 1.0 / 24.0);
-    pc = fma(pc, x2, -0.5);
-    const double cx = fma(pc, x2, 1.0);
-    const int o = (int)q & 3;  // sin/cos of q pi/2 + x
-    s = o == 0 ? sx : o == 1 ? cx : o == 2 ? -sx : -cx;
-    c = o == 0 ? cx : o == 1 ? -sx : o == 2 ? -cx : sx;
-}
-
-// e^{2 pi i f t} in FP64: the phase reduced to [-1/2, 1/2] revolutions with
-// the product f t fused (exact before the subtraction).
-__device__ __forceinline__ void phasor64(double f, double t, double &c, double &s) {
-    const double n = __builtin_rint(f * t);
-    sincos_rev64(fma(f, t, -n), s, c);
-}
-
-// n / d for d > 0 (normal): the hardware reciprocal refined by two Newton
-// steps, then one correction of the quotient (within an ulp or two; the
-// IEEE division sequence is twice as long).
-__device__ __forceinline__ double fdiv(double n, double d) {
-    double r = __builtin_amdgcn_rcp(d);
-    r = fma(fma(-d, r, 1.0), r, r);
-    r = fma(fma(-d, r, 1.0), r, r);
-    const double q = n * r;
-    return fma(fma(-d, q, n), r, q);
-}
-
-// Power of the standard variant from its uncentred sums (SS = N - CC);
-// `ill` when its condition number exceeds kCondMax (or D <= 0, or NaN).
-__device__ __forceinline__ double std_power(double XC, double XS, double CC, double CS, double N, bool &ill) {
-    const double SS = N - CC, D = CC * SS - CS * CS;
-    ill = !((CC + SS) * (CC + SS) <= 4.0 * kCondMax * D) || !(D > 0.0);
-    return fdiv(0.5 * (SS * XC * XC - 2.0 * CS * XC * XS + CC * XS * XS), D);
-}
-
-// Power of the generalized variant from sums over weights normalised to
-// sum 1 (C, S, CCw, SSw, CSw, YCw, YSw; Yb = weighted mean of the y in them,
-// YY the centred weighted sum of squares); `ill` as for std_power.
-__device__ __forceinline__ double gen_power(double C, double S, double CCw, double SSw, double CSw,
-                                            double YCw, double YSw, double Yb, double YY, bool &ill) {
-    const double YC = YCw - Yb * C, YS = YSw - Yb * S;
-    const double CC = CCw - C * C, SS = SSw - S * S, CS = CSw - C * S;
-    const double D = CC * SS - CS * CS;
-    ill = !((1.0 + C * C + S * S) * (CC + SS) <= kCondMax * D) || !(D > 0.0);
-    return fdiv(SS * YC * YC - 2.0 * CS * YC * YS + CC * YS * YS, D * YY);
-}
-
-// FP64 power of bin kf of object obj (before the object's scale); every lane
-// of the wavefront calls it with the same (obj, kf) and gets the result.
-// Standard: raw y, unit weights.  Generalized: w = dy^-2 / W and y - ybar with
-// W and ybar from the statistics kernel (the power does not depend on them
-// beyond rounding: the weights are normalised and the mean floats).
-template <bool GEN, typename IN>
-__device__ double exact_power(const SweepArgs &a, uint32_t obj, uint32_t kf) {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint64_t b = a.offsets[obj], e = a.offsets[obj + 1];
-    const double f = a.fmin_rev + (double)kf * a.df_rev;
-    const IN *y = static_cast<const IN *>(a.y);
-    const IN *dy = static_cast<const IN *>(a.dy);
-    double iW = 1.0, ybar = 0.0;
-    if constexpr (GEN) {
-        iW = 1.0 / a.obj_gen[kGen * obj + 4];
-        ybar = a.obj_gen[kGen * obj + 3];
-    }
-    double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0, s4 = 0.0, s5 = 0.0, s6 = 0.0, s7 = 0.0, s8 = 0.0;
-    for (uint64_t j = b + lane; j < e; j += 64) {
-        double c, sn;
-        phasor64(f, a.rec_t[j], c, sn);
-        if constexpr (GEN) {
-            const double dj = (double)dy[j], w = iW / (dj * dj), yc = (double)y[j] - ybar;
-            const double wc = w * c, wy = w * yc;
-            s0 += wc;
-            s1 = fma(w, sn, s1);
-            s2 = fma(wc, c, s2);
-            s3 = fma(wc, sn, s3);
-            s4 = fma(wy, c, s4);
-            s5 = fma(wy, sn, s5);
-            s6 += w;
-            s7 += wy;
-            s8 = fma(wy, yc, s8);
-        } else {
-            const double yj = (double)y[j];
-            s0 = fma(yj, c, s0);
-            s1 = fma(yj, sn, s1);
-            s2 = fma(c, c, s2);
-            s3 = fma(c, sn, s3);
-        }
-    }
-    bool ill;
-    if constexpr (GEN) {
-        const double W = wave_sum(s6), iWn = 1.0 / W;
-        const double C = wave_sum(s0) * iWn, S = wave_sum(s1) * iWn, CCw = wave_sum(s2) * iWn;
-        const double CSw = wave_sum(s3) * iWn, YCw = wave_sum(s4) * iWn, YSw = wave_sum(s5) * iWn;
-        const double Yb = wave_sum(s7) * iWn, YY = wave_sum(s8) * iWn - Yb * Yb;
-        return gen_power(C, S, CCw, 1.0 - CCw, CSw, YCw, YSw, Yb, YY, ill);
-    } else {
-        return std_power(wave_sum(s0), wave_sum(s1), wave_sum(s2), wave_sum(s3), (double)(e - b), ill);
-    }
-}
 
 // Recomputes, in FP64, the bins this wavefront's lanes flagged (bit m of a
 // lane's `flags` for its bin m, whose number bin_of(lane, m) gives), one bin
@@ -282,11 +130,6 @@ __device__ void small_object_powers(const SweepArgs &a, uint32_t obj, uint32_t k
             P[v] = std_power(acc[0][v], acc[1][v], acc[2][v], acc[3][v], N, ill);
         }
     }
-}
-
-// Bin of result entry v of lane (rc, kh) in a matrix-core work item.
-__device__ __forceinline__ uint32_t mfma_bin(uint32_t kbase, uint32_t rc, uint32_t kh, int v) {
-    return kbase + 32u * (8u * (uint32_t)(v / 4) + 4u * kh + (uint32_t)(v % 4)) + rc;
 }
 
 // ---------------------------------------------------------------------------
@@ -796,41 +639,62 @@ __global__ __launch_bounds__(T) void k_sweep_split64(SweepArgs a) {
 // column (B) l % 32 and observations 8 (l / 32) .. +7 of the block; the
 // result holds column l % 32, rows 8 (v / 4) + 4 (l / 32) + v % 4, v < 16.
 // ---------------------------------------------------------------------------
-typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
-
-constexpr float kFacScale = 1024.0f;  // 2^10 on the column factors
-
-// Heads and tails of two factors x: h = fp16(x), l = fp16(x - h) (x - h is
-// exact in FP32).  The head must be one value.  When x is a product a b, the compiler may
-// round the exact product to FP16 in one step for the tail's head
-// (v_fma_mixlo_f16 h, a, b, 0) yet convert the FP32-rounded x for the packed
-// MFMA operand (v_cvt_pk_f16_f32); the two roundings differ by one FP16 ulp
-// in ~1 of 2^13 factors, which are then wrong by 2^-11 (seen as 4e-3 power
-// errors).  Here the two heads of a pair of factors come from one packed
-// conversion of their FP32 values (v_cvt_pk_f16_f32), and the tails are
-// taken against those very heads (the compiler may form x - h from the exact
-// product; that only makes h + l closer to it).  tests/test_split_rounding.py
-// checks the built kernels for the one-step product-to-FP16 form.
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
-typedef float float2_t __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ void split16x2(float x0, float x1, half2_t &h, half2_t &l) {
-    h = __builtin_convertvector((float2_t){x0, x1}, half2_t);
-    const float2_t hf = __builtin_convertvector(h, float2_t);
-    l = __builtin_convertvector((float2_t){x0 - hf.x, x1 - hf.y}, half2_t);
-}
-
-// First column-factor slot of an object: the slots of object k are
-// [floor(beg/16) + k, floor(beg/16) + k + ceil(N/16)), which never reach the
-// next object's floor((beg + N)/16) + k + 1.
-__device__ __forceinline__ uint64_t colfac_slot(uint64_t beg, uint32_t obj) { return (beg >> 4) + obj; }
-
-// Heads and tails of two FP64 factors: h = fp16(fp32(x)), l = fp16(x - h),
-// the remainder x - h exact in FP64 (~22 bits of x in h + l).
-__device__ __forceinline__ void split64x2(double x0, double x1, half2_t &h, half2_t &l) {
-    h = __builtin_convertvector((float2_t){(float)x0, (float)x1}, half2_t);
-    l = __builtin_convertvector((float2_t){(float)(x0 - (double)h.x), (float)(x1 - (double)h.y)}, half2_t);
+// ---------------------------------------------------------------------------
+// Chunks (1024 bins) that can hold one of an object's top_k bins: those that
+// overlap a result tile whose best power reaches the top_k-th best of the
+// tiles' lane maxima (a lower bound of the top_k-th best power) less
+// kIpMargin.  The direct tile computes them again, so that peaks come from the
+// same arithmetic whichever way the rest of the grid was formed.  One
+// wavefront per object; bit c % 64 of word c / 64.
+// ---------------------------------------------------------------------------
+__device__ void mark_chunks(const SweepArgs &a, uint32_t obj) {
+    const uint32_t lane = threadIdx.x;
+    const int mode = (int)a.obj_ip[obj].mode;
+    if (mode == 0) return;
+    const uint32_t rb = (uint32_t)(ip_step(mode) * ip_per_row(mode)), rows = (uint32_t)ip_rows(mode);
+    const uint32_t tpi = (rows + 31u) / 32u, S = rows * rb;
+    const float *tmax = reinterpret_cast<const float *>(a.part_pow + (uint64_t)obj * a.chunks * kPeaks);
+    auto tile_of_bin = [&](uint32_t bin) {
+        const uint32_t it = bin / S;
+        return it * tpi + (bin - it * S) / (32u * rb);
+    };
+    const uint32_t ntiles = tile_of_bin(a.nf - 1u) + 1u;
+    float t0 = 0.0f, t1 = 0.0f, t2 = 0.0f;
+#pragma unroll 8
+    for (uint32_t i = lane; i < 3u * ntiles; i += 64u) {  // into the lane's descending three
+        const float p = tmax[i], a0 = fminf(t0, p), a1 = fminf(t1, a0);
+        t0 = fmaxf(t0, p);
+        t1 = fmaxf(t1, a0);
+        t2 = fmaxf(t2, a1);
+    }
+    float tau = 0.0f;
+    for (int r = 0; r < a.top_k; ++r) {
+        tau = t0;
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) tau = fmaxf(tau, __shfl_xor(tau, off, 64));
+        const uint64_t at = __ballot(t0 == tau);
+        if (at && lane == (uint32_t)__builtin_ctzll(at)) {
+            t0 = t1;
+            t1 = t2;
+            t2 = 0.0f;
+        }
+    }
+    const float least = tau * (1.0f - kIpMargin);
+    uint64_t *bits = a.cand + (uint64_t)obj * a.cand_words;
+    for (uint32_t w = 0; w < a.cand_words; ++w) {
+        const uint32_t c = 64u * w + lane;
+        bool yes = false;
+        if (c < a.chunks) {
+            const uint32_t last = 1024u * c + 1023u < a.nf ? 1024u * c + 1023u : a.nf - 1u;
+            const uint32_t end = tile_of_bin(last);
+            for (uint32_t t = tile_of_bin(1024u * c); t <= end; ++t) {
+                const float p = tmax[3u * t];
+                yes = yes || (p > 0.0f && p >= least);
+            }
+        }
+        const uint64_t word = __ballot(yes);
+        if (lane == 0) bits[w] = word;
+    }
 }
 
 // Wavefronts (object, y) with y < gridDim.y write the column-factor fragments
@@ -843,14 +707,19 @@ __device__ __forceinline__ void split64x2(double x0, double x1, half2_t &h, half
 // caller's FP64 (or FP32) t, y, dy in FP64 arithmetic: FP64 phase and
 // sin/cos, w/W = 1 / (dy^2 W) the normalised weight, y_c = y - ybar; y (or
 // (w/W) y_c) scaled per object by a power of two ys, and w/W by a power of
-// two ws, to a maximum in [0.5, 1), then all by 2^10 (FP16 range; the scales
-// are undone exactly in the power; wavefront y = 0 stores them); and the
+// two ws, to a maximum in [0.5, 1) (from the statistics), then all by 2^10
+// (FP16 range; the scales are undone exactly in the power); and the
 // row-step fragments (e^{2 pi i 32 a df t}, row a = l % 32).  Observations
 // past the object's end have zero factors.
 template <bool GEN, typename IN>
 __global__ __launch_bounds__(64) void k_colfac(SweepArgs a) {
     constexpr int NF = GEN ? kColfacFragsGen : kColfacFragsStd;
     const uint32_t k = blockIdx.x, l = threadIdx.x;
+    // beside the coarse-grid sweep: the marks of its objects (the last y), and
+    // their tables only if marked chunks are swept
+    const uint32_t gy = gridDim.y - (a.cand ? 1u : 0u);
+    if (blockIdx.y == gy) return mark_chunks(a, k);
+    if (a.obj_ip && a.obj_ip[k].mode != 0u && !a.cand) return;
     const uint64_t beg = a.offsets[k], end = a.offsets[k + 1];
     const uint32_t n = (uint32_t)(end - beg);
     const IN *y = static_cast<const IN *>(a.y);
@@ -872,31 +741,13 @@ __global__ __launch_bounds__(64) void k_colfac(SweepArgs a) {
         if constexpr (GEN) return weight(i) * ((double)y[i] - ybar);
         else return (double)y[i];
     };
-    double my = 0.0, mw = 0.0;
-    for (uint64_t i = beg + l; i < end; i += 64) {
-        my = fmax(my, fabs(yfac(i)));
-        mw = fmax(mw, weight(i));
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        my = fmax(my, __shfl_xor(my, off, 64));
-        mw = fmax(mw, __shfl_xor(mw, off, 64));
-    }
-    int ey = 0, ew = 0;
-    (void)frexp(my, &ey);  // my = f 2^ey, f in [0.5, 1)
-    (void)frexp(mw, &ew);
-    const double ys = my > 0.0 ? ldexp(1.0, -ey) : 1.0;
-    const double ws = mw > 0.0 ? ldexp(1.0, -ew) : 1.0;
-    if (blockIdx.y == 0 && l == 0) {
-        a.obj_ys[2 * k] = (float)ys;
-        a.obj_ys[2 * k + 1] = (float)ws;
-    }
+    const double ys = (double)a.obj_ys[2 * k], ws = (double)a.obj_ys[2 * k + 1];
     const double sy = ys * (double)kFacScale, sw = ws * (double)kFacScale;  // exact: powers of two
     const double fb = (double)(l & 31u) * a.df_rev;
     const double fr = (double)(32u * (l & 31u)) * a.df_rev;  // row step of row l % 32
     uint4 *dst = a.colfac + colfac_slot(beg, k) * (uint64_t)(NF * 64) + l;
     uint4 *rdst = a.rowfac + colfac_slot(beg, k) * (uint64_t)(kRowfacFrags * 64) + l;
-    for (uint32_t q = blockIdx.y; q * 16u < n; q += gridDim.y) {
+    for (uint32_t q = blockIdx.y; q * 16u < n; q += gy) {
         // row-step phasors R = e^{2 pi i 32 (l % 32) df t} of observations
         // 8 (l / 32) .. + 7, in FP64 rounded to FP32 (zero past the end)
 #pragma unroll
@@ -974,16 +825,6 @@ struct RowFrags {
     half8_t ur_h, ur_l, ui_h, ui_l, qr_h, qr_l, qi_h, qi_l;
     half8_t nui_h, nui_l, nqi_h, nqi_l;  // -u_i, -(u^2)_i: the sign bits flipped
 };
-__device__ __forceinline__ half8_t neg8(half8_t x) {
-    uint4 u;
-    __builtin_memcpy(&u, &x, sizeof(u));
-    u.x ^= 0x80008000u;
-    u.y ^= 0x80008000u;
-    u.z ^= 0x80008000u;
-    u.w ^= 0x80008000u;
-    __builtin_memcpy(&x, &u, sizeof(u));
-    return x;
-}
 __device__ __forceinline__ void row_factors(const float2 *s_u0, uint32_t j0, uint32_t kh,
                                             const uint4 (&rr)[kRowfacFrags], RowFrags &R) {
 #pragma unroll
@@ -1022,12 +863,6 @@ __device__ __forceinline__ void row_factors(const float2 *s_u0, uint32_t j0, uin
     R.nqi_l = neg8(R.qi_l);
 }
 
-// Loads the row-step fragments of one 16-observation block.
-__device__ __forceinline__ void load_rows(const uint4 *rf, uint4 (&rr)[kRowfacFrags]) {
-#pragma unroll
-    for (int i = 0; i < kRowfacFrags; ++i) rr[i] = rf[i * 64];
-}
-
 // e^{2 pi i f0 t} of observation b0 + l of the current stage into s_u0[l]
 // (zero past cnt, the object's end: zero row factors).
 __device__ __forceinline__ void stage_u0(const SweepArgs &a, uint64_t b0, uint32_t cnt, double f0, float2 *s_u0) {
@@ -1040,18 +875,6 @@ __device__ __forceinline__ void stage_u0(const SweepArgs &a, uint64_t b0, uint32
     }
     s_u0[l] = u0;
 }
-
-// Loads the column-factor fragments of one 16-observation block.
-template <int NF>
-__device__ __forceinline__ void load_cols(const uint4 *cf, half8_t (&col)[NF]) {
-#pragma unroll
-    for (int i = 0; i < NF; ++i) {
-        const uint4 u = cf[i * 64];
-        __builtin_memcpy(&col[i], &u, sizeof(u));
-    }
-}
-
-#define LS_MFMA(ACC, A, B) ACC = __builtin_amdgcn_mfma_f32_32x32x16_f16(A, B, ACC, 0, 0, 0)
 
 // Emits a lane's 16 bins of a matrix-core work item.  power(v, ill) gives
 // result entry v's power (before the object's scale) and whether its
@@ -1138,8 +961,8 @@ __global__ __launch_bounds__(64, 2) void k_sweep_mfma(SweepArgs a) {
     __shared__ uint64_t s_item;
     const uint32_t l = threadIdx.x, rc = l & 31u, kh = l >> 5;
     constexpr double kUnscale = 1.0 / (double)kFacScale;  // column factors scaled, rows not
-    for (uint64_t item = first_item(a, &s_item); item < a.total_items;
-         item = next_item(a, &s_item, item)) {
+    for (uint64_t item = direct_first(a, &s_item); item < a.total_items;
+         item = direct_next(a, &s_item, item)) {
         // (object, chunk, slice); slices hold a multiple of 16 observations
         uint64_t oc = item;
         uint32_t slice = 0, obj, chunk;
@@ -1323,8 +1146,8 @@ __global__ __launch_bounds__(64) void k_sweep_mfma_gen(SweepArgs a) {
     __shared__ uint64_t s_item;
     const uint32_t l = threadIdx.x, rc = l & 31u, kh = l >> 5;
     constexpr double kUnscale = 1.0 / (double)kFacScale;  // column factors scaled, rows not
-    for (uint64_t item = first_item(a, &s_item); item < a.total_items;
-         item = next_item(a, &s_item, item)) {
+    for (uint64_t item = direct_first(a, &s_item); item < a.total_items;
+         item = direct_next(a, &s_item, item)) {
         uint64_t oc = item;
         uint32_t slice = 0, obj, chunk;
         if (a.slices > 1) {

@@ -41,9 +41,10 @@ class SweepPlan:
     t, y, dy: 1-D float32/float64 CUDA tensors (dy only for the generalized
     variant); offsets: int64 CUDA tensor of K+1 row offsets.  order (optional
     int32/uint32 CUDA tensor of K object numbers) is the processing order;
-    by default objects are processed longest first.  obs_slices=1 keeps a
-    single-object split-form sweep from spreading its observations over
-    workgroups (0, the default, lets it).  tile=(threads, freqs_per_thread)
+    by default objects are processed longest first.  obs_slices=1 keeps the
+    way an object's sums are formed independent of what else the plan sweeps
+    (0, the default, lets a single object's observations be spread over
+    workgroups and small float32 split32 sweeps keep the direct sums).  tile=(threads, freqs_per_thread)
     picks a compiled tile shape for this plan only (None: the process
     default); autotune() sets it to the fastest.
     """

@@ -138,8 +138,10 @@ typedef struct lsamd_sweep_args {
     void *peak_period;       /* device, K*top_k (days), or NULL */
     int32_t schedule;        /* enum lsamd_schedule */
     int32_t obs_slices;      /* split forms, 0: a sweep of one object with many observations
-                              * spreads them over workgroups (results then differ from the
-                              * same object swept in a batch by rounding only); 1: never */
+                              * spreads them over workgroups, and a small FP32 split32 sweep
+                              * takes its sums at every bin where a larger one takes them on a
+                              * coarse grid (results then differ from the same object swept in
+                              * another batch by rounding only); 1: neither */
     /* Tile shape of this sweep (threads per workgroup, frequencies per
      * thread), one of the shapes compiled for form/variant (lsamd_autotune
      * reports the fastest); 0, 0: the process default (lsamd_set_tile, else
