@@ -57,6 +57,7 @@ struct SweepArgs {
     const InterpObj *obj_ip;
     uint4 *ip_tab;
     uint32_t ip_items;
+    float ip_margin;  // of the marked chunks' powers
     uint32_t cand_words, cand_split;  // words per object; workgroups per object of the direct passes
     uint64_t *cand;
 };

@@ -51,6 +51,7 @@ struct Workspace {
     // coarse-grid sweep (interp): modes per object, interpolation operands,
     // marked chunks
     bool interp = false;
+    bool screen = false;    // interp, for peaks alone
     size_t obj_ip = 0;      // InterpObj[K]
     size_t ip_tab = 0;
     size_t cand = 0;        // uint64[K * ceil(chunks / 64)]

@@ -2,13 +2,19 @@
 // statistics and record kernels that choose a mode per object (ls_sweep.hip).
 //
 // A mode has a coarse step of h bins and result rows of m coarse steps (h m
-// <= 32 bins, one lane each).  W = 8 taps at an oversampling of at least
-// kIpSigma = 1.95 keep the aliasing at 2e-8 and leave the rounding, which at
-// 1.95 is no larger than the direct sums': emulated over light curves of 30 to
-// 700 observations, worst power 7.3e-6 (bins of at least 1e-3 of the peak)
-// against 7.7e-6; W = 7 reaches 1.5e-5, an oversampling of 1.45 with W = 10
-// 2.5e-5 (the observations at the ends of the span carry weights 1/Phi of 18
-// there, 2.9 at 1.95).  h = 5 is the grid of ten bins per resolution element.
+// <= 32 bins, one lane each).  Two uses:
+//   sums   (FP32 periodograms) W = 8 taps at an oversampling of at least
+//     kIpSigma = 1.95 keep the aliasing at 2e-8 and leave the rounding, which
+//     at 1.95 is no larger than the direct sums': emulated over light curves
+//     of 30 to 700 observations, worst power 7.3e-6 (bins of at least 1e-3 of
+//     the peak) against 7.7e-6; W = 7 reaches 1.5e-5, an oversampling of 1.45
+//     with W = 10 2.5e-5 (the observations at the ends of the span carry
+//     weights 1/Phi of 18 there, 2.9 at 1.95).  The generalized power, from
+//     four interpolated sums, needs 2.4 (measured on 200 objects, h = 5 / 4:
+//     1.1e-5 / 8.0e-6, direct 7.6e-6).
+//   screen (peaks without a periodogram) FP16 heads alone, W = 6 taps at an
+//     oversampling of at least 1.3: aliasing 1.2e-4, powers near the peak
+//     good to ~1e-3, which only decide which chunks the direct tile sweeps.
 #pragma once
 
 #include "ls_device.h"
@@ -17,28 +23,30 @@ namespace lsamd {
 
 namespace {
 
-constexpr int kIpModes = 6;
-constexpr int kIpTaps = 8;
-constexpr double kIpSigma = 1.95, kIpSigmaGen = 2.4;
-constexpr int kIpFrags = 8;           // column-factor fragments per 16 observations
-constexpr float kIpMargin = 1e-4f;    // ten times the form's error bound
+constexpr int kIpModes = 7;           // h = 3 in the screen only
+constexpr double kIpSigma = 1.95, kIpSigmaGen = 2.4, kIpSigmaScreen = 1.3;
+__host__ __device__ constexpr int ip_frags(bool screen) { return screen ? 4 : 8; }  // column-factor fragments per 16 observations
+// Relative margin of the marked chunks below the top_k-th best power: ten
+// times the sums' error bound; the screen's: see k_sweep_interp.
+constexpr float kIpMargin = 1e-4f, kIpMarginScreen = 0.125f;
 __host__ __device__ constexpr int ip_step(int mode) {
-    return mode == 1 ? 4 : mode == 2 ? 5 : mode == 3 ? 6 : mode == 4 ? 8 : mode == 5 ? 10 : 16;
+    return mode == 1 ? 3 : mode == 2 ? 4 : mode == 3 ? 5 : mode == 4 ? 6 : mode == 5 ? 8 : mode == 6 ? 10 : 16;
 }
 __host__ __device__ constexpr int ip_per_row(int mode) { return 32 / ip_step(mode); }
 // rows of a workgroup: m rows + W - 1 <= 2048 points, a multiple of 32 where that loses less than a tile
 __host__ __device__ constexpr int ip_rows(int mode) {
-    return mode == 1 ? 255 : mode == 2 ? 320 : mode == 3 ? 408 : mode == 4 ? 510 : mode == 5 ? 672 : 1020;
+    return mode == 1 ? 192 : mode == 2 ? 255 : mode == 3 ? 320 : mode == 4 ? 408 : mode == 5 ? 510 : mode == 6 ? 672 : 1020;
 }
-__host__ __device__ constexpr int ip_taps(int) { return kIpTaps; }
-__host__ __device__ constexpr double ip_beta(int mode) {
-    return 3.14159265358979323846 * ip_taps(mode) * (1.0 - 1.0 / (2.0 * kIpSigma));
+__host__ __device__ constexpr int ip_taps(bool screen) { return screen ? 6 : 8; }
+__host__ __device__ constexpr double ip_beta(bool screen) {
+    return 3.14159265358979323846 * ip_taps(screen) * (1.0 - 1.0 / (2.0 * (screen ? kIpSigmaScreen : kIpSigma)));
 }
-constexpr uint32_t kIpLeastBins = 255 * 32;  // bins per workgroup, smallest mode
-// Objects up to here (at most two 16-observation blocks) keep the direct sums,
-// those of at most 16 observations their FP64 ones: with 18 observations and
-// weights over a factor of 400 the worst bin reached 1.4e-5 (direct 1.0e-5).
-constexpr uint32_t kIpLeastObs = 24;
+constexpr uint32_t kIpLeastBins = 255 * 32, kIpLeastBinsScreen = 192 * 30;  // bins per workgroup, smallest mode
+constexpr uint32_t kIpGroup = 4;  // consecutive items of an object per workgroup, at most
+// Objects up to here keep the direct sums, those of at most 16 observations
+// their FP64 ones: with 18 observations and weights over a factor of 400 the
+// worst bin reached 1.4e-5 (direct 1.0e-5).
+constexpr uint32_t kIpLeastObs = 24, kIpLeastObsScreen = 16;
 // Below these the direct sums are sooner done (FP32, top-1, ten bins per
 // resolution element; direct / coarse, us): 400 objects x 20,000 bins, 1.4e9
 // terms, 152 / 170 standard and 288 / 260 generalized; 100 x 80,000, 1.4e9:
@@ -47,25 +55,30 @@ constexpr uint32_t kIpLeastObs = 24;
 // coarse grid from 2^18 bins on, where a few objects lose ~25 us by it.
 constexpr uint32_t kIpMinFreqs = 8192;  // bins a workgroup takes, smallest mode
 constexpr double kIpMinTerms = 1.5e9;
+// Peaks alone (FP64, top-3, direct / coarse): 10 objects x 300,000 bins, 0.5e9
+// terms, 82 / 76 standard and 127 / 110 generalized; 40 x 100,000, 0.7e9: 87 / 99
+// and 135 / 139; 200 x 20,000, 0.7e9: 104 / 137 and 166 / 205; 200 x 50,000,
+// 1.7e9: 160 / 149 and 240 / 212.
+constexpr double kIpMinTermsScreen = 1e9;
 constexpr uint32_t kIpAloneFreqs = 1u << 18;
 constexpr uint32_t kIpMaxFreqs = 1u << 29;   // byte offsets of an object's row in 32 bits
 
-// 1 / Phi(xi) of a mode's window, Phi(0) = 1, at xi = h df t' cycles per
-// coarse step, |xi| <= 1 / (2 kIpSigma): s = sqrt(beta^2 - (pi W xi)^2) >= 17,
-// where sinh s = e^s / 2 to FP64.
-__device__ __forceinline__ double ip_inv_window(int mode, double xi) {
-    const double beta = ip_beta(mode), u = 3.14159265358979323846 * ip_taps(mode) * xi;
+// 1 / Phi(xi) of the window, Phi(0) = 1, at xi = h df t' cycles per coarse
+// step, |xi| <= 1 / (2 sigma): s = sqrt(beta^2 - (pi W xi)^2) >= 17 (screen 9),
+// where sinh s = e^s / 2 to FP64 (screen: 2e-8).
+__device__ __forceinline__ double ip_inv_window(bool screen, double xi) {
+    const double beta = ip_beta(screen), u = 3.14159265358979323846 * ip_taps(screen) * xi;
     const double s = sqrt(beta * beta - u * u);
     return s / beta * exp(beta - s);
 }
 
 }  // namespace
 
-// Kernels of the coarse-grid sweep, [variant].
+// Kernels of the coarse-grid sweep, [screen][variant][dtype] (sums: FP32 only).
 struct InterpEntry {
     SweepFn fac, sweep;
     int threads;
 };
-extern const InterpEntry kInterp[2];
+extern const InterpEntry kInterp[2][2][2];
 
 }  // namespace lsamd

@@ -68,6 +68,9 @@ struct StatsArgs {
     double2 *rec_r;
     InterpObj *obj_ip;
     double df_rev;
+    double sigma;        // least oversampling of the coarse grid, observations an object needs
+    uint32_t least_obs;  // more than, and the first mode
+    int first_mode, screen;
 };
 
 struct RecArgs {
@@ -311,9 +314,9 @@ __global__ __launch_bounds__(T) void k_obj_stats_split(StatsArgs a) {
         });
         lo = -most(-lo);
         hi = most(hi);
-        const double cycles = (hi - lo) * a.df_rev * (a.split_gen ? kIpSigmaGen : kIpSigma);
-        if (n > kIpLeastObs && cycles > 0.0)
-            for (int q = 1; q <= kIpModes; ++q)
+        const double cycles = (hi - lo) * a.df_rev * a.sigma;
+        if (n > a.least_obs && cycles > 0.0)
+            for (int q = a.first_mode; q <= kIpModes; ++q)
                 if (cycles * (double)ip_step(q) <= 1.0) mode = (uint32_t)q;
         tc = 0.5 * (lo + hi);
         if (tid == 0) {
@@ -329,7 +332,7 @@ __global__ __launch_bounds__(T) void k_obj_stats_split(StatsArgs a) {
         a.rec_t[b + i] = ti;
         if (mode) {
             const double tp = ti - tc;
-            a.rec_r[b + i] = make_double2(tp, ip_inv_window((int)mode, step * tp));
+            a.rec_r[b + i] = make_double2(tp, ip_inv_window(a.screen != 0, step * tp));
         }
     });
 }
@@ -612,8 +615,14 @@ int plan_workspace(const lsamd_sweep_args *a, Workspace *w) {
                                                  (double)n * (double)a->num_freqs >= kIpMinTerms;
     // (Its room does not depend on which outputs the arguments name.)
     const bool room = te && te->prep && w->slices == 1 && enough && a->num_freqs < kIpMaxFreqs;
-    w->interp = room && a->dtype == LSAMD_F32 && a->pgram != nullptr;
-    if (room) {
+    // Peaks without a periodogram, of either type: the coarse grid only finds
+    // the chunks that can hold them, and the direct tile sweeps those, so that
+    // the results are the direct sums' whatever the route.
+    const bool screen_room = te && te->prep && w->slices == 1 && a->num_freqs >= kIpMinFreqs &&
+                             a->num_freqs < kIpMaxFreqs && (double)n * (double)a->num_freqs >= kIpMinTermsScreen;
+    w->screen = screen_room && a->pgram == nullptr && a->top_k > 0;
+    w->interp = w->screen || (room && a->dtype == LSAMD_F32 && a->pgram != nullptr);
+    if (room || screen_room) {
         w->obj_ip = take(sizeof(InterpObj) * K);
         w->ip_tab = take((size_t)16 * 64 * 6 * kIpModes);
         w->cand = take((size_t)8 * K * ((w->chunks + 63) / 64));
@@ -758,7 +767,9 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
                  (split && gen) ? 1 : 0, obj_shift, obj_scale, obj_gen,
                  mfma ? reinterpret_cast<float *>(ws + w.obj_ys) : nullptr, a->t,
                  mfma ? reinterpret_cast<double *>(ws + w.rec_t) : nullptr,
-                 mfma ? reinterpret_cast<double2 *>(ws + w.rec_r) : nullptr, obj_ip, dw * kInv2Pi};
+                 mfma ? reinterpret_cast<double2 *>(ws + w.rec_r) : nullptr, obj_ip, dw * kInv2Pi,
+                 w.screen ? kIpSigmaScreen : gen ? kIpSigmaGen : kIpSigma,
+                 w.screen ? kIpLeastObsScreen : kIpLeastObs, w.screen ? 1 : 2, w.screen ? 1 : 0};
     if (split) {
         const bool wide = w.slices > 1;  // one long object alone
         void (*fn)(StatsArgs) = wide ? (f64 ? k_obj_stats_split<double, 512> : k_obj_stats_split<float, 512>)
@@ -843,7 +854,9 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
     if (w.interp) {
         sw.obj_ip = obj_ip;
         sw.ip_tab = reinterpret_cast<uint4 *>(ws + w.ip_tab);
-        sw.ip_items = (a->num_freqs + kIpLeastBins - 1) / kIpLeastBins;
+        const uint32_t least = w.screen ? kIpLeastBinsScreen : kIpLeastBins;
+        sw.ip_items = (a->num_freqs + least - 1) / least;
+        sw.ip_margin = w.screen ? kIpMarginScreen : kIpMargin;
         sw.cand_words = (w.chunks + 63) / 64;
     }
 
@@ -889,13 +902,18 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
         // The coarse-grid sweep, the marks of the chunks to sweep again and the
         // direct tile's tables (which replace the coarse ones) in one launch,
         // then the direct tile over those chunks and the objects in direct mode.
-        const InterpEntry &ip = kInterp[gen ? 1 : 0];
+        const InterpEntry &ip = kInterp[w.screen ? 1 : 0][gen ? 1 : 0][f64 ? 1 : 0];
         SweepArgs si = sw;
-        si.xcd_run = si.ip_items;
+        // screen: consecutive items of an object per workgroup, where enough
+        // workgroups are left to fill the chip ten times over
+        si.group = 1;
+        while (w.screen && si.group < kIpGroup && (uint64_t)K * si.ip_items / (2 * si.group) >= 8192) si.group *= 2;
+        const uint32_t per_obj = (si.ip_items + si.group - 1) / si.group;
+        si.xcd_run = per_obj;
         void *iargs[] = {&si};
         LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(ip.fac), dim3(K + 3 * kIpModes, gy), dim3(64), iargs, 0,
                                st));
-        const uint64_t ip_groups = (uint64_t)K * si.ip_items, most = 0xFFFFFFFFull / (uint64_t)ip.threads - 1;
+        const uint64_t ip_groups = (uint64_t)K * per_obj, most = 0xFFFFFFFFull / (uint64_t)ip.threads - 1;
         for (uint64_t g = 0; g < ip_groups; g += most) {
             si.item_base = g;
             LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(ip.sweep),
@@ -905,8 +923,11 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
         SweepArgs sd = sw;
         sd.cand = a->top_k > 0 ? reinterpret_cast<uint64_t *>(ws + w.cand) : nullptr;
         sd.queue = nullptr;
-        // workgroups per object: ~16 rounds of the chip, or one per item
-        sd.cand_split = (uint32_t)std::min<uint64_t>(w.chunks, std::max<uint64_t>(1, 16384 / K));
+        // workgroups per object: 8 rounds of the chip over all objects (most
+        // find nothing to do), and at most 32 chunks of an object in direct mode
+        // each (8000 objects x 196 chunks, 10% of them direct: 2.2 ms with 98
+        // chunks each, 1.7 with 28)
+        sd.cand_split = (uint32_t)std::min<uint64_t>(w.chunks, std::max<uint64_t>(16384 / K, (w.chunks + 31) / 32));
         sd.xcd_run = sd.cand_split;
         void *dargs[] = {&sd};
         LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->prep), dim3(K, gy + (sd.cand ? 1u : 0u)), dim3(64),

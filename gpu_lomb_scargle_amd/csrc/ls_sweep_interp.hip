@@ -15,17 +15,27 @@
 // or 3; the interpolation itself is a matrix product with a constant 16-point
 // (or 32-point) operand, on the matrix cores as well.
 //
-// Measured (FP32, top-1, kernel ms of the whole sweep, direct -> coarse): 1000
-// objects (164,000 observations) x 10^6 bins, standard, 23 bins per resolution
-// element, h = 10: 10.4 -> 2.84; 250 objects (42,700) x 429,119, generalized,
-// ten bins, h = 4: 2.0 -> 0.68.  k_sweep_interp takes 2.8 ms of the first:
-// 0.9 the coarse points, 2.0 the interpolation and the FP64 powers (22 FP64
-// instructions per bin; VALU 58% and matrix cores 16% of the SIMD cycles at 2.0
-// GHz), of which the stores 0.2 and the bins past the condition bound 0.04.
-// Tried on the way: points of one sign per row factor (3.47 ms: twice the
-// MFMAs and row factors), three wavefronts per standard workgroup (2.99: six
-// wavefronts fit a CU instead of eight), a branch per bin around the store
-// (its FP64 chains then run one after another: 5.1 against 4.5).
+// FP32 periodograms, measured (top-1, ms of the whole sweep, direct -> coarse):
+// 1000 objects (164,000 observations) x 10^6 bins, standard, 23 bins per
+// resolution element, h = 10: 10.5 -> 2.84; 250 objects (42,700) x 429,119,
+// generalized, ten bins, h = 4: 2.0 -> 0.68.  k_sweep_interp takes 2.6 ms of
+// the first: a third the coarse points, the rest the interpolation and the
+// FP64 powers (22 FP64 instructions per bin; VALU 58% and matrix cores 16% of
+// the SIMD cycles at 2.0 GHz), the stores 0.2 and the bins past the condition
+// bound 0.04.  Tried on the way: points of one sign per row factor (3.47 ms:
+// twice the MFMAs and row factors), three wavefronts per standard workgroup
+// (2.99: six wavefronts fit a CU instead of eight), a branch per bin around
+// the store (its FP64 chains then run one after another: 5.1 against 4.5).
+//
+// Peaks without a periodogram (SCREEN): the powers only choose which chunks of
+// 1024 bins the direct tile sweeps, so FP16 heads alone, six taps, larger
+// steps and FP32 powers do: the powers near the peak are good to 7e-3 at worst
+// (17 observations of uneven weight), 1e-3 typically, against a margin of
+// 1/8.  The results are the direct sums', bit for bit.  Measured: 8000 uneven
+// objects x 200,000 bins, top-3, standard FP64, 4.7 bins per resolution
+// element, h = 3: 13.1 -> 5.2 ms (screen 3.1, the marked chunks and the objects
+// of at most 16 observations 1.6, tables 0.45); 1000 objects x 500,000,
+// generalized, 10.5 bins, h = 8: 11.2 -> 1.4 ms.
 #include <type_traits>
 
 #include "ls_split_device.h"
@@ -55,10 +65,11 @@ __device__ double bessel_i0(double x) {  // power series, 0 <= x < 20
     return sum;
 }
 
+template <bool SCREEN>
 __device__ void interp_table(uint4 *tab, int mode, int f) {  // f: sums at f; at 2 f, rows 0..15; 16..31
     const int lane = (int)threadIdx.x;
-    const int h = ip_step(mode), W = ip_taps(mode);
-    const double beta = ip_beta(mode);
+    const int h = ip_step(mode), W = ip_taps(SCREEN);
+    const double beta = ip_beta(SCREEN);
     // phi(x) = I0(beta sqrt(1 - (2x/W)^2)) / Phi(0), Phi(0) = W sinh(beta) / beta
     const double norm = 1024.0 * beta / ((double)W * sinh(beta));
     const double pos = (f == 0 ? 1.0 : 2.0) * (double)(lane & 31) / (double)h;
@@ -85,6 +96,20 @@ __device__ void interp_table(uint4 *tab, int mode, int f) {  // f: sums at f; at
     dst[64] = u;
 }
 
+// e^{2 pi i f t} from the FP64 phase: in FP64, or (screen) by the hardware FP32
+// sine and cosine (1e-7, below the FP16 heads' 5e-4).
+template <bool SCREEN>
+__device__ __forceinline__ void ip_phasor(double f, double t, double &c, double &s) {
+    if constexpr (SCREEN) {
+        const double n = __builtin_rint(f * t);
+        const float r = (float)fma(f, t, -n);
+        c = (double)__builtin_amdgcn_cosf(r);
+        s = (double)__builtin_amdgcn_sinf(r);
+    } else {
+        phasor64(f, t, c, s);
+    }
+}
+
 // Workgroups past the last object write the interpolation operands (blockIdx.x
 // = K + 3 (mode - 1) + which third).  Wavefronts (object, y) write the tables of the object's 16-observation
 // blocks y, y + gridDim.y, ..., as k_colfac does for the direct tile, into the
@@ -92,11 +117,12 @@ __device__ void interp_table(uint4 *tab, int mode, int f) {  // f: sums at f; at
 // two weights a = y (generalized: (w/W) (y - ybar)) and a = 1 (w/W), four head
 // and tail fragments each, and the row steps e^{2 pi i 64 a h df t'} (a < 32),
 // with t' = t - tc and 1/Phi from the records.
-template <bool GEN, typename IN>
+template <bool GEN, typename IN, bool SCREEN>
 __global__ __launch_bounds__(64) void k_interp_fac(SweepArgs a) {
+    constexpr int FR = ip_frags(SCREEN), NC = SCREEN ? 1 : 2;  // fragments; heads alone or with tails
     const uint32_t k = blockIdx.x, l = threadIdx.x;
     if (k >= a.K) {
-        if (blockIdx.y == 0) interp_table(a.ip_tab, (int)(k - a.K) / 3 + 1, (int)(k - a.K) % 3);
+        if (blockIdx.y == 0) interp_table<SCREEN>(a.ip_tab, (int)(k - a.K) / 3 + 1, (int)(k - a.K) % 3);
         return;
     }
     const int mode = (int)a.obj_ip[k].mode;
@@ -117,7 +143,7 @@ __global__ __launch_bounds__(64) void k_interp_fac(SweepArgs a) {
     uint4 *dst = a.colfac + colfac_slot(beg, k) * (uint64_t)(NF * 64) + l;
     uint4 *rdst = a.rowfac + colfac_slot(beg, k) * (uint64_t)(kRowfacFrags * 64) + l;
     for (uint32_t q = blockIdx.y; q * 16u < n; q += gridDim.y) {
-        half8_t f[kIpFrags];
+        half8_t f[FR];
 #pragma unroll
         for (int v = 0; v < 8; v += 2) {
             double x[4][2];
@@ -129,10 +155,10 @@ __global__ __launch_bounds__(64) void k_interp_fac(SweepArgs a) {
                 if (j < n) {
                     const double2 tp = a.rec_r[beg + j];  // t', 1/Phi
                     double c, sn;
-                    phasor64(fr, tp.x, c, sn);
+                    ip_phasor<SCREEN>(fr, tp.x, c, sn);
                     r4[2 * e] = (float)c;
                     r4[2 * e + 1] = (float)sn;
-                    phasor64(fb, tp.x, cb, sb);
+                    ip_phasor<SCREEN>(fb, tp.x, cb, sb);
                     double w = 1.0, yj = (double)y[beg + j];
                     if constexpr (GEN) {
                         const double d = (double)dy[beg + j];
@@ -154,15 +180,17 @@ __global__ __launch_bounds__(64) void k_interp_fac(SweepArgs a) {
             for (int p = 0; p < 4; ++p) {
                 half2_t hd, tl;
                 split64x2(x[p][0], x[p][1], hd, tl);
-                f[2 * p][v] = hd.x; f[2 * p][v + 1] = hd.y;
-                f[2 * p + 1][v] = tl.x; f[2 * p + 1][v + 1] = tl.y;
+                f[NC * p][v] = hd.x; f[NC * p][v + 1] = hd.y;
+                if constexpr (!SCREEN) {
+                    f[2 * p + 1][v] = tl.x; f[2 * p + 1][v + 1] = tl.y;
+                }
             }
         }
 #pragma unroll
-        for (int i = 0; i < kIpFrags; ++i) {
+        for (int i = 0; i < FR; ++i) {
             uint4 u;
             __builtin_memcpy(&u, &f[i], sizeof(u));
-            dst[(uint64_t)(q * kIpFrags + i) * 64] = u;
+            dst[(uint64_t)(q * FR + i) * 64] = u;
         }
     }
 }
@@ -171,6 +199,7 @@ __global__ __launch_bounds__(64) void k_interp_fac(SweepArgs a) {
 struct UnitFrags {
     half8_t r_h, r_l, i_h, i_l;
 };
+template <bool SCREEN>
 __device__ __forceinline__ void unit_factors(const float2 *s_u0, uint32_t j0, uint32_t kh,
                                              const uint4 (&rr)[kRowfacFrags], UnitFrags &R) {
 #pragma unroll
@@ -186,6 +215,13 @@ __device__ __forceinline__ void unit_factors(const float2 *s_u0, uint32_t j0, ui
             ui[e] = fmaf(b.x, ry[e], b.y * rx[e]);
         }
         half2_t h, t;
+        if constexpr (SCREEN) {
+            h = __builtin_convertvector((float2_t){ur[0], ur[1]}, half2_t);
+            R.r_h[v] = h.x; R.r_h[v + 1] = h.y;
+            h = __builtin_convertvector((float2_t){ui[0], ui[1]}, half2_t);
+            R.i_h[v] = h.x; R.i_h[v + 1] = h.y;
+            continue;
+        }
         split16x2(ur[0], ur[1], h, t);
         R.r_h[v] = h.x; R.r_h[v + 1] = h.y;
         R.r_l[v] = t.x; R.r_l[v + 1] = t.y;
@@ -193,6 +229,12 @@ __device__ __forceinline__ void unit_factors(const float2 *s_u0, uint32_t j0, ui
         R.i_h[v] = h.x; R.i_h[v + 1] = h.y;
         R.i_l[v] = t.x; R.i_l[v + 1] = t.y;
     }
+}
+
+// A value that is the same in all lanes, held in scalar registers.
+__device__ __forceinline__ double uniform(double v) { return lane_value(v, 0); }
+__device__ __forceinline__ float uniform(float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
 }
 
 // Orders a wavefront's LDS writes before its own later reads (LDS operations
@@ -238,28 +280,29 @@ __device__ __forceinline__ float wave_fmax(float x) {
 // when a row spans more than 16), B = the table, three products each.  The
 // power, the condition bound and its FP64 recomputation are the direct tile's.
 // ---------------------------------------------------------------------------
-template <bool GEN>
-__global__ __launch_bounds__(256, 2) void k_sweep_interp(SweepArgs a) {
+template <bool GEN, typename IN, bool SCREEN>
+__global__ __launch_bounds__(256, SCREEN ? 3 : 2) void k_sweep_interp(SweepArgs a) {
+    static_assert(SCREEN || sizeof(IN) == 4, "periodograms: FP32");
+    constexpr int NC = SCREEN ? 1 : 2, FR = ip_frags(SCREEN);
     constexpr int NW = 4, NZ = GEN ? 2 : 1;
     constexpr uint32_t kFoldObs = 256;
     constexpr int kZ = 2048 + 32, kX = 4096 + 32;  // points and zeros read past them
     __shared__ float2 s_u0[NW][64];
-    __shared__ __align__(16) _Float16 s_z[NZ][2][2][kZ];  // [sum][re, im][head, tail]
-    __shared__ __align__(16) _Float16 s_x[2][2][kX];
-    const uint32_t l = threadIdx.x & 63u, rc = l & 31u, kh = l >> 5;
+    __shared__ __align__(16) _Float16 s_z[NZ][2][NC][kZ];  // [sum][re, im][head, tail]
+    __shared__ __align__(16) _Float16 s_x[2][NC][kX];
+    const uint32_t l = threadIdx.x & 63u;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint64_t g = a.item_base + grid_group(a);
-    const uint32_t pos = (uint32_t)(g / a.ip_items), it = (uint32_t)(g - (uint64_t)pos * a.ip_items);
+    const uint32_t per_obj = (a.ip_items + a.group - 1u) / a.group;  // workgroups
+    const uint32_t pos = (uint32_t)(g / per_obj), it0 = (uint32_t)(g - (uint64_t)pos * per_obj) * a.group;
     if (pos >= a.K) return;
     const uint32_t obj = a.order ? a.order[pos] : pos;
     const int mode = (int)a.obj_ip[obj].mode;
     if (mode == 0) return;
     const uint32_t h = (uint32_t)ip_step(mode), m = (uint32_t)ip_per_row(mode), rb = h * m;
     const uint32_t rows = (uint32_t)ip_rows(mode);
-    const uint64_t kbase64 = (uint64_t)it * (rows * rb);
-    if (kbase64 >= a.nf) return;
-    const uint32_t kbase = (uint32_t)kbase64;
-    constexpr int W = kIpTaps;
+    if ((uint64_t)it0 * (rows * rb) >= a.nf) return;
+    constexpr int W = ip_taps(SCREEN);
 
     const uint64_t obeg = a.offsets[obj], oend = a.offsets[obj + 1];
     const uint32_t n = (uint32_t)(oend - obeg);
@@ -267,114 +310,7 @@ __global__ __launch_bounds__(256, 2) void k_sweep_interp(SweepArgs a) {
     // |G| <= n max(1/Phi) 2^10 < n 2^12: into FP16's range
     const float gs = ldexpf(1.0f, 3 - (32 - __clz((int)n)));
     const bool at2f = wave >= (uint32_t)NZ;
-    if (GEN || wave < 3u) {
-        const double step = (double)h * a.df_rev;
-        double f0 = a.fmin_rev + (double)kbase * a.df_rev;
-        if (at2f) f0 = 2.0 * f0 + (wave > (uint32_t)NZ ? 2048.0 * step : 0.0);
-        f0 += (31.5 - (double)(W / 2 - 1)) * step;  // the first row's middle
-        constexpr int NF = GEN ? kColfacFragsGen : kColfacFragsStd;
-        const uint64_t slot = colfac_slot(obeg, obj);
-        const uint4 *cf = a.colfac + slot * (uint64_t)(NF * 64) + (wave == 0 ? 0 : 4 * 64) + l;
-        const uint4 *rf = a.rowfac + slot * (uint64_t)(kRowfacFrags * 64) + l;
-        f32x16_t sum[4] = {}, cross[4] = {};  // A, B, C, D: head x head, cross products
-        // sums of whole 256-observation runs, in the room of this wavefront's
-        // points: entry i of lane l, each lane its own
-        _Float16 *const base = at2f ? &s_x[0][0][0] + 2048u * (wave - NZ) : &s_z[wave < NZ ? wave : 0][0][0][0];
-        const uint32_t len = at2f ? kX : kZ;
-        auto run_sum = [&](int q, int v) { return reinterpret_cast<float *>(base + (uint32_t)q * len) + 64 * v + l; };
-        bool folded = false;
-        uint4 rr[kRowfacFrags];
-        load_rows(rf, rr);
-        for (uint32_t g0 = 0; g0 < n; g0 += kFoldObs) {
-            const uint32_t gend = n - g0 < kFoldObs ? n : g0 + kFoldObs;
-            for (uint32_t b0 = g0; b0 < gend; b0 += 64) {
-                const uint32_t cnt = gend - b0 < 64u ? gend - b0 : 64u;
-                float2 u0 = make_float2(0.0f, 0.0f);
-                if (l < cnt) {
-                    double c, sn;
-                    phasor64(f0, a.rec_r[obeg + b0 + l].x, c, sn);
-                    u0 = make_float2((float)c, (float)sn);
-                }
-                wave_lds_fence();
-                s_u0[wave][l] = u0;
-                wave_lds_fence();
-                for (uint32_t j0 = 0; j0 < cnt; j0 += 16, cf += kIpFrags * 64, rf += kRowfacFrags * 64) {
-                    half8_t col[4];
-                    load_cols<4>(cf, col);
-                    UnitFrags R;
-                    unit_factors(s_u0[wave], j0, kh, rr, R);
-                    load_rows(rf + kRowfacFrags * 64, rr);  // the next block's (one slot past the end is allocated)
-                    LS_MFMA(sum[0], R.r_h, col[0]);
-                    LS_MFMA(cross[0], R.r_h, col[1]);
-                    LS_MFMA(cross[0], R.r_l, col[0]);
-                    LS_MFMA(sum[2], R.r_h, col[2]);
-                    LS_MFMA(cross[2], R.r_h, col[3]);
-                    LS_MFMA(cross[2], R.r_l, col[2]);
-                    LS_MFMA(sum[1], R.i_h, col[2]);
-                    LS_MFMA(cross[1], R.i_h, col[3]);
-                    LS_MFMA(cross[1], R.i_l, col[2]);
-                    LS_MFMA(sum[3], R.i_h, col[0]);
-                    LS_MFMA(cross[3], R.i_h, col[1]);
-                    LS_MFMA(cross[3], R.i_l, col[0]);
-                }
-            }
-            if (gend < n) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-#pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        float *r = run_sum(q, v);
-                        *r = (folded ? *r : 0.0f) + (sum[q][v] + cross[q][v]);
-                    }
-                    sum[q] = f32x16_t{};
-                    cross[q] = f32x16_t{};
-                }
-                folded = true;
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < 4; ++q) sum[q] += cross[q];
-        if (folded) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) sum[q][v] += *run_sum(q, v);
-            wave_lds_fence();  // all read before the points overwrite them
-        }
-#pragma unroll
-        for (int v = 0; v < 16; v += 2) {
-            // row 8 (v / 4) + 4 kh + v % 4, point 64 row + 32 + b and 64 row + 31 - b; v + 1: 64 on
-            const uint32_t ip = 64u * (8u * (uint32_t)(v / 4) + 4u * kh + (uint32_t)(v % 4)) + 32u + rc, im = ip - 1u - 2u * rc;
-            half2_t hd, tl;
-            auto put = [&](int c, uint32_t at, float x0, float x1) {
-                split16x2(x0 * gs, x1 * gs, hd, tl);
-                base[2 * c * len + at] = hd.x; base[2 * c * len + at + 64] = hd.y;
-                base[(2 * c + 1) * len + at] = tl.x; base[(2 * c + 1) * len + at + 64] = tl.y;
-            };
-            put(0, ip, sum[0][v] - sum[1][v], sum[0][v + 1] - sum[1][v + 1]);
-            put(1, ip, sum[2][v] + sum[3][v], sum[2][v + 1] + sum[3][v + 1]);
-            put(0, im, sum[0][v] + sum[1][v], sum[0][v + 1] + sum[1][v + 1]);
-            put(1, im, sum[3][v] - sum[2][v], sum[3][v + 1] - sum[2][v + 1]);
-        }
-        if (l < 32) {  // zeros past the last point (a window's unused rows meet them with weight 0)
-            if (wave < (uint32_t)NZ) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) base[c * kZ + 2048 + l] = (_Float16)0.0f;
-            } else if (wave == (uint32_t)NZ) {
-#pragma unroll
-                for (int c = 0; c < 4; ++c) base[c * kX + 4096 + l] = (_Float16)0.0f;
-            }
-        }
-    }
-    __syncthreads();
-
-    // the table's operands (fragments 4, 5: rows 16..31 of the sums at 2 f)
-    half8_t tb[6];
-    load_cols<6>(a.ip_tab + (mode - 1) * (6 * 64) + l, tb);
     const bool wide = 2u * m - 1u + (uint32_t)W > 16u;
-    const uint32_t left = a.nf - kbase;
-    const uint32_t rows_here = left < rows * rb ? (left + rb - 1u) / rb : rows;
-
     const double un = 1.0 / ((double)kFacScale * 1024.0 * (double)gs);  // power of two
     const double uy = un / (double)ys, uw = un / (double)ws;
     const double scale = a.obj_scale[obj];
@@ -392,12 +328,156 @@ __global__ __launch_bounds__(256, 2) void k_sweep_interp(SweepArgs a) {
     }
     // generalized: gen_power with y in units of its result
     const double iW = 1.0 / Wf, sw = uw * iW, sy = uy * iW, hsw = 0.5 * sw, ybu = Yb / sy, kg = sy * sy / YY * scale;
+    typedef std::conditional_t<SCREEN, float, double> R;
+    const R rsw = uniform((R)sw), rhsw = uniform((R)hsw), rybu = uniform((R)ybu), rkg = uniform((R)kg);
+    const R rhn = uniform((R)hn), rhn2 = uniform((R)hn2), rdmin = uniform((R)dmin), rkp = uniform((R)kp);
+    const R rcond = (R)kCondMax;
+    // screen: a.group workgroups' worths of bins in turn, the object's constants
+    // and addresses stay (its workgroups are short)
+    auto sweep_item = [&](const uint32_t it, const uint32_t l) {
+    const uint32_t rc = l & 31u, kh = l >> 5;
+    const uint32_t kbase = it * (rows * rb);
+    if (GEN || wave < 3u) {
+        const double step = (double)h * a.df_rev;
+        double f0 = a.fmin_rev + (double)kbase * a.df_rev;
+        if (at2f) f0 = 2.0 * f0 + (wave > (uint32_t)NZ ? 2048.0 * step : 0.0);
+        f0 += (31.5 - (double)(W / 2 - 1)) * step;  // the first row's middle
+        constexpr int NF = GEN ? kColfacFragsGen : kColfacFragsStd;
+        const uint64_t slot = colfac_slot(obeg, obj);
+        const uint4 *cf = a.colfac + slot * (uint64_t)(NF * 64) + (wave == 0 ? 0 : FR / 2 * 64) + l;
+        const uint4 *rf = a.rowfac + slot * (uint64_t)(kRowfacFrags * 64) + l;
+        f32x16_t sum[4] = {}, cross[SCREEN ? 1 : 4] = {};  // A, B, C, D: head x head, cross products
+        // sums of whole 256-observation runs, in the room of this wavefront's
+        // points: entry i of lane l, each lane its own
+        _Float16 *const base = at2f ? &s_x[0][0][0] + 2048u * (wave - NZ) : &s_z[wave < NZ ? wave : 0][0][0][0];
+        const uint32_t len = at2f ? kX : kZ;
+        auto run_sum = [&](int q, int v) { return reinterpret_cast<float *>(base + (uint32_t)q * len) + 64 * v + l; };
+        constexpr bool kRuns = !SCREEN;  // the screen's sums stay in the accumulators
+        bool folded = false;
+        uint4 rr[kRowfacFrags];
+        load_rows(rf, rr);
+        half8_t next[FR / 2];
+        if constexpr (SCREEN) load_cols<FR / 2>(cf, next);
+        for (uint32_t g0 = 0; g0 < n; g0 += kRuns ? kFoldObs : n) {
+            const uint32_t gend = !kRuns || n - g0 < kFoldObs ? n : g0 + kFoldObs;
+            for (uint32_t b0 = g0; b0 < gend; b0 += 64) {
+                const uint32_t cnt = gend - b0 < 64u ? gend - b0 : 64u;
+                float2 u0 = make_float2(0.0f, 0.0f);
+                if (l < cnt) {
+                    double c, sn;
+                    ip_phasor<SCREEN>(f0, a.rec_r[obeg + b0 + l].x, c, sn);
+                    u0 = make_float2((float)c, (float)sn);
+                }
+                wave_lds_fence();
+                s_u0[wave][l] = u0;
+                wave_lds_fence();
+                for (uint32_t j0 = 0; j0 < cnt; j0 += 16, cf += FR * 64, rf += kRowfacFrags * 64) {
+                    half8_t col[FR / 2];
+                    if constexpr (SCREEN) {  // one block ahead, as the rows
+#pragma unroll
+                        for (int i = 0; i < FR / 2; ++i) col[i] = next[i];
+                        load_cols<FR / 2>(cf + FR * 64, next);
+                    } else {
+                        load_cols<FR / 2>(cf, col);
+                    }
+                    UnitFrags R;
+                    unit_factors<SCREEN>(s_u0[wave], j0, kh, rr, R);
+                    load_rows(rf + kRowfacFrags * 64, rr);  // the next block's (one slot past the end is allocated)
+                    if constexpr (SCREEN) {
+                        LS_MFMA(sum[0], R.r_h, col[0]);
+                        LS_MFMA(sum[1], R.i_h, col[1]);
+                        LS_MFMA(sum[2], R.r_h, col[1]);
+                        LS_MFMA(sum[3], R.i_h, col[0]);
+                    } else {
+                        LS_MFMA(sum[0], R.r_h, col[0]);
+                        LS_MFMA(cross[0], R.r_h, col[1]);
+                        LS_MFMA(cross[0], R.r_l, col[0]);
+                        LS_MFMA(sum[2], R.r_h, col[2]);
+                        LS_MFMA(cross[2], R.r_h, col[3]);
+                        LS_MFMA(cross[2], R.r_l, col[2]);
+                        LS_MFMA(sum[1], R.i_h, col[2]);
+                        LS_MFMA(cross[1], R.i_h, col[3]);
+                        LS_MFMA(cross[1], R.i_l, col[2]);
+                        LS_MFMA(sum[3], R.i_h, col[0]);
+                        LS_MFMA(cross[3], R.i_h, col[1]);
+                        LS_MFMA(cross[3], R.i_l, col[0]);
+                    }
+                }
+            }
+            if constexpr (kRuns) {
+                if (gend < n) {
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) {
+                            float *r = run_sum(q, v);
+                            *r = (folded ? *r : 0.0f) + (sum[q][v] + cross[q][v]);
+                        }
+                        sum[q] = f32x16_t{};
+                        cross[q] = f32x16_t{};
+                    }
+                    folded = true;
+                }
+            }
+        }
+        if constexpr (kRuns) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) sum[q] += cross[q];
+            if (folded) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) sum[q][v] += *run_sum(q, v);
+                wave_lds_fence();  // all read before the points overwrite them
+            }
+        }
+        if (SCREEN && it != it0) __syncthreads();  // the last tiles' points are read
+#pragma unroll
+        for (int v = 0; v < 16; v += 2) {
+            // row 8 (v / 4) + 4 kh + v % 4, point 64 row + 32 + b and 64 row + 31 - b; v + 1: 64 on
+            const uint32_t ip = 64u * (8u * (uint32_t)(v / 4) + 4u * kh + (uint32_t)(v % 4)) + 32u + rc, im = ip - 1u - 2u * rc;
+            half2_t hd, tl;
+            auto put = [&](int c, uint32_t at, float x0, float x1) {
+                if constexpr (SCREEN) hd = __builtin_convertvector((float2_t){x0 * gs, x1 * gs}, half2_t);
+                else split16x2(x0 * gs, x1 * gs, hd, tl);
+                base[NC * c * len + at] = hd.x; base[NC * c * len + at + 64] = hd.y;
+                if constexpr (!SCREEN) {
+                    base[(2 * c + 1) * len + at] = tl.x; base[(2 * c + 1) * len + at + 64] = tl.y;
+                }
+            };
+            put(0, ip, sum[0][v] - sum[1][v], sum[0][v + 1] - sum[1][v + 1]);
+            put(1, ip, sum[2][v] + sum[3][v], sum[2][v + 1] + sum[3][v + 1]);
+            put(0, im, sum[0][v] + sum[1][v], sum[0][v + 1] + sum[1][v + 1]);
+            put(1, im, sum[3][v] - sum[2][v], sum[3][v + 1] - sum[2][v + 1]);
+        }
+        if (l < 32) {  // zeros past the last point (a window's unused rows meet them with weight 0)
+            if (wave < (uint32_t)NZ) {
+#pragma unroll
+                for (int c = 0; c < 2 * NC; ++c) base[c * kZ + 2048 + l] = (_Float16)0.0f;
+            } else if (wave == (uint32_t)NZ) {
+#pragma unroll
+                for (int c = 0; c < 2 * NC; ++c) base[c * kX + 4096 + l] = (_Float16)0.0f;
+            }
+        }
+    } else if (SCREEN && it != it0) {
+        __syncthreads();  // as the other wavefronts, before their points
+    }
+    // the table's operands (fragments 4, 5: rows 16..31 of the sums at 2 f)
+    half8_t tb[6];
+#pragma unroll
+    for (int i = 0; i < 6; i += SCREEN ? 2 : 1) {  // (the screen uses the heads)
+        const uint4 u = a.ip_tab[((mode - 1) * 6 + i) * 64 + (int)l];
+        __builtin_memcpy(&tb[i], &u, sizeof(u));
+    }
+    __syncthreads();
     float *tmax = reinterpret_cast<float *>(a.part_pow + (uint64_t)obj * a.chunks * kPeaks) + 3u * it * ((rows + 31u) / 32u);
+    const uint32_t left = a.nf - kbase;
+    const uint32_t rows_here = left < rows * rb ? (left + rb - 1u) / rb : rows;
     // Stores past the workgroup's bins (rows of the next one, the grid's end,
     // lanes beyond rb) are dropped by the buffer's range: no branch per bin, so
     // that the bins' FP64 chains overlap.
     const uint32_t bin_end = left < rows * rb ? a.nf : kbase + rows * rb;
-    float *pg = static_cast<float *>(a.pgram) + (uint64_t)obj * a.nf;
+    float *pg = SCREEN ? nullptr : static_cast<float *>(a.pgram) + (uint64_t)obj * a.nf;
     const auto out = __builtin_amdgcn_make_buffer_rsrc(pg, 0, (int)(bin_end * 4u), 0x00027000);
 
     for (uint32_t tile = wave; 32u * tile < rows_here; tile += NW) {
@@ -406,9 +486,11 @@ __global__ __launch_bounds__(256, 2) void k_sweep_interp(SweepArgs a) {
         auto product = [&](const _Float16 *gh, const _Float16 *gt, const half8_t &th, const half8_t &tt, f32x16_t &acc) {
             half8_t ah, at;
             __builtin_memcpy(&ah, __builtin_assume_aligned(gh, 2), 16);
-            __builtin_memcpy(&at, __builtin_assume_aligned(gt, 2), 16);
-            LS_MFMA(acc, at, th);
-            LS_MFMA(acc, ah, tt);
+            if constexpr (!SCREEN) {
+                __builtin_memcpy(&at, __builtin_assume_aligned(gt, 2), 16);
+                LS_MFMA(acc, at, th);
+                LS_MFMA(acc, ah, tt);
+            }
             LS_MFMA(acc, ah, th);
         };
         const uint32_t zo = m * s + 8u * kh, xo = 2u * m * s + 8u * kh;
@@ -417,66 +499,73 @@ __global__ __launch_bounds__(256, 2) void k_sweep_interp(SweepArgs a) {
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 z[2 * q + c] = f32x16_t{};
-                product(&s_z[q][c][0][zo], &s_z[q][c][1][zo], tb[0], tb[1], z[2 * q + c]);
+                product(&s_z[q][c][0][zo], &s_z[q][c][NC - 1][zo], tb[0], tb[1], z[2 * q + c]);
             }
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             x[c] = f32x16_t{};
-            product(&s_x[c][0][xo], &s_x[c][1][xo], tb[2], tb[3], x[c]);
-            if (wide) product(&s_x[c][0][xo + 16], &s_x[c][1][xo + 16], tb[4], tb[5], x[c]);
+            product(&s_x[c][0][xo], &s_x[c][NC - 1][xo], tb[2], tb[3], x[c]);
+            if (wide) product(&s_x[c][0][xo + 16], &s_x[c][NC - 1][xo + 16], tb[4], tb[5], x[c]);
         }
         // result entry v: row 8 (v / 4) + 4 kh + v % 4 of the tile, bin rb row + rc
         const uint32_t bin0 = kbase + rb * (32u * tile + 4u * kh) + rc;
         const uint32_t off0 = rc < rb ? bin0 : 0x3FFF0000u;  // past any bin_end (nf < kIpMaxFreqs)
         // power of entry v, and whether its condition number exceeds the bound
-        auto power = [&](int v, bool &ill) -> float {
-            double num, D;
-            if constexpr (GEN) {
-                const double C = (double)z[2][v] * sw, S = (double)z[3][v] * sw;
-                const double half = fma((double)x[0][v], hsw, 0.5);
-                const double CC = fma(-C, C, half), SS = fma(-S, S, 1.0 - half);
-                const double CS = fma(-C, S, (double)x[1][v] * hsw);
-                const double yc = fma(-ybu, C, (double)z[0][v]), ysn = fma(-ybu, S, (double)z[1][v]);
-                D = fma(CC, SS, -(CS * CS));
-                const double t = fma(C, C, S * S);  // (1 + t) (CC + SS) = 1 - t^2
-                ill = !(fma(-t, t, 1.0) <= kCondMax * D) | !(D > 0.0);
-                num = kg * fma(SS, yc * yc, fma(CC, ysn * ysn, -2.0 * CS * (yc * ysn)));
-            } else {
-                const double XC = (double)z[0][v], XS = (double)z[1][v], c = (double)x[0][v], sn = (double)x[1][v];
-                D = fma(-c, c, fma(-sn, sn, hn2));
-                ill = !(D >= dmin);
-                const double q = XC * XC;
-                num = kp * fma(hn, fma(XS, XS, q), -fma(c, fma(-XS, XS, q), (sn + sn) * (XC * XS)));
-            }
-            // num / D, the hardware reciprocal's error e taken off to third order
-            const double r = __builtin_amdgcn_rcp(D), e = fma(-D, r, 1.0);
-            return (float)(num * fma(r, fma(e, e, e), r));
+        // (the screen's in FP32: a few 1e-6 beside the heads' ~1e-3)
+        auto fm = [](R p, R q, R r) {
+            if constexpr (SCREEN) return fmaf(p, q, r);
+            else return fma(p, q, r);
         };
-        float best = 0.0f;
-        bool any_ill = false;
+        auto power = [&](int v, bool &ill) -> float {
+            R num, D;
+            if constexpr (GEN) {
+                const R C = (R)z[2][v] * rsw, S = (R)z[3][v] * rsw;
+                const R half = fm((R)x[0][v], rhsw, (R)0.5);
+                const R CC = fm(-C, C, half), SS = fm(-S, S, (R)1.0 - half);
+                const R CS = fm(-C, S, (R)x[1][v] * rhsw);
+                const R yc = fm(-rybu, C, (R)z[0][v]), ysn = fm(-rybu, S, (R)z[1][v]);
+                D = fm(CC, SS, -(CS * CS));
+                const R t = fm(C, C, S * S);  // (1 + t) (CC + SS) = 1 - t^2
+                ill = !(fm(-t, t, (R)1.0) <= rcond * D) | !(D > (R)0.0);
+                num = rkg * fm(SS, yc * yc, fm(CC, ysn * ysn, (R)-2.0 * CS * (yc * ysn)));
+            } else {
+                const R XC = (R)z[0][v], XS = (R)z[1][v], c = (R)x[0][v], sn = (R)x[1][v];
+                D = fm(-c, c, fm(-sn, sn, rhn2));
+                ill = !(D >= rdmin);
+                const R q = XC * XC;
+                num = rkp * fm(rhn, fm(XS, XS, q), -fm(c, fm(-XS, XS, q), (sn + sn) * (XC * XS)));
+            }
+            if constexpr (SCREEN) return num * __builtin_amdgcn_rcpf(D);
+            else {
+                // num / D, the hardware reciprocal's error e taken off to third order
+                const double r = __builtin_amdgcn_rcp(D), e = fma(-D, r, 1.0);
+                return (float)(num * fma(r, fma(e, e, e), r));
+            }
+        };
+        float best = 0.0f, pw[16];
+        uint64_t any_ill = 0u, ills[16];  // lanes of entry v past the condition bound (scalar registers)
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             const uint32_t kf = off0 + rb * (8u * (uint32_t)(v / 4) + (uint32_t)(v % 4));
             bool ill;
-            const float pw = power(v, ill);
-            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(pw), out, kf * 4u, 0, 0);
-            best = fmaxf(best, pw);
-            any_ill |= ill;
+            pw[v] = power(v, ill);
+            if constexpr (!SCREEN) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(pw[v]), out, kf * 4u, 0, 0);
+            best = fmaxf(best, pw[v]);
+            ills[v] = __ballot(ill);
+            any_ill |= ills[v];
         }
         best = rc < rb ? best : 0.0f;
         // rarely: bins past the condition bound, or a tile that the workgroup's
         // last row or the grid's end cuts (whose other entries count for nothing)
         uint32_t flags = 0u;
-        if (kbase + rb * (32u * tile + 32u) > bin_end || __ballot(any_ill) != 0ull) {
+        if (kbase + rb * (32u * tile + 32u) > bin_end || any_ill != 0u) {
             best = 0.0f;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const uint32_t kf = off0 + rb * (8u * (uint32_t)(v / 4) + (uint32_t)(v % 4));
-                bool ill;
-                const float pw = power(v, ill);
                 if (kf < bin_end) {
-                    if (ill) flags |= 1u << v;
-                    else best = fmaxf(best, pw);
+                    if ((ills[v] >> l) & 1u) flags |= 1u << v;
+                    else best = fmaxf(best, pw[v]);
                 }
             }
         }
@@ -485,10 +574,10 @@ __global__ __launch_bounds__(256, 2) void k_sweep_interp(SweepArgs a) {
             const uint32_t src = (uint32_t)__builtin_ctzll(lanes);
             const uint32_t f = (uint32_t)__shfl((int)flags, (int)src, 64), v = (uint32_t)__builtin_ctz(f);
             const uint32_t kf = kbase + rb * (32u * tile + 4u * (src >> 5) + 8u * (v / 4u) + v % 4u) + (src & 31u);
-            const double pe = exact_power<GEN, float>(a, obj, kf);
+            const double pe = exact_power<GEN, IN>(a, obj, kf);
             if (l == src) {
                 const float pw = (float)(pe * scale);
-                pg[kf] = pw;
+                if constexpr (!SCREEN) pg[kf] = pw;
                 best = fmaxf(best, pw);
                 flags &= flags - 1u;
             }
@@ -507,13 +596,25 @@ __global__ __launch_bounds__(256, 2) void k_sweep_interp(SweepArgs a) {
             if (l < 3) tmax[3u * tile + l] = l == 0 ? t0 : l == 1 ? t1 : t2;
         }
     }
+    };
+    if constexpr (SCREEN) {
+        for (uint32_t it = it0; it < it0 + a.group && (uint64_t)it * (rows * rb) < a.nf; ++it) {
+            uint32_t lane = l;  // opaque: nothing derived from it is worth registers across items
+            asm volatile("" : "+v"(lane));
+            sweep_item(it, lane);
+        }
+    } else {
+        sweep_item(it0, l);
+    }
 }
 
 }  // namespace
 
-const InterpEntry kInterp[2] = {
-    {k_interp_fac<false, float>, k_sweep_interp<false>, 256},
-    {k_interp_fac<true, float>, k_sweep_interp<true>, 256},
+#define LS_IP(GEN, IN, SCREEN) {k_interp_fac<GEN, IN, SCREEN>, k_sweep_interp<GEN, IN, SCREEN>, 256}
+
+const InterpEntry kInterp[2][2][2] = {
+    {{LS_IP(false, float, false), {nullptr, nullptr, 0}}, {LS_IP(true, float, false), {nullptr, nullptr, 0}}},
+    {{LS_IP(false, float, true), LS_IP(false, double, true)}, {LS_IP(true, float, true), LS_IP(true, double, true)}},
 };
 
 }  // namespace lsamd

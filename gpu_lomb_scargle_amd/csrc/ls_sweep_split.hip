@@ -643,7 +643,7 @@ __global__ __launch_bounds__(T) void k_sweep_split64(SweepArgs a) {
 // Chunks (1024 bins) that can hold one of an object's top_k bins: those that
 // overlap a result tile whose best power reaches the top_k-th best of the
 // tiles' lane maxima (a lower bound of the top_k-th best power) less
-// kIpMargin.  The direct tile computes them again, so that peaks come from the
+// a.ip_margin.  The direct tile computes them again, so that peaks come from the
 // same arithmetic whichever way the rest of the grid was formed.  One
 // wavefront per object; bit c % 64 of word c / 64.
 // ---------------------------------------------------------------------------
@@ -679,7 +679,7 @@ __device__ void mark_chunks(const SweepArgs &a, uint32_t obj) {
             t2 = 0.0f;
         }
     }
-    const float least = tau * (1.0f - kIpMargin);
+    const float least = tau * (1.0f - a.ip_margin);
     uint64_t *bits = a.cand + (uint64_t)obj * a.cand_words;
     for (uint32_t w = 0; w < a.cand_words; ++w) {
         const uint32_t c = 64u * w + lane;

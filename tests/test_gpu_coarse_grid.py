@@ -1,9 +1,9 @@
-"""The coarse-grid sweep of split32 (FP32 periodograms on grids finer than an
-object's resolution): every mode and its edges against the plain FP64 form on
-the same float inputs, and its peaks against its own periodogram.
-
-Tolerance: the split forms', relative 1e-5 on bins of at least 1e-3 Pmax and
-2e-6 Pmax absolute (tests/test_gpu_parity.py).
+"""The coarse-grid sweep of split32.  FP32 periodograms on grids finer than an
+object's resolution: every mode and its edges against the plain FP64 form on
+the same float inputs, and its peaks against its own periodogram.  Tolerance:
+the split forms', relative 1e-5 on bins of at least 1e-3 Pmax and 2e-6 Pmax
+absolute (tests/test_gpu_parity.py).  Peaks without a periodogram: equal, bit
+for bit, to those of the objects swept one by one, which takes the direct sums.
 """
 import numpy as np
 import pytest
@@ -106,3 +106,46 @@ def test_grid_and_persistent_and_graph_agree(gen):
         torch.cuda.synchronize()
         for k, v in plan.results().items():
             assert torch.equal(v, a[k]), k
+
+
+@pytest.mark.parametrize("gen", [False, True], ids=["standard", "generalized"])
+@pytest.mark.parametrize("dtype", [F32, F64])
+@pytest.mark.parametrize("nf,top_k", [(420007, 1), (420007, 3), (440640, 3), (1000000, 3)])
+def test_peaks_alone_equal_the_direct_sums(nf, top_k, dtype, gen):
+    """Every coarse step and its neighbourhood, observation counts around the
+    blocks and stages, noise without a peak, a pair of equal peaks, constant
+    and NaN magnitudes; persistent and grid schedules."""
+    torch = pytest.importorskip("torch")
+    from gpu_lomb_scargle_amd import device
+    over = np.array([3.5, 3.95, 5.1, 5.3, 6.4, 6.6, 7.7, 7.9, 10.3, 10.5, 12.9, 13.1, 20.5, 21.0, 33.0, 60.0, 9.0, 9.0, 9.0, 9.0])
+    counts = [200, 17, 33, 64, 65, 255, 256, 257, 12, 512, 513, 18, 100, 30, 48, 300, 90, 120, 60, 80]
+    o, t, y, dy = light_curves(counts, nf / DF / over, gen, nf + top_k)
+    first = np.concatenate([[0], np.cumsum(counts)])
+    rng = np.random.default_rng(8)
+    part = lambda k: slice(first[k], first[k + 1])
+    y[part(16)] = rng.normal(0, 1, 90)                                          # noise
+    tk = t[part(17)].astype(F64)
+    y[part(17)] = np.sin(2 * np.pi * 5.0 * tk) + np.sin(2 * np.pi * 11.0 * tk)  # two peaks of one height
+    y[part(18)] = 3.0
+    y[first[19] + 7] = np.nan
+    tt, yy, dd, off = device.numpy_to_device(o, t, y, dy, dtype)
+    kw = dict(min_freq=synth.OMEGA_MIN, max_freq=synth.OMEGA_MAX, num_freqs=nf, form=_native.FORM_SPLIT32, top_k=top_k,
+              variant=_native.GENERALIZED if gen else _native.STANDARD, pgram=False)
+    assert int(first[-1]) * nf >= 1e9  # below, the direct sums
+    got = []
+    for schedule in (_native.SCHEDULE_GRID, _native.SCHEDULE_PERSISTENT):
+        plan = device.SweepPlan(tt, yy, dd, off, schedule=schedule, **kw)
+        for x in (plan.peak_power, plan.peak_period, plan.peak_index):
+            x.fill_(-1)
+        plan.run()
+        torch.cuda.synchronize()
+        got.append({k: v.clone() for k, v in plan.results().items()})
+    for k in range(len(counts)):
+        a = part(k)
+        one = device.SweepPlan(tt[a], yy[a], None if dd is None else dd[a], torch.tensor([0, counts[k]], device="cuda"),
+                               obs_slices=1, **kw)
+        one.run()
+        torch.cuda.synchronize()
+        for name, v in one.results().items():
+            for g in got:
+                assert torch.equal(g[name][k], v[0]), (k, name, g[name][k], v[0])
