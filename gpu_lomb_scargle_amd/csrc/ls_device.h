@@ -58,8 +58,11 @@ struct SweepArgs {
     uint4 *ip_tab;
     uint32_t ip_items;
     float ip_margin;  // of the marked chunks' powers
-    uint32_t cand_words, cand_split;  // words per object; workgroups per object of the direct passes
+    uint32_t cand_words, cand_split;  // words per object; workgroups per object that sweep them,
+    uint32_t marked_groups;           // and of all objects (a multiple of 8)
     uint64_t *cand;
+    // the objects in direct mode, about in processing order, and their number
+    uint32_t *direct_list, *direct_count;
 };
 
 typedef void (*SweepFn)(SweepArgs);
@@ -414,7 +417,10 @@ __device__ __forceinline__ void item_coords_sliced(const SweepArgs &a, uint64_t 
 // order) and, once that queue is exhausted, takes groups from the next ones in
 // turn, so that an object's tables stay in one XCD's L2 while its work lasts
 // and no XCD idles while another has work.
-constexpr uint32_t kQueues = 8;
+// Each counter has a cache line of its own (one line for all eight serialised
+// the ~16,000 fetches that find the queues dry, 0.25 ms), and a queue that
+// reads as exhausted, which it then stays, is passed by without an atomic.
+constexpr uint32_t kQueues = 8, kQueueStride = 16;  // 64-bit counters, words apart
 __device__ __forceinline__ uint64_t queue_group(const SweepArgs &a, uint32_t q, uint64_t i) {
     const uint64_t L = a.xcd_run ? a.xcd_run : 1u;
     const uint64_t rho = i / L, x = (rho & 1u) ? 7u - q : q;
@@ -431,8 +437,9 @@ __device__ __forceinline__ uint64_t fetch_item(const SweepArgs &a, uint64_t *s_i
         const uint64_t groups = (a.total_items - a.item_base + a.group - 1u) / a.group;
         uint64_t item = ~0ull;
         while (s_tried < kQueues) {
-            const uint64_t i = atomicAdd(&a.queue[s_queue], 1ull);
-            const uint64_t g = queue_group(a, s_queue, i);
+            unsigned long long *const c = &a.queue[s_queue * kQueueStride];
+            uint64_t g = queue_group(a, s_queue, __hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+            if (g < groups) g = queue_group(a, s_queue, atomicAdd(c, 1ull));
             if (g < groups) {
                 item = a.item_base + g * a.group;
                 break;
@@ -453,14 +460,14 @@ __device__ __forceinline__ uint64_t fetch_item(const SweepArgs &a, uint64_t *s_i
 // x' = x, or 7 - x for odd r), group i % L of it; a bijection on the whole
 // rounds of 8 L groups (the rest in blockIdx order).  An object's tables are
 // then fetched into one L2, and the XCDs get equal shares of the work.
-__device__ __forceinline__ uint64_t grid_group(const SweepArgs &a) {
-    const uint64_t w = blockIdx.x, L = a.xcd_run;
+__device__ __forceinline__ uint64_t xcd_group(uint64_t w, uint64_t groups, uint64_t L) {
     if (L == 0) return w;
-    const uint64_t round = 8u * L, full = ((uint64_t)gridDim.x / round) * round;
+    const uint64_t round = 8u * L, full = (groups / round) * round;
     if (w >= full) return w;
     const uint64_t i = w >> 3, r = i / L, x = (r & 1u) ? 7u - (w & 7u) : (w & 7u);
     return r * round + x * L + i % L;
 }
+__device__ __forceinline__ uint64_t grid_group(const SweepArgs &a) { return xcd_group(blockIdx.x, gridDim.x, a.xcd_run); }
 __device__ __forceinline__ uint64_t first_item(const SweepArgs &a, uint64_t *s_item) {
     return a.queue ? fetch_item(a, s_item, true) : a.item_base + grid_group(a) * a.group;
 }

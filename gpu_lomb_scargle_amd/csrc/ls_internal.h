@@ -55,6 +55,7 @@ struct Workspace {
     size_t obj_ip = 0;      // InterpObj[K]
     size_t ip_tab = 0;
     size_t cand = 0;        // uint64[K * ceil(chunks / 64)]
+    size_t direct = 0;      // uint32[1 + K]  objects in direct mode: number, list
     uint32_t chunks = 0;
     uint32_t slices = 1;    // observation slices per (object, chunk)
     Tile tile{};

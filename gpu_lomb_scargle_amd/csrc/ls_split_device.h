@@ -205,6 +205,119 @@ __device__ __forceinline__ void split64x2(double x0, double x1, half2_t &h, half
     l = __builtin_convertvector((float2_t){(float)(x0 - (double)h.x), (float)(x1 - (double)h.y)}, half2_t);
 }
 
+// The direct tile's tables of object k: wavefront y0 of gy writes the
+// column-factor fragments of 16-observation blocks y0, y0 + gy, ... of the object, each factor
+// as head and tail of the real and imaginary parts (a product that needs -f_i
+// takes the row factor's negated fragment instead):
+//   standard:    y v (4 fragments), w (4)
+//   generalized: (w/W) v (4), (w/W) y_c v (4), (w/W) w (4)
+// with v = e^{2 pi i b df t} (b < 32 the column) and w = v^2, from the
+// caller's FP64 (or FP32) t, y, dy in FP64 arithmetic: FP64 phase and
+// sin/cos, w/W = 1 / (dy^2 W) the normalised weight, y_c = y - ybar; y (or
+// (w/W) y_c) scaled per object by a power of two ys, and w/W by a power of
+// two ws, to a maximum in [0.5, 1) (from the statistics), then all by 2^10
+// (FP16 range; the scales are undone exactly in the power); and the
+// row-step fragments (e^{2 pi i 32 a df t}, row a = l % 32).  Observations
+// past the object's end have zero factors.
+template <bool GEN, typename IN>
+__device__ __forceinline__ void direct_tables(const SweepArgs &a, uint32_t k, uint32_t y0, uint32_t gy) {
+    constexpr int NF = GEN ? kColfacFragsGen : kColfacFragsStd;
+    const uint32_t l = threadIdx.x;
+    const uint64_t beg = a.offsets[k], end = a.offsets[k + 1];
+    const uint32_t n = (uint32_t)(end - beg);
+    const IN *y = static_cast<const IN *>(a.y);
+    const IN *dy = static_cast<const IN *>(a.dy);
+    double iW = 1.0, ybar = 0.0;
+    if constexpr (GEN) {
+        iW = 1.0 / a.obj_gen[kGen * k + 4];
+        ybar = a.obj_gen[kGen * k + 3];
+    }
+    auto weight = [&](uint64_t i) -> double {  // w / W (1 for the standard variant)
+        if constexpr (GEN) {
+            const double d = (double)dy[i];
+            return iW / (d * d);
+        } else {
+            return 1.0;
+        }
+    };
+    auto yfac = [&](uint64_t i) -> double {  // y, or (w / W) (y - ybar)
+        if constexpr (GEN) return weight(i) * ((double)y[i] - ybar);
+        else return (double)y[i];
+    };
+    const double ys = (double)a.obj_ys[2 * k], ws = (double)a.obj_ys[2 * k + 1];
+    const double sy = ys * (double)kFacScale, sw = ws * (double)kFacScale;  // exact: powers of two
+    const double fb = (double)(l & 31u) * a.df_rev;
+    const double fr = (double)(32u * (l & 31u)) * a.df_rev;  // row step of row l % 32
+    uint4 *dst = a.colfac + colfac_slot(beg, k) * (uint64_t)(NF * 64) + l;
+    uint4 *rdst = a.rowfac + colfac_slot(beg, k) * (uint64_t)(kRowfacFrags * 64) + l;
+    for (uint32_t q = y0; q * 16u < n; q += gy) {
+        // row-step phasors R = e^{2 pi i 32 (l % 32) df t} of observations
+        // 8 (l / 32) .. + 7, in FP64 rounded to FP32 (zero past the end)
+#pragma unroll
+        for (int p = 0; p < kRowfacFrags; ++p) {
+            float r4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const uint32_t j = q * 16u + 8u * (l >> 5) + (uint32_t)(2 * p + e);
+                if (j < n) {
+                    double c, sn;
+                    phasor64(fr, a.rec_t[beg + j], c, sn);
+                    r4[2 * e] = (float)c;
+                    r4[2 * e + 1] = (float)sn;
+                }
+            }
+            uint4 u;
+            __builtin_memcpy(&u, r4, sizeof(u));
+            rdst[(uint64_t)(q * kRowfacFrags + p) * 64] = u;
+        }
+        half8_t f[NF];
+#pragma unroll
+        for (int v = 0; v < 8; v += 2) {
+            double x[NF / 2][2];  // the factors of observations v, v + 1: real, imaginary per sum
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const uint32_t j = q * 16u + 8u * (l >> 5) + (uint32_t)(v + e);
+                double cb = 0.0, sb = 0.0, yv = 0.0, wv = 0.0;
+                if (j < n) {
+                    phasor64(fb, a.rec_t[beg + j], cb, sb);
+                    yv = yfac(beg + j) * sy;
+                    wv = weight(beg + j) * sw;
+                }
+                const double wr = cb * cb - sb * sb, wi = 2.0 * cb * sb;  // v^2
+                if constexpr (GEN) {
+                    x[0][e] = wv * cb;
+                    x[1][e] = wv * sb;
+                    x[2][e] = yv * cb;
+                    x[3][e] = yv * sb;
+                    x[4][e] = wv * wr;
+                    x[5][e] = wv * wi;
+                } else {
+                    x[0][e] = yv * cb;
+                    x[1][e] = yv * sb;
+                    x[2][e] = wv * wr;
+                    x[3][e] = wv * wi;
+                }
+            }
+#pragma unroll
+            for (int p = 0; p < NF / 4; ++p) {  // each complex factor: r (h, l), i (h, l)
+                half2_t h, t;
+                split64x2(x[2 * p][0], x[2 * p][1], h, t);
+                f[4 * p + 0][v] = h.x; f[4 * p + 0][v + 1] = h.y;
+                f[4 * p + 1][v] = t.x; f[4 * p + 1][v + 1] = t.y;
+                split64x2(x[2 * p + 1][0], x[2 * p + 1][1], h, t);
+                f[4 * p + 2][v] = h.x; f[4 * p + 2][v + 1] = h.y;
+                f[4 * p + 3][v] = t.x; f[4 * p + 3][v + 1] = t.y;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NF; ++i) {
+            uint4 u;
+            __builtin_memcpy(&u, &f[i], sizeof(u));
+            dst[(uint64_t)(q * NF + i) * 64] = u;
+        }
+    }
+}
+
 __device__ __forceinline__ half8_t neg8(half8_t x) {
     uint4 u;
     __builtin_memcpy(&u, &x, sizeof(u));
@@ -233,33 +346,48 @@ __device__ __forceinline__ void load_cols(const uint4 *cf, half8_t (&col)[NF]) {
 }
 
 // Work items of the direct matrix-core tiles: the sweep's; or, beside the
-// coarse-grid sweep, with a.cand_split workgroups per object, the chunks r,
-// r + cand_split, ... of an object in direct mode (a workgroup per item would
-// mostly find objects that are not its business: 0.25 ms for 10^6 items), and
-// every cand_split-th of the marked chunks of an object in coarse mode.
-__device__ __forceinline__ uint64_t direct_pick(const SweepArgs &a, uint32_t pos, uint32_t from, uint32_t skip) {
-    const uint32_t obj = a.order ? a.order[pos] : pos;
-    if (a.obj_ip[obj].mode == 0u) return from + skip < a.chunks ? (uint64_t)pos * a.chunks + from + skip : ~0ull;
-    if (!a.cand) return ~0ull;
+// coarse-grid sweep, two kinds of workgroups.  The first a.marked_groups take
+// the marked chunks of the objects in coarse mode, workgroup r of an object
+// every cand_split-th, an object's workgroups on one XCD (its tables are then
+// fetched once and found in the L2: 0.46 -> 0.15 ms for 1000 generalized
+// objects).  The others take the groups of the objects in direct mode, in the
+// grid schedule's order; the launch has a workgroup for every group that there
+// could be, and those past the list's end, which only the device knows, leave
+// at once.  (In their place, where all objects are direct, 4000 x 100,000 bins,
+// 4.53 ms with the plain grid: workgroups that stay on the chip and stride over
+// the groups 5.9, the persistent queues 4.9, groups of eight items 4.8.)
+__device__ __forceinline__ uint64_t cand_item(const SweepArgs &a, uint32_t obj, uint32_t from, uint32_t skip) {
     const uint64_t *bits = a.cand + (uint64_t)obj * a.cand_words;
     for (uint32_t w = from >> 6; w < a.cand_words; ++w) {
         uint64_t b = bits[w];
         if (w == from >> 6) b &= ~0ull << (from & 63u);
         for (; b; b &= b - 1u, --skip)
-            if (skip == 0u) return (uint64_t)pos * a.chunks + 64u * w + (uint32_t)__builtin_ctzll(b);
+            if (skip == 0u) return (uint64_t)obj * a.chunks + 64u * w + (uint32_t)__builtin_ctzll(b);
     }
     return ~0ull;
 }
-__device__ __forceinline__ uint64_t direct_first(const SweepArgs &a, uint64_t *s_item) {
+__device__ __forceinline__ uint64_t direct_first(SweepArgs &a, uint64_t *s_item) {
     if (!a.obj_ip) return first_item(a, s_item);
-    const uint64_t g = grid_group(a);
-    const uint32_t pos = (uint32_t)(g / a.cand_split);
-    return direct_pick(a, pos, 0u, (uint32_t)(g - (uint64_t)pos * a.cand_split));
+    if (blockIdx.x >= a.marked_groups) {
+        a.cand = nullptr;
+        a.order = a.direct_list;
+        a.total_items = (uint64_t)*a.direct_count * a.chunks;
+        const uint64_t groups = (a.total_items + a.group - 1u) / a.group, w = a.item_base + blockIdx.x - a.marked_groups;
+        if (w >= groups) return ~0ull;
+        a.item_base = 0;
+        return xcd_group(w, groups, a.xcd_run) * a.group;
+    }
+    const uint32_t g = (uint32_t)xcd_group(blockIdx.x, a.marked_groups, a.cand_split);
+    const uint32_t pos = g / a.cand_split, r = g - pos * a.cand_split;
+    if (pos >= a.K) return ~0ull;
+    const uint32_t obj = a.order ? a.order[pos] : pos;
+    a.order = nullptr;  // the items name the object itself
+    return a.obj_ip[obj].mode ? cand_item(a, obj, 0u, r) : ~0ull;
 }
 __device__ __forceinline__ uint64_t direct_next(const SweepArgs &a, uint64_t *s_item, uint64_t item) {
-    if (!a.obj_ip) return next_item(a, s_item, item);
-    const uint32_t pos = (uint32_t)(item / a.chunks);
-    return direct_pick(a, pos, (uint32_t)(item - (uint64_t)pos * a.chunks) + 1u, a.cand_split - 1u);
+    if (!a.cand) return next_item(a, s_item, item);
+    const uint32_t obj = (uint32_t)(item / a.chunks);
+    return cand_item(a, obj, (uint32_t)(item - (uint64_t)obj * a.chunks) + 1u, a.cand_split - 1u);
 }
 
 #define LS_MFMA(ACC, A, B) ACC = __builtin_amdgcn_mfma_f32_32x32x16_f16(A, B, ACC, 0, 0, 0)

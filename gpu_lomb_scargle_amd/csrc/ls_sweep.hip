@@ -400,7 +400,7 @@ __global__ void k_records_split(RecArgs a) {
 }
 
 __global__ void k_zero_counters(unsigned long long *c, uint32_t n) {
-    if (threadIdx.x < n) c[threadIdx.x] = 0ull;
+    if (threadIdx.x < n) c[threadIdx.x * kQueueStride] = 0ull;
 }
 
 // ---------------------------------------------------------------------------
@@ -626,8 +626,9 @@ int plan_workspace(const lsamd_sweep_args *a, Workspace *w) {
         w->obj_ip = take(sizeof(InterpObj) * K);
         w->ip_tab = take((size_t)16 * 64 * 6 * kIpModes);
         w->cand = take((size_t)8 * K * ((w->chunks + 63) / 64));
+        w->direct = take((size_t)4 * (K + 1));
     }
-    w->queue = take(8 * kQueues);
+    w->queue = take(8 * kQueues * kQueueStride);
     w->bytes = off + 256;
     return LSAMD_OK;
 }
@@ -769,7 +770,7 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
                  mfma ? reinterpret_cast<double *>(ws + w.rec_t) : nullptr,
                  mfma ? reinterpret_cast<double2 *>(ws + w.rec_r) : nullptr, obj_ip, dw * kInv2Pi,
                  w.screen ? kIpSigmaScreen : gen ? kIpSigmaGen : kIpSigma,
-                 w.screen ? kIpLeastObsScreen : kIpLeastObs, w.screen ? 1 : 2, w.screen ? 1 : 0};
+                 w.screen ? (gen ? kIpLeastObsScreenGen : kIpLeastObsScreen) : kIpLeastObs, w.screen ? 1 : 2, w.screen ? 1 : 0};
     if (split) {
         const bool wide = w.slices > 1;  // one long object alone
         void (*fn)(StatsArgs) = wide ? (f64 ? k_obj_stats_split<double, 512> : k_obj_stats_split<float, 512>)
@@ -853,6 +854,8 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
 
     if (w.interp) {
         sw.obj_ip = obj_ip;
+        sw.direct_count = reinterpret_cast<uint32_t *>(ws + w.direct);
+        sw.direct_list = sw.direct_count + 1;
         sw.ip_tab = reinterpret_cast<uint4 *>(ws + w.ip_tab);
         const uint32_t least = w.screen ? kIpLeastBinsScreen : kIpLeastBins;
         sw.ip_items = (a->num_freqs + least - 1) / least;
@@ -911,7 +914,7 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
         const uint32_t per_obj = (si.ip_items + si.group - 1) / si.group;
         si.xcd_run = per_obj;
         void *iargs[] = {&si};
-        LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(ip.fac), dim3(K + 3 * kIpModes, gy), dim3(64), iargs, 0,
+        LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(ip.fac), dim3(K + 1 + 3 * kIpModes, gy), dim3(64), iargs, 0,
                                st));
         const uint64_t ip_groups = (uint64_t)K * per_obj, most = 0xFFFFFFFFull / (uint64_t)ip.threads - 1;
         for (uint64_t g = 0; g < ip_groups; g += most) {
@@ -923,17 +926,24 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
         SweepArgs sd = sw;
         sd.cand = a->top_k > 0 ? reinterpret_cast<uint64_t *>(ws + w.cand) : nullptr;
         sd.queue = nullptr;
-        // workgroups per object: 8 rounds of the chip over all objects (most
-        // find nothing to do), and at most 32 chunks of an object in direct mode
-        // each (8000 objects x 196 chunks, 10% of them direct: 2.2 ms with 98
-        // chunks each, 1.7 with 28)
-        sd.cand_split = (uint32_t)std::min<uint64_t>(w.chunks, std::max<uint64_t>(16384 / K, (w.chunks + 31) / 32));
-        sd.xcd_run = sd.cand_split;
+        sd.item_base = 0;
+        // workgroups per object for its marked chunks (one to four of them
+        // mostly), then one for every group of items that could be an object's
+        // in direct mode (launches of under 2^32 threads)
+        sd.cand_split = (uint32_t)std::min<uint64_t>(64, std::max<uint64_t>(2, 4096 / K));
+        sd.marked_groups = sd.cand ? (K * sd.cand_split + 7u) & ~7u : 0u;
         void *dargs[] = {&sd};
-        LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->prep), dim3(K, gy + (sd.cand ? 1u : 0u)), dim3(64),
-                               dargs, 0, st));
-        LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->fn), dim3(K * sd.cand_split), dim3(T), dargs, 0,
-                               st));
+        if (sd.cand)
+            LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->prep), dim3(K, gy + 1u), dim3(64), dargs, 0, st));
+        const uint64_t launch_most = 0xFFFFFFFFull / (uint64_t)T - 1;
+        for (uint64_t g = 0; g < groups;) {
+            const uint64_t cnt = std::min<uint64_t>(launch_most - sd.marked_groups, groups - g);
+            sd.item_base = g;
+            LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->fn), dim3((uint32_t)(sd.marked_groups + cnt)),
+                                   dim3(T), dargs, 0, st));
+            g += cnt;
+            sd.marked_groups = 0;
+        }
     } else if (te->prep) {  // per-object set-up of the tile, inside the timed sweep
         void *kargs[] = {&sw};
         LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->prep), dim3(K, gy), dim3(64), kargs, 0, st));

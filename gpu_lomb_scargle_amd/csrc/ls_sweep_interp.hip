@@ -110,23 +110,49 @@ __device__ __forceinline__ void ip_phasor(double f, double t, double &c, double 
     }
 }
 
-// Workgroups past the last object write the interpolation operands (blockIdx.x
-// = K + 3 (mode - 1) + which third).  Wavefronts (object, y) write the tables of the object's 16-observation
+// The objects in direct mode, in processing order, and their number (one
+// wavefront; 512 objects' modes in flight).
+__device__ void list_direct(const SweepArgs &a) {
+    const uint32_t lane = threadIdx.x;
+    uint32_t count = 0;
+    for (uint32_t base = 0; base < a.K; base += 512u) {
+        uint32_t obj[8], mode[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const uint32_t pos = base + 64u * (uint32_t)q + lane;
+            obj[q] = pos < a.K ? (a.order ? a.order[pos] : pos) : 0u;
+        }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) mode[q] = base + 64u * (uint32_t)q + lane < a.K ? a.obj_ip[obj[q]].mode : 1u;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const uint64_t direct = __ballot(mode[q] == 0u);
+            if (mode[q] == 0u) a.direct_list[count + (uint32_t)__popcll(direct & ((1ull << lane) - 1ull))] = obj[q];
+            count += (uint32_t)__popcll(direct);
+        }
+    }
+    if (lane == 0) *a.direct_count = count;
+}
+
+// Workgroups past the last object list the objects in direct mode (blockIdx.x =
+// K) and write the interpolation operands (K + 1 + 3 (mode - 1) + which third).  Wavefronts (object, y) write the tables of the object's 16-observation
 // blocks y, y + gridDim.y, ..., as k_colfac does for the direct tile, into the
-// same slots: column factors e^{2 pi i (b + 1/2) h df t'} a / Phi (b < 32) of the
+// same slots (objects in direct mode: the direct tile's themselves): column factors e^{2 pi i (b + 1/2) h df t'} a / Phi (b < 32) of the
 // two weights a = y (generalized: (w/W) (y - ybar)) and a = 1 (w/W), four head
 // and tail fragments each, and the row steps e^{2 pi i 64 a h df t'} (a < 32),
 // with t' = t - tc and 1/Phi from the records.
 template <bool GEN, typename IN, bool SCREEN>
 __global__ __launch_bounds__(64) void k_interp_fac(SweepArgs a) {
     constexpr int FR = ip_frags(SCREEN), NC = SCREEN ? 1 : 2;  // fragments; heads alone or with tails
-    const uint32_t k = blockIdx.x, l = threadIdx.x;
-    if (k >= a.K) {
-        if (blockIdx.y == 0) interp_table<SCREEN>(a.ip_tab, (int)(k - a.K) / 3 + 1, (int)(k - a.K) % 3);
-        return;
+    const uint32_t pos = blockIdx.x, l = threadIdx.x;
+    if (pos >= a.K) {
+        if (blockIdx.y != 0) return;
+        if (pos == a.K) return list_direct(a);
+        return interp_table<SCREEN>(a.ip_tab, (int)(pos - a.K - 1u) / 3 + 1, (int)(pos - a.K - 1u) % 3);
     }
+    const uint32_t k = a.order ? a.order[pos] : pos;
     const int mode = (int)a.obj_ip[k].mode;
-    if (mode == 0) return;
+    if (mode == 0) return direct_tables<GEN, IN>(a, k, blockIdx.y, gridDim.y);
     const uint64_t beg = a.offsets[k], end = a.offsets[k + 1];
     const uint32_t n = (uint32_t)(end - beg);
     const IN *y = static_cast<const IN *>(a.y);
@@ -570,6 +596,10 @@ __global__ __launch_bounds__(256, SCREEN ? 3 : 2) void k_sweep_interp(SweepArgs 
             }
         }
         uint64_t lanes = __ballot(flags != 0u);
+        // The screen leaves a tile with many of them to the direct sums, which
+        // compute them again anyway: all its chunks are marked by the sign.
+        const bool unread = SCREEN && __popcll(lanes) > kIpScreenIll;
+        if (unread) lanes = 0u;
         while (lanes) {
             const uint32_t src = (uint32_t)__builtin_ctzll(lanes);
             const uint32_t f = (uint32_t)__shfl((int)flags, (int)src, 64), v = (uint32_t)__builtin_ctz(f);
@@ -593,7 +623,8 @@ __global__ __launch_bounds__(256, SCREEN ? 3 : 2) void k_sweep_interp(SweepArgs 
                 if (l == (uint32_t)__builtin_ctzll(__ballot(best == t1))) best = 0.0f;
                 t2 = wave_fmax(best);
             }
-            if (l < 3) tmax[3u * tile + l] = l == 0 ? t0 : l == 1 ? t1 : t2;
+            const float tv = l == 0 ? t0 : l == 1 ? t1 : t2;
+            if (l < 3) tmax[3u * tile + l] = unread ? -tv : tv;
         }
     }
     };

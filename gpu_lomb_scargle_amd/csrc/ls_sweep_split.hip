@@ -662,7 +662,7 @@ __device__ void mark_chunks(const SweepArgs &a, uint32_t obj) {
     float t0 = 0.0f, t1 = 0.0f, t2 = 0.0f;
 #pragma unroll 8
     for (uint32_t i = lane; i < 3u * ntiles; i += 64u) {  // into the lane's descending three
-        const float p = tmax[i], a0 = fminf(t0, p), a1 = fminf(t1, a0);
+        const float p = fabsf(tmax[i]), a0 = fminf(t0, p), a1 = fminf(t1, a0);
         t0 = fmaxf(t0, p);
         t1 = fmaxf(t1, a0);
         t2 = fmaxf(t2, a1);
@@ -689,7 +689,7 @@ __device__ void mark_chunks(const SweepArgs &a, uint32_t obj) {
             const uint32_t end = tile_of_bin(last);
             for (uint32_t t = tile_of_bin(1024u * c); t <= end; ++t) {
                 const float p = tmax[3u * t];
-                yes = yes || (p > 0.0f && p >= least);
+                yes = yes || (p > 0.0f && p >= least) || __builtin_signbitf(p);  // sign: bins left to the direct sums
             }
         }
         const uint64_t word = __ballot(yes);
@@ -697,122 +697,15 @@ __device__ void mark_chunks(const SweepArgs &a, uint32_t obj) {
     }
 }
 
-// Wavefronts (object, y) with y < gridDim.y write the column-factor fragments
-// of 16-observation blocks y, y + gridDim.y, ... of the object, each factor
-// as head and tail of the real and imaginary parts (a product that needs -f_i
-// takes the row factor's negated fragment instead):
-//   standard:    y v (4 fragments), w (4)
-//   generalized: (w/W) v (4), (w/W) y_c v (4), (w/W) w (4)
-// with v = e^{2 pi i b df t} (b < 32 the column) and w = v^2, from the
-// caller's FP64 (or FP32) t, y, dy in FP64 arithmetic: FP64 phase and
-// sin/cos, w/W = 1 / (dy^2 W) the normalised weight, y_c = y - ybar; y (or
-// (w/W) y_c) scaled per object by a power of two ys, and w/W by a power of
-// two ws, to a maximum in [0.5, 1) (from the statistics), then all by 2^10
-// (FP16 range; the scales are undone exactly in the power); and the
-// row-step fragments (e^{2 pi i 32 a df t}, row a = l % 32).  Observations
-// past the object's end have zero factors.
+// Tables of the direct tile, wavefronts (object, y).  Beside the coarse-grid
+// sweep: the marks of its objects (the last y) and their tables, which replace
+// the coarse ones; those of the objects in direct mode are there already.
 template <bool GEN, typename IN>
 __global__ __launch_bounds__(64) void k_colfac(SweepArgs a) {
-    constexpr int NF = GEN ? kColfacFragsGen : kColfacFragsStd;
-    const uint32_t k = blockIdx.x, l = threadIdx.x;
-    // beside the coarse-grid sweep: the marks of its objects (the last y), and
-    // their tables only if marked chunks are swept
     const uint32_t gy = gridDim.y - (a.cand ? 1u : 0u);
-    if (blockIdx.y == gy) return mark_chunks(a, k);
-    if (a.obj_ip && a.obj_ip[k].mode != 0u && !a.cand) return;
-    const uint64_t beg = a.offsets[k], end = a.offsets[k + 1];
-    const uint32_t n = (uint32_t)(end - beg);
-    const IN *y = static_cast<const IN *>(a.y);
-    const IN *dy = static_cast<const IN *>(a.dy);
-    double iW = 1.0, ybar = 0.0;
-    if constexpr (GEN) {
-        iW = 1.0 / a.obj_gen[kGen * k + 4];
-        ybar = a.obj_gen[kGen * k + 3];
-    }
-    auto weight = [&](uint64_t i) -> double {  // w / W (1 for the standard variant)
-        if constexpr (GEN) {
-            const double d = (double)dy[i];
-            return iW / (d * d);
-        } else {
-            return 1.0;
-        }
-    };
-    auto yfac = [&](uint64_t i) -> double {  // y, or (w / W) (y - ybar)
-        if constexpr (GEN) return weight(i) * ((double)y[i] - ybar);
-        else return (double)y[i];
-    };
-    const double ys = (double)a.obj_ys[2 * k], ws = (double)a.obj_ys[2 * k + 1];
-    const double sy = ys * (double)kFacScale, sw = ws * (double)kFacScale;  // exact: powers of two
-    const double fb = (double)(l & 31u) * a.df_rev;
-    const double fr = (double)(32u * (l & 31u)) * a.df_rev;  // row step of row l % 32
-    uint4 *dst = a.colfac + colfac_slot(beg, k) * (uint64_t)(NF * 64) + l;
-    uint4 *rdst = a.rowfac + colfac_slot(beg, k) * (uint64_t)(kRowfacFrags * 64) + l;
-    for (uint32_t q = blockIdx.y; q * 16u < n; q += gy) {
-        // row-step phasors R = e^{2 pi i 32 (l % 32) df t} of observations
-        // 8 (l / 32) .. + 7, in FP64 rounded to FP32 (zero past the end)
-#pragma unroll
-        for (int p = 0; p < kRowfacFrags; ++p) {
-            float r4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const uint32_t j = q * 16u + 8u * (l >> 5) + (uint32_t)(2 * p + e);
-                if (j < n) {
-                    double c, sn;
-                    phasor64(fr, a.rec_t[beg + j], c, sn);
-                    r4[2 * e] = (float)c;
-                    r4[2 * e + 1] = (float)sn;
-                }
-            }
-            uint4 u;
-            __builtin_memcpy(&u, r4, sizeof(u));
-            rdst[(uint64_t)(q * kRowfacFrags + p) * 64] = u;
-        }
-        half8_t f[NF];
-#pragma unroll
-        for (int v = 0; v < 8; v += 2) {
-            double x[NF / 2][2];  // the factors of observations v, v + 1: real, imaginary per sum
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const uint32_t j = q * 16u + 8u * (l >> 5) + (uint32_t)(v + e);
-                double cb = 0.0, sb = 0.0, yv = 0.0, wv = 0.0;
-                if (j < n) {
-                    phasor64(fb, a.rec_t[beg + j], cb, sb);
-                    yv = yfac(beg + j) * sy;
-                    wv = weight(beg + j) * sw;
-                }
-                const double wr = cb * cb - sb * sb, wi = 2.0 * cb * sb;  // v^2
-                if constexpr (GEN) {
-                    x[0][e] = wv * cb;
-                    x[1][e] = wv * sb;
-                    x[2][e] = yv * cb;
-                    x[3][e] = yv * sb;
-                    x[4][e] = wv * wr;
-                    x[5][e] = wv * wi;
-                } else {
-                    x[0][e] = yv * cb;
-                    x[1][e] = yv * sb;
-                    x[2][e] = wv * wr;
-                    x[3][e] = wv * wi;
-                }
-            }
-#pragma unroll
-            for (int p = 0; p < NF / 4; ++p) {  // each complex factor: r (h, l), i (h, l)
-                half2_t h, t;
-                split64x2(x[2 * p][0], x[2 * p][1], h, t);
-                f[4 * p + 0][v] = h.x; f[4 * p + 0][v + 1] = h.y;
-                f[4 * p + 1][v] = t.x; f[4 * p + 1][v + 1] = t.y;
-                split64x2(x[2 * p + 1][0], x[2 * p + 1][1], h, t);
-                f[4 * p + 2][v] = h.x; f[4 * p + 2][v + 1] = h.y;
-                f[4 * p + 3][v] = t.x; f[4 * p + 3][v + 1] = t.y;
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < NF; ++i) {
-            uint4 u;
-            __builtin_memcpy(&u, &f[i], sizeof(u));
-            dst[(uint64_t)(q * NF + i) * 64] = u;
-        }
-    }
+    if (blockIdx.y == gy) return mark_chunks(a, blockIdx.x);
+    if (a.obj_ip && a.obj_ip[blockIdx.x].mode == 0u) return;
+    direct_tables<GEN, IN>(a, blockIdx.x, blockIdx.y, gy);
 }
 
 // Row factors of a 16-observation block for lane (row rc, half kh): u = u0 R
