@@ -99,6 +99,15 @@ constexpr int kColfacFragsStd = 8, kColfacFragsGen = 12;
 // Matrix-core tile: row-step phasors e^{2 pi i 32 a df t} per 16 observations
 // (lane a + 32 h: observations 8 h .. 8 h + 7 as 4 x two complex FP32).
 constexpr int kRowfacFrags = 4;
+// Groups of T threads that share the M bins per thread of a tile when its
+// observation slices are added up: the largest divisor of M that fits a
+// workgroup of 1024 threads.
+constexpr int combine_groups(int T, int M) {
+    int g = 1;
+    for (int d = 2; d <= M && d * T <= 1024; ++d)
+        if (M % d == 0) g = d;
+    return g;
+}
 constexpr int kPeaks = 3;      // peaks tracked per object (top-1 and top-3)
 // doubles per object of split-generalized constants: [0..2] Wf, Yb, YY over
 // the FP32-rounded weights the VALU split sweeps apply; [3] ybar, [4] W (sum

@@ -970,13 +970,12 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
         if (!te->combine) return set_error(LSAMD_ERR_INVALID, "lsamd_sweep: no slice combiner");
         void *kargs[] = {&sw};
         LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->combine),
-                               dim3((uint32_t)((uint64_t)K * w.chunks)), dim3(T), kargs, 0, st));
+                               dim3((uint32_t)((uint64_t)K * w.chunks)), dim3(T * combine_groups(T, M)), kargs, 0, st));
     }
     if (timing) {
         LS_HIP(hipEventRecord(tm.ev[1], st));
         tm.pending = true;
     }
-    (void)M;
 
     // 4. peaks
     if (a->top_k > 0) {
