@@ -404,7 +404,7 @@ int lsamd_batch_host(int variant, int dtype, int form, int normalize, int precen
             a.peak_power = static_cast<char *>(c.ppow.p) + (size_t)s0 * tk * rsz;
             a.peak_period = static_cast<char *>(c.pper.p) + (size_t)s0 * tk * rsz;
         }
-        const size_t wsb = lsamd_sweep_workspace_size(&a);
+        const size_t wsb = sweep_part_bytes(&a, K);
         int r = LSAMD_OK;
         if (c.ws.cap < wsb) {
             // growing the workspace frees it: wait for the sweeps using it
@@ -412,7 +412,7 @@ int lsamd_batch_host(int variant, int dtype, int form, int normalize, int precen
             r = ensure(c.ws, wsb);
             if (r) return r;
         }
-        r = lsamd_sweep(&a, c.ws.p, c.ws.cap, c.stream);
+        r = sweep_part(&a, K, c.ws.p, c.ws.cap, c.stream);
         if (r) return r;
         HIP_OK(hipEventRecord(c.slice[i & 1], c.stream));
         return LSAMD_OK;
