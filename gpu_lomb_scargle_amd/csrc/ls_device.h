@@ -50,6 +50,7 @@ struct SweepArgs {
     // matrix-core tile: per-object column- and row-factor fragments, y scale
     uint4 *colfac;
     uint4 *rowfac;
+    uint32_t *slot_obj;  // the object of each 16-observation slot
     float *obj_ys;  // per object: y scale, weight scale
     // coarse-grid sweep (null: every object direct): the objects' modes, the
     // interpolation operands, workgroups per object, and the chunks to sweep

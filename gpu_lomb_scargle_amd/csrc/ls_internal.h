@@ -48,6 +48,7 @@ struct Workspace {
     size_t obj_ys = 0;      // float[2K]  matrix-core tile: power-of-two y and weight scales
     size_t colfac = 0;      // matrix-core tile: column-factor fragments, 8 (12 generalized) KiB per 16 observations
     size_t rowfac = 0;      // matrix-core tile: row-step phasors, 4 KiB per 16 observations
+    size_t slot_obj = 0;    // matrix-core tile: uint32 object of each such slot
     // coarse-grid sweep (interp): modes per object, interpolation operands,
     // marked chunks
     bool interp = false;

@@ -198,6 +198,23 @@ __device__ __forceinline__ void split16x2(float x0, float x1, half2_t &h, half2_
 // next object's floor((beg + N)/16) + k + 1.
 __device__ __forceinline__ uint64_t colfac_slot(uint64_t beg, uint32_t obj) { return (beg >> 4) + obj; }
 
+// The tables are made by a wavefront per slot, whatever object it is of (the
+// statistics kernel writes that down), so that a long object's blocks are made
+// side by side: with wavefronts (object, one of the mean object's blocks) the
+// longest object's took its several blocks, ~5 us each, one after another: 499
+// objects of up to 1500 observations 50 -> 24 us, 8000 of up to 5000, coarse and
+// direct tables with the marks, 480 -> 345.  Slots count from the first
+// object's; false: past the last object, or between two.
+__device__ __forceinline__ bool slot_block(const SweepArgs &a, uint64_t slot, uint32_t &obj, uint32_t &block) {
+    const uint64_t first = a.offsets[0], last = a.offsets[a.K];
+    slot += colfac_slot(first, 0u);
+    if (slot >= colfac_slot(last, a.K)) return false;
+    obj = a.slot_obj[slot];
+    const uint64_t beg = a.offsets[obj];
+    block = (uint32_t)(slot - colfac_slot(beg, obj));
+    return (uint64_t)block * 16u < a.offsets[obj + 1] - beg;
+}
+
 // Heads and tails of two FP64 factors: h = fp16(fp32(x)), l = fp16(x - h),
 // the remainder x - h exact in FP64 (~22 bits of x in h + l).
 __device__ __forceinline__ void split64x2(double x0, double x1, half2_t &h, half2_t &l) {
@@ -220,7 +237,7 @@ __device__ __forceinline__ void split64x2(double x0, double x1, half2_t &h, half
 // row-step fragments (e^{2 pi i 32 a df t}, row a = l % 32).  Observations
 // past the object's end have zero factors.
 template <bool GEN, typename IN>
-__device__ __forceinline__ void direct_tables(const SweepArgs &a, uint32_t k, uint32_t y0, uint32_t gy) {
+__device__ __forceinline__ void direct_table(const SweepArgs &a, uint32_t k, uint32_t q) {
     constexpr int NF = GEN ? kColfacFragsGen : kColfacFragsStd;
     const uint32_t l = threadIdx.x;
     const uint64_t beg = a.offsets[k], end = a.offsets[k + 1];
@@ -250,71 +267,69 @@ __device__ __forceinline__ void direct_tables(const SweepArgs &a, uint32_t k, ui
     const double fr = (double)(32u * (l & 31u)) * a.df_rev;  // row step of row l % 32
     uint4 *dst = a.colfac + colfac_slot(beg, k) * (uint64_t)(NF * 64) + l;
     uint4 *rdst = a.rowfac + colfac_slot(beg, k) * (uint64_t)(kRowfacFrags * 64) + l;
-    for (uint32_t q = y0; q * 16u < n; q += gy) {
-        // row-step phasors R = e^{2 pi i 32 (l % 32) df t} of observations
-        // 8 (l / 32) .. + 7, in FP64 rounded to FP32 (zero past the end)
+    // row-step phasors R = e^{2 pi i 32 (l % 32) df t} of observations
+    // 8 (l / 32) .. + 7, in FP64 rounded to FP32 (zero past the end)
 #pragma unroll
-        for (int p = 0; p < kRowfacFrags; ++p) {
-            float r4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int p = 0; p < kRowfacFrags; ++p) {
+        float r4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const uint32_t j = q * 16u + 8u * (l >> 5) + (uint32_t)(2 * p + e);
-                if (j < n) {
-                    double c, sn;
-                    phasor64(fr, a.rec_t[beg + j], c, sn);
-                    r4[2 * e] = (float)c;
-                    r4[2 * e + 1] = (float)sn;
-                }
+        for (int e = 0; e < 2; ++e) {
+            const uint32_t j = q * 16u + 8u * (l >> 5) + (uint32_t)(2 * p + e);
+            if (j < n) {
+                double c, sn;
+                phasor64(fr, a.rec_t[beg + j], c, sn);
+                r4[2 * e] = (float)c;
+                r4[2 * e + 1] = (float)sn;
             }
-            uint4 u;
-            __builtin_memcpy(&u, r4, sizeof(u));
-            rdst[(uint64_t)(q * kRowfacFrags + p) * 64] = u;
         }
-        half8_t f[NF];
+        uint4 u;
+        __builtin_memcpy(&u, r4, sizeof(u));
+        rdst[(uint64_t)(q * kRowfacFrags + p) * 64] = u;
+    }
+    half8_t f[NF];
 #pragma unroll
-        for (int v = 0; v < 8; v += 2) {
-            double x[NF / 2][2];  // the factors of observations v, v + 1: real, imaginary per sum
+    for (int v = 0; v < 8; v += 2) {
+        double x[NF / 2][2];  // the factors of observations v, v + 1: real, imaginary per sum
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const uint32_t j = q * 16u + 8u * (l >> 5) + (uint32_t)(v + e);
-                double cb = 0.0, sb = 0.0, yv = 0.0, wv = 0.0;
-                if (j < n) {
-                    phasor64(fb, a.rec_t[beg + j], cb, sb);
-                    yv = yfac(beg + j) * sy;
-                    wv = weight(beg + j) * sw;
-                }
-                const double wr = cb * cb - sb * sb, wi = 2.0 * cb * sb;  // v^2
-                if constexpr (GEN) {
-                    x[0][e] = wv * cb;
-                    x[1][e] = wv * sb;
-                    x[2][e] = yv * cb;
-                    x[3][e] = yv * sb;
-                    x[4][e] = wv * wr;
-                    x[5][e] = wv * wi;
-                } else {
-                    x[0][e] = yv * cb;
-                    x[1][e] = yv * sb;
-                    x[2][e] = wv * wr;
-                    x[3][e] = wv * wi;
-                }
+        for (int e = 0; e < 2; ++e) {
+            const uint32_t j = q * 16u + 8u * (l >> 5) + (uint32_t)(v + e);
+            double cb = 0.0, sb = 0.0, yv = 0.0, wv = 0.0;
+            if (j < n) {
+                phasor64(fb, a.rec_t[beg + j], cb, sb);
+                yv = yfac(beg + j) * sy;
+                wv = weight(beg + j) * sw;
             }
-#pragma unroll
-            for (int p = 0; p < NF / 4; ++p) {  // each complex factor: r (h, l), i (h, l)
-                half2_t h, t;
-                split64x2(x[2 * p][0], x[2 * p][1], h, t);
-                f[4 * p + 0][v] = h.x; f[4 * p + 0][v + 1] = h.y;
-                f[4 * p + 1][v] = t.x; f[4 * p + 1][v + 1] = t.y;
-                split64x2(x[2 * p + 1][0], x[2 * p + 1][1], h, t);
-                f[4 * p + 2][v] = h.x; f[4 * p + 2][v + 1] = h.y;
-                f[4 * p + 3][v] = t.x; f[4 * p + 3][v + 1] = t.y;
+            const double wr = cb * cb - sb * sb, wi = 2.0 * cb * sb;  // v^2
+            if constexpr (GEN) {
+                x[0][e] = wv * cb;
+                x[1][e] = wv * sb;
+                x[2][e] = yv * cb;
+                x[3][e] = yv * sb;
+                x[4][e] = wv * wr;
+                x[5][e] = wv * wi;
+            } else {
+                x[0][e] = yv * cb;
+                x[1][e] = yv * sb;
+                x[2][e] = wv * wr;
+                x[3][e] = wv * wi;
             }
         }
 #pragma unroll
-        for (int i = 0; i < NF; ++i) {
-            uint4 u;
-            __builtin_memcpy(&u, &f[i], sizeof(u));
-            dst[(uint64_t)(q * NF + i) * 64] = u;
+        for (int p = 0; p < NF / 4; ++p) {  // each complex factor: r (h, l), i (h, l)
+            half2_t h, t;
+            split64x2(x[2 * p][0], x[2 * p][1], h, t);
+            f[4 * p + 0][v] = h.x; f[4 * p + 0][v + 1] = h.y;
+            f[4 * p + 1][v] = t.x; f[4 * p + 1][v + 1] = t.y;
+            split64x2(x[2 * p + 1][0], x[2 * p + 1][1], h, t);
+            f[4 * p + 2][v] = h.x; f[4 * p + 2][v + 1] = h.y;
+            f[4 * p + 3][v] = t.x; f[4 * p + 3][v + 1] = t.y;
         }
+    }
+#pragma unroll
+    for (int i = 0; i < NF; ++i) {
+        uint4 u;
+        __builtin_memcpy(&u, &f[i], sizeof(u));
+        dst[(uint64_t)(q * NF + i) * 64] = u;
     }
 }
 

@@ -66,6 +66,7 @@ struct StatsArgs {
     const void *t;       // matrix-core tile (rec_t): its records, and the object's mode of the
     double *rec_t;       // coarse-grid sweep (obj_ip, else null)
     double2 *rec_r;
+    uint32_t *slot_obj;
     InterpObj *obj_ip;
     double df_rev;
     double sigma;        // least oversampling of the coarse grid, observations an object needs
@@ -282,6 +283,8 @@ __global__ __launch_bounds__(T) void k_obj_stats_split(StatsArgs a) {
         }
     }
     if (!a.rec_t) return;
+    // the object's 16-observation slots, up to the next object's first
+    for (uint64_t s = (b >> 4) + k + tid; s < (e >> 4) + k + 1; s += T) a.slot_obj[s] = k;
     {  // largest |y| (generalized: (w/W) |y - ybar|) and weight, as powers of two
         const double iW = 1.0 / W;
         double my = 0.0, mw = a.split_gen ? 0.0 : 1.0;
@@ -600,6 +603,7 @@ int plan_workspace(const lsamd_sweep_args *a, Workspace *w, uint32_t call_object
         const size_t frags = a->variant == LSAMD_GENERALIZED ? kColfacFragsGen : kColfacFragsStd;
         w->colfac = take((size_t)16 * 64 * frags * (n / 16 + K + 1));
         w->rowfac = take((size_t)16 * 64 * kRowfacFrags * (n / 16 + K + 1));
+        w->slot_obj = take((size_t)4 * (n / 16 + K + 1));
     }
     const size_t parts = (size_t)K * w->chunks * kPeaks;
     w->part_pow = take(8 * parts);
@@ -788,7 +792,8 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
                  (split && gen) ? 1 : 0, obj_shift, obj_scale, obj_gen,
                  mfma ? reinterpret_cast<float *>(ws + w.obj_ys) : nullptr, a->t,
                  mfma ? reinterpret_cast<double *>(ws + w.rec_t) : nullptr,
-                 mfma ? reinterpret_cast<double2 *>(ws + w.rec_r) : nullptr, obj_ip, dw * kInv2Pi,
+                 mfma ? reinterpret_cast<double2 *>(ws + w.rec_r) : nullptr,
+                 mfma ? reinterpret_cast<uint32_t *>(ws + w.slot_obj) : nullptr, obj_ip, dw * kInv2Pi,
                  w.screen ? kIpSigmaScreen : gen ? kIpSigmaGen : kIpSigma,
                  w.screen ? (gen ? kIpLeastObsScreenGen : kIpLeastObsScreen) : kIpLeastObs, w.screen ? 1 : 2, w.screen ? 1 : 0};
     if (split) {
@@ -870,6 +875,7 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
     sw.top_k = (int)a->top_k;
     sw.colfac = w.colfac ? reinterpret_cast<uint4 *>(ws + w.colfac) : nullptr;
     sw.rowfac = w.rowfac ? reinterpret_cast<uint4 *>(ws + w.rowfac) : nullptr;
+    sw.slot_obj = mfma ? reinterpret_cast<uint32_t *>(ws + w.slot_obj) : nullptr;
     sw.obj_ys = w.obj_ys ? reinterpret_cast<float *>(ws + w.obj_ys) : nullptr;
 
     if (w.interp) {
@@ -917,10 +923,7 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
         LS_HIP(timing_events(tm));
         LS_HIP(hipEventRecord(tm.ev[0], st));
     }
-    // wavefronts per object of its set-up: enough for the mean object's
-    // 16-observation blocks, up to 256 (one object of many observations)
-    const uint64_t blocks = (a->num_obs / 16 + K - 1) / K + 1;
-    const uint32_t gy = (uint32_t)std::min<uint64_t>(256, blocks);
+    const uint32_t slots = (uint32_t)(a->num_obs / 16 + K + 1);
     if (w.interp) {
         // The coarse-grid sweep, the marks of the chunks to sweep again and the
         // direct tile's tables (which replace the coarse ones) in one launch,
@@ -934,7 +937,7 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
         const uint32_t per_obj = (si.ip_items + si.group - 1) / si.group;
         si.xcd_run = per_obj;
         void *iargs[] = {&si};
-        LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(ip.fac), dim3(K + 1 + 3 * kIpModes, gy), dim3(64), iargs, 0,
+        LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(ip.fac), dim3(1 + 3 * kIpModes + slots), dim3(64), iargs, 0,
                                st));
         const uint64_t ip_groups = (uint64_t)K * per_obj, most = 0xFFFFFFFFull / (uint64_t)ip.threads - 1;
         for (uint64_t g = 0; g < ip_groups; g += most) {
@@ -954,7 +957,7 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
         sd.marked_groups = sd.cand ? (K * sd.cand_split + 7u) & ~7u : 0u;
         void *dargs[] = {&sd};
         if (sd.cand)
-            LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->prep), dim3(K, gy + 1u), dim3(64), dargs, 0, st));
+            LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->prep), dim3(K + slots), dim3(64), dargs, 0, st));
         const uint64_t launch_most = 0xFFFFFFFFull / (uint64_t)T - 1;
         for (uint64_t g = 0; g < groups;) {
             const uint64_t cnt = std::min<uint64_t>(launch_most - sd.marked_groups, groups - g);
@@ -966,7 +969,7 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
         }
     } else if (te->prep) {  // per-object set-up of the tile, inside the timed sweep
         void *kargs[] = {&sw};
-        LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->prep), dim3(K, gy), dim3(64), kargs, 0, st));
+        LS_HIP(hipLaunchKernel(reinterpret_cast<const void *>(te->prep), dim3(slots), dim3(64), kargs, 0, st));
     }
     if (w.interp) {
         // done

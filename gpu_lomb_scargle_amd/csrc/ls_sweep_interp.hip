@@ -134,25 +134,25 @@ __device__ void list_direct(const SweepArgs &a) {
     if (lane == 0) *a.direct_count = count;
 }
 
-// Workgroups past the last object list the objects in direct mode (blockIdx.x =
-// K) and write the interpolation operands (K + 1 + 3 (mode - 1) + which third).  Wavefronts (object, y) write the tables of the object's 16-observation
-// blocks y, y + gridDim.y, ..., as k_colfac does for the direct tile, into the
-// same slots (objects in direct mode: the direct tile's themselves): column factors e^{2 pi i (b + 1/2) h df t'} a / Phi (b < 32) of the
+// The first workgroups list the objects in direct mode (blockIdx.x = 0) and
+// write the interpolation operands (1 + 3 (mode - 1) + which third).  The others
+// write the tables of a slot's 16 observations, as k_colfac does for the direct
+// tile, into the same slots (objects in direct mode: the direct tile's
+// themselves): column factors e^{2 pi i (b + 1/2) h df t'} a / Phi (b < 32) of the
 // two weights a = y (generalized: (w/W) (y - ybar)) and a = 1 (w/W), four head
 // and tail fragments each, and the row steps e^{2 pi i 64 a h df t'} (a < 32),
 // with t' = t - tc and 1/Phi from the records.
 template <bool GEN, typename IN, bool SCREEN>
 __global__ __launch_bounds__(64) void k_interp_fac(SweepArgs a) {
     constexpr int FR = ip_frags(SCREEN), NC = SCREEN ? 1 : 2;  // fragments; heads alone or with tails
-    const uint32_t pos = blockIdx.x, l = threadIdx.x;
-    if (pos >= a.K) {
-        if (blockIdx.y != 0) return;
-        if (pos == a.K) return list_direct(a);
-        return interp_table<SCREEN>(a.ip_tab, (int)(pos - a.K - 1u) / 3 + 1, (int)(pos - a.K - 1u) % 3);
-    }
-    const uint32_t k = a.order ? a.order[pos] : pos;
+    const uint32_t l = threadIdx.x;
+    if (blockIdx.x == 0) return list_direct(a);
+    if (blockIdx.x <= 3u * kIpModes)
+        return interp_table<SCREEN>(a.ip_tab, (int)(blockIdx.x - 1u) / 3 + 1, (int)(blockIdx.x - 1u) % 3);
+    uint32_t k, q;
+    if (!slot_block(a, blockIdx.x - 1u - 3u * kIpModes, k, q)) return;
     const int mode = (int)a.obj_ip[k].mode;
-    if (mode == 0) return direct_tables<GEN, IN>(a, k, blockIdx.y, gridDim.y);
+    if (mode == 0) return direct_table<GEN, IN>(a, k, q);
     const uint64_t beg = a.offsets[k], end = a.offsets[k + 1];
     const uint32_t n = (uint32_t)(end - beg);
     const IN *y = static_cast<const IN *>(a.y);
@@ -168,56 +168,54 @@ __global__ __launch_bounds__(64) void k_interp_fac(SweepArgs a) {
     constexpr int NF = GEN ? kColfacFragsGen : kColfacFragsStd;
     uint4 *dst = a.colfac + colfac_slot(beg, k) * (uint64_t)(NF * 64) + l;
     uint4 *rdst = a.rowfac + colfac_slot(beg, k) * (uint64_t)(kRowfacFrags * 64) + l;
-    for (uint32_t q = blockIdx.y; q * 16u < n; q += gridDim.y) {
-        half8_t f[FR];
+    half8_t f[FR];
 #pragma unroll
-        for (int v = 0; v < 8; v += 2) {
-            double x[4][2];
-            float r4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int v = 0; v < 8; v += 2) {
+        double x[4][2];
+        float r4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const uint32_t j = q * 16u + 8u * (l >> 5) + (uint32_t)(v + e);
-                double cb = 0.0, sb = 0.0, yv = 0.0, wv = 0.0;
-                if (j < n) {
-                    const double2 tp = a.rec_r[beg + j];  // t', 1/Phi
-                    double c, sn;
-                    ip_phasor<SCREEN>(fr, tp.x, c, sn);
-                    r4[2 * e] = (float)c;
-                    r4[2 * e + 1] = (float)sn;
-                    ip_phasor<SCREEN>(fb, tp.x, cb, sb);
-                    double w = 1.0, yj = (double)y[beg + j];
-                    if constexpr (GEN) {
-                        const double d = (double)dy[beg + j];
-                        w = iW / (d * d);
-                        yj = w * (yj - ybar);
-                    }
-                    yv = yj * sy * tp.y;
-                    wv = w * sw * tp.y;
+        for (int e = 0; e < 2; ++e) {
+            const uint32_t j = q * 16u + 8u * (l >> 5) + (uint32_t)(v + e);
+            double cb = 0.0, sb = 0.0, yv = 0.0, wv = 0.0;
+            if (j < n) {
+                const double2 tp = a.rec_r[beg + j];  // t', 1/Phi
+                double c, sn;
+                ip_phasor<SCREEN>(fr, tp.x, c, sn);
+                r4[2 * e] = (float)c;
+                r4[2 * e + 1] = (float)sn;
+                ip_phasor<SCREEN>(fb, tp.x, cb, sb);
+                double w = 1.0, yj = (double)y[beg + j];
+                if constexpr (GEN) {
+                    const double d = (double)dy[beg + j];
+                    w = iW / (d * d);
+                    yj = w * (yj - ybar);
                 }
-                x[0][e] = yv * cb;
-                x[1][e] = yv * sb;
-                x[2][e] = wv * cb;
-                x[3][e] = wv * sb;
+                yv = yj * sy * tp.y;
+                wv = w * sw * tp.y;
             }
-            uint4 u;
-            __builtin_memcpy(&u, r4, sizeof(u));
-            rdst[(uint64_t)(q * kRowfacFrags + (uint32_t)(v >> 1)) * 64] = u;
+            x[0][e] = yv * cb;
+            x[1][e] = yv * sb;
+            x[2][e] = wv * cb;
+            x[3][e] = wv * sb;
+        }
+        uint4 u;
+        __builtin_memcpy(&u, r4, sizeof(u));
+        rdst[(uint64_t)(q * kRowfacFrags + (uint32_t)(v >> 1)) * 64] = u;
 #pragma unroll
-            for (int p = 0; p < 4; ++p) {
-                half2_t hd, tl;
-                split64x2(x[p][0], x[p][1], hd, tl);
-                f[NC * p][v] = hd.x; f[NC * p][v + 1] = hd.y;
-                if constexpr (!SCREEN) {
-                    f[2 * p + 1][v] = tl.x; f[2 * p + 1][v + 1] = tl.y;
-                }
+        for (int p = 0; p < 4; ++p) {
+            half2_t hd, tl;
+            split64x2(x[p][0], x[p][1], hd, tl);
+            f[NC * p][v] = hd.x; f[NC * p][v + 1] = hd.y;
+            if constexpr (!SCREEN) {
+                f[2 * p + 1][v] = tl.x; f[2 * p + 1][v + 1] = tl.y;
             }
         }
+    }
 #pragma unroll
-        for (int i = 0; i < FR; ++i) {
-            uint4 u;
-            __builtin_memcpy(&u, &f[i], sizeof(u));
-            dst[(uint64_t)(q * FR + i) * 64] = u;
-        }
+    for (int i = 0; i < FR; ++i) {
+        uint4 u;
+        __builtin_memcpy(&u, &f[i], sizeof(u));
+        dst[(uint64_t)(q * FR + i) * 64] = u;
     }
 }
 

@@ -710,15 +710,18 @@ __device__ void mark_chunks(const SweepArgs &a, uint32_t obj) {
     }
 }
 
-// Tables of the direct tile, wavefronts (object, y).  Beside the coarse-grid
-// sweep: the marks of its objects (the last y) and their tables, which replace
-// the coarse ones; those of the objects in direct mode are there already.
+// Tables of the direct tile, a wavefront per slot.  Beside the coarse-grid
+// sweep: first the marks of its objects, a wavefront each, and then their tables,
+// which replace the coarse ones; those of the objects in direct mode are there
+// already.
 template <bool GEN, typename IN>
 __global__ __launch_bounds__(64) void k_colfac(SweepArgs a) {
-    const uint32_t gy = gridDim.y - (a.cand ? 1u : 0u);
-    if (blockIdx.y == gy) return mark_chunks(a, blockIdx.x);
-    if (a.obj_ip && a.obj_ip[blockIdx.x].mode == 0u) return;
-    direct_tables<GEN, IN>(a, blockIdx.x, blockIdx.y, gy);
+    const uint32_t marks = a.cand ? a.K : 0u;
+    if (blockIdx.x < marks) return mark_chunks(a, blockIdx.x);
+    uint32_t obj, block;
+    if (!slot_block(a, blockIdx.x - marks, obj, block)) return;
+    if (a.obj_ip && a.obj_ip[obj].mode == 0u) return;
+    direct_table<GEN, IN>(a, obj, block);
 }
 
 // Row factors of a 16-observation block for lane (row rc, half kh): u = u0 R
