@@ -33,7 +33,7 @@ SCHEDULE_GRID, SCHEDULE_PERSISTENT = 0, 1
 # drop-in libraries).
 EXPORTED = [
     "lsamd_sweep_workspace_size", "lsamd_sweep", "lsamd_batch_host", "lsamd_cpu_batch",
-    "lsamd_cpu_single", "lsamd_count_objects", "lsamd_object_offsets", "lsamd_last_error_code",
+    "lsamd_cpu_single", "lsamd_row_argmax", "lsamd_count_objects", "lsamd_object_offsets", "lsamd_last_error_code",
     "lsamd_last_error", "lsamd_clear_error", "lsamd_device_count", "lsamd_set_timing",
     "lsamd_last_sweep_kernel_ms", "lsamd_set_tile", "lsamd_get_tile", "lsamd_version",
     "lsamd_graph_create", "lsamd_graph_launch", "lsamd_graph_destroy", "lsamd_autotune",
@@ -93,6 +93,8 @@ def _declare(L):
     L.lsamd_cpu_single.argtypes = [c_int, c_int, c_int, c_void_p, c_void_p, c_void_p, c_uint64,
                                    c_double, c_double, c_uint32, c_void_p, c_int]
     L.lsamd_cpu_single.restype = c_int
+    L.lsamd_row_argmax.argtypes = [c_int, c_void_p, c_uint64, c_uint64, c_void_p]
+    L.lsamd_row_argmax.restype = c_int
     L.lsamd_count_objects.argtypes = [c_void_p, c_uint64]
     L.lsamd_count_objects.restype = c_uint32
     L.lsamd_object_offsets.argtypes = [c_void_p, c_uint64, c_void_p, c_void_p]

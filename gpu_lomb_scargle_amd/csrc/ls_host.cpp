@@ -3,12 +3,26 @@
 // pre-centring, device buffers, memory-budget batching and the pinned,
 // double-buffered copy of the periodogram back into the caller's memory.
 //
+// A drop-in call on a few stars is all latency, a catalogue's mostly the way of
+// its periodogram into fresh host memory.  So small inputs travel packed, in one
+// copy; outputs of up to 256 MiB are written by the sweep itself into pinned
+// memory, a slice of objects at a time, and copied from there, page faults
+// included, while the next slices are swept.  No copy queue takes part: copies
+// are kernels here, and two streams of a process with several libraries may
+// share a hardware queue, where a copy waits for every sweep enqueued before it.
+// Larger outputs go through device memory and staging buffers as before.
+// Whole call, us: one star of 29 observations, 1188 bins, 204 -> 99; 136 stars
+// x 100,000 bins, generalized FP32 (54 MB), 7678 -> 4840 (the sweep alone 3530; with
+// slices copied on a second stream 5400, or 8700 beside another library).
+//
 // Replaces the reference's GPU host path: computeObjectRanges
 // (source/main.cu:468-510), computeNumBatches (main.cu:423-466),
 // batchGPULSWrapper / batchGPULS (main.cu:742-1280), GPULSOneObject
 // (main.cu:570-720) and pinnedMemoryCopyDtoH (main.cu:513-559).
 
 #include <hip/hip_runtime.h>
+
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <cmath>
@@ -93,17 +107,25 @@ struct DevBuf {
     size_t cap = 0;
 };
 
+// Slices whose sweeps are enqueued, each with pinned memory of its own, before the
+// first of them is copied on, at most.
+constexpr size_t kAhead = 4;
+
 struct Ctx {
     std::mutex mu;
     bool ready = false;
     int device = -1;
     hipStream_t stream = nullptr;       // uploads and sweeps
     hipStream_t copy_stream = nullptr;  // periodogram copy-back
-    DevBuf t, y, dy, off, order, ws, pgram, pidx, ppow, pper;
+    DevBuf in, ws, pgram, peaks;
+    char *io = nullptr;                 // pinned: packed inputs, then small outputs
+    bool busy = false;                  // a call is enqueued (or failed half-way)
     void *pinned[2] = {nullptr, nullptr};
     size_t pinned_cap = 0;
     hipEvent_t ev[2] = {nullptr, nullptr};     // staging chunks (copy stream)
-    hipEvent_t slice[2] = {nullptr, nullptr};  // sweep of a slice done (sweep stream)
+    hipEvent_t slice[kAhead] = {};             // sweep of a slice done (sweep stream)
+    char *ring[kAhead] = {};                   // pinned: periodograms of the slices under way
+    size_t ring_cap = 0;                       // bytes of each
 };
 
 // One context per device, for the device current on the calling thread.
@@ -141,14 +163,20 @@ Ctx *ctx_for_current_device(int *err) {
                              std::string(#call) + ": " + hipGetErrorString(e_));              \
     } while (0)
 
+// Pinned room of a context: packed inputs (larger ones are copied from the
+// caller's arrays), and outputs (larger ones go through the staging buffers).
+constexpr size_t kIoIn = size_t(1) << 20, kIoOut = size_t(8) << 20;
+// Periodograms up to here are written into pinned memory in slices of at most
+// kRingSlice.
+constexpr size_t kRingTotal = size_t(256) << 20, kRingSlice = size_t(32) << 20;
+
 int ctx_init(Ctx &c) {
     if (c.ready) return LSAMD_OK;
     HIP_OK(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking));
     HIP_OK(hipStreamCreateWithFlags(&c.copy_stream, hipStreamNonBlocking));
-    for (int i = 0; i < 2; ++i) {
-        HIP_OK(hipEventCreateWithFlags(&c.ev[i], hipEventDisableTiming));
-        HIP_OK(hipEventCreateWithFlags(&c.slice[i], hipEventDisableTiming));
-    }
+    for (hipEvent_t &e : c.ev) HIP_OK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    for (hipEvent_t &e : c.slice) HIP_OK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    HIP_OK(hipHostMalloc(reinterpret_cast<void **>(&c.io), kIoIn + kIoOut, hipHostMallocCoherent));
     c.ready = true;
     return LSAMD_OK;
 }
@@ -166,49 +194,102 @@ int ensure(DevBuf &b, size_t bytes) {
     return LSAMD_OK;
 }
 
-constexpr size_t kPinnedChunk = size_t(64) << 20;  // 64 MiB per staging buffer
+constexpr size_t kPinnedChunk = size_t(64) << 20;  // a staging buffer, at most
+
+// Pinned to pageable memory: first touches of fresh pages dominate, which
+// threads share.
+void host_copy(char *to, const char *from, size_t len) {
+    if (len <= (size_t(1) << 20)) {
+        std::memcpy(to, from, len);
+        return;
+    }
+    const size_t parts = 8, step = (len + parts - 1) / parts;
+#pragma omp parallel for num_threads(8) schedule(static)
+    for (long long p = 0; p < (long long)parts; ++p) {
+        const size_t a = (size_t)p * step;
+        if (a < len) std::memcpy(to + a, from + a, std::min(step, len - a));
+    }
+}
 
 // Device -> pageable host copy on the copy stream through two pinned staging
-// buffers, so the DMA of one chunk overlaps the host copy of the previous one.
-// Returns when the data is in dst.
+// buffers, so the DMA of one chunk overlaps the host copy of the previous one:
+// four chunks or more, of 2 to 64 MiB.  Returns when the data is in dst.
 int copy_to_host(Ctx &c, void *dst, const void *src, size_t bytes) {
     if (bytes == 0) return LSAMD_OK;
-    if (bytes <= (size_t(8) << 20)) {
-        HIP_OK(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, c.copy_stream));
-        HIP_OK(hipStreamSynchronize(c.copy_stream));
-        return LSAMD_OK;
-    }
-    if (c.pinned_cap < kPinnedChunk) {
+    const size_t chunk = std::min(kPinnedChunk, std::max(size_t(2) << 20, (bytes / 4 + 4095) & ~size_t(4095)));
+    if (c.pinned_cap < chunk) {
+        c.pinned_cap = 0;
         for (int i = 0; i < 2; ++i) {
             if (c.pinned[i]) HIP_OK(hipHostFree(c.pinned[i]));
             c.pinned[i] = nullptr;
-            HIP_OK(hipHostMalloc(&c.pinned[i], kPinnedChunk, hipHostMallocDefault));
+            HIP_OK(hipHostMalloc(&c.pinned[i], chunk, hipHostMallocDefault));
         }
-        c.pinned_cap = kPinnedChunk;
+        c.pinned_cap = chunk;
     }
-    const size_t nch = (bytes + kPinnedChunk - 1) / kPinnedChunk;
-    auto chunk_len = [&](size_t i) { return std::min(kPinnedChunk, bytes - i * kPinnedChunk); };
+    const size_t nch = (bytes + chunk - 1) / chunk;
+    auto chunk_len = [&](size_t i) { return std::min(chunk, bytes - i * chunk); };
     const char *s = static_cast<const char *>(src);
     char *d = static_cast<char *>(dst);
     HIP_OK(hipMemcpyAsync(c.pinned[0], s, chunk_len(0), hipMemcpyDeviceToHost, c.copy_stream));
     HIP_OK(hipEventRecord(c.ev[0], c.copy_stream));
     for (size_t i = 1; i <= nch; ++i) {
         if (i < nch) {
-            HIP_OK(hipMemcpyAsync(c.pinned[i & 1], s + i * kPinnedChunk, chunk_len(i),
-                                  hipMemcpyDeviceToHost, c.copy_stream));
+            HIP_OK(hipMemcpyAsync(c.pinned[i & 1], s + i * chunk, chunk_len(i), hipMemcpyDeviceToHost,
+                                  c.copy_stream));
             HIP_OK(hipEventRecord(c.ev[i & 1], c.copy_stream));
         }
         HIP_OK(hipEventSynchronize(c.ev[(i - 1) & 1]));
-        const size_t len = chunk_len(i - 1);
-        const char *from = static_cast<const char *>(c.pinned[(i - 1) & 1]);
-        char *to = d + (i - 1) * kPinnedChunk;
-        const size_t parts = 8, step = (len + parts - 1) / parts;
-#pragma omp parallel for num_threads(8) schedule(static)
-        for (long long p = 0; p < (long long)parts; ++p) {
-            const size_t a = (size_t)p * step;
-            if (a < len) std::memcpy(to + a, from + a, std::min(step, len - a));
+        host_copy(d + (i - 1) * chunk, static_cast<const char *>(c.pinned[(i - 1) & 1]), chunk_len(i - 1));
+    }
+    return LSAMD_OK;
+}
+
+// numpy.argmax of a row: the first NaN, else the first maximum.
+template <typename R>
+uint64_t row_argmax(const R *x, uint64_t n) {
+    constexpr uint64_t kBlock = 512, kLanes = 16;
+    R best = x[0];
+    uint64_t at = 0;
+    for (uint64_t b = 0; b < n; b += kBlock) {
+        const uint64_t len = std::min(kBlock, n - b);
+        const R *p = x + b;
+        R m[kLanes];
+        int odd[kLanes] = {};
+        uint64_t i = 0;
+        if (len >= kLanes) {
+            for (uint64_t l = 0; l < kLanes; ++l) m[l] = p[l];
+            for (; i + kLanes <= len; i += kLanes)
+                for (uint64_t l = 0; l < kLanes; ++l) {
+                    const R v = p[i + l];
+                    m[l] = v > m[l] ? v : m[l];
+                    odd[l] |= v != v;
+                }
+        }
+        bool some = false;  // a NaN, or more than the best so far
+        if (len >= kLanes)
+            for (uint64_t l = 0; l < kLanes; ++l) some |= odd[l] != 0 || m[l] > best;
+        for (; i < len; ++i) some |= p[i] != p[i] || p[i] > best;
+        if (!some && !(b == 0 && best != best)) continue;
+        for (i = 0; i < len; ++i) {
+            if (p[i] != p[i]) return b + i;
+            if (p[i] > best) {
+                best = p[i];
+                at = b + i;
+            }
         }
     }
+    return at;
+}
+
+int ensure_ring(Ctx &c, size_t bytes) {
+    if (c.ring_cap >= bytes) return LSAMD_OK;
+    c.ring_cap = 0;
+    for (char *&r : c.ring) {
+        if (r) HIP_OK(hipHostFree(r));
+        r = nullptr;
+        HIP_OK(hipHostMalloc(reinterpret_cast<void **>(&r), bytes, hipHostMallocCoherent));
+    }
+    c.ring_cap = bytes;
     return LSAMD_OK;
 }
 
@@ -299,42 +380,44 @@ int lsamd_batch_host(int variant, int dtype, int form, int normalize, int precen
     rc = ctx_init(c);
     if (rc) return rc;
 
+    // an earlier call that failed half-way may still use the pinned memory
+    if (c.busy) {
+        HIP_OK(hipStreamSynchronize(c.stream));
+        HIP_OK(hipStreamSynchronize(c.copy_stream));
+    }
+    c.busy = true;
+
     // memory budget for the periodogram (computeNumBatches, main.cu:423-466):
     // a fraction of the free device memory, LSAMD_MEM_FRACTION (default 0.5),
-    // or an absolute LSAMD_PGRAM_BUDGET_BYTES.
-    size_t freeb = 0, totalb = 0;
-    HIP_OK(hipMemGetInfo(&freeb, &totalb));
-    size_t budget = (size_t)(env_double("LSAMD_MEM_FRACTION", 0.5) * (double)freeb);
-    const double abs_budget = env_double("LSAMD_PGRAM_BUDGET_BYTES", 0.0);
-    if (abs_budget > 0) budget = (size_t)abs_budget;
+    // or an absolute LSAMD_PGRAM_BUDGET_BYTES.  What an earlier call's buffer
+    // holds needs no look at the free memory.
     const size_t per_obj = pgram ? (size_t)nf * rsz : 0;
+    const double abs_budget = env_double("LSAMD_PGRAM_BUDGET_BYTES", 0.0);
+    const double fraction = env_double("LSAMD_MEM_FRACTION", -1.0);
     uint32_t objs_per_batch = K;
-    if (per_obj > 0) {
+    const bool ring_call = pgram && (size_t)K * per_obj <= kRingTotal && per_obj <= kRingSlice && !(abs_budget > 0) &&
+                           fraction < 0;
+    if (per_obj > 0 && !ring_call && (abs_budget > 0 || fraction >= 0 || c.pgram.cap / per_obj < K)) {
+        size_t budget = (size_t)abs_budget;
+        if (!(abs_budget > 0)) {
+            size_t freeb = 0, totalb = 0;
+            HIP_OK(hipMemGetInfo(&freeb, &totalb));
+            budget = (size_t)((fraction >= 0 ? fraction : 0.5) * (double)freeb);
+        }
         const size_t fit = std::max<size_t>(1, budget / per_obj);
         objs_per_batch = (uint32_t)std::min<size_t>(K, fit);
     }
 
-    // inputs, once
-    rc = ensure(c.t, n * rsz);
-    if (!rc) rc = ensure(c.y, n * rsz);
-    if (!rc && variant == LSAMD_GENERALIZED) rc = ensure(c.dy, n * rsz);
-    if (!rc) rc = ensure(c.off, ((size_t)K + 1) * 8);
-    if (!rc) rc = ensure(c.order, (size_t)K * 4);
-    if (rc) return rc;
-    HIP_OK(hipMemcpyAsync(c.t.p, t, n * rsz, hipMemcpyHostToDevice, c.stream));
-    HIP_OK(hipMemcpyAsync(c.y.p, y, n * rsz, hipMemcpyHostToDevice, c.stream));
-    if (variant == LSAMD_GENERALIZED)
-        HIP_OK(hipMemcpyAsync(c.dy.p, dy, n * rsz, hipMemcpyHostToDevice, c.stream));
-    HIP_OK(hipMemcpyAsync(c.off.p, off.data(), ((size_t)K + 1) * 8, hipMemcpyHostToDevice,
-                          c.stream));
-
     // Each memory-budget batch is swept in slices of objects: while the
-    // periodogram of slice s is copied back on the copy stream, slice s+1 is
-    // swept, so the end-to-end time approaches the copy time alone.  Slices
-    // hold ~2 GiB of periodogram (at least 1 object; LSAMD_SLICE_BYTES
-    // overrides): each slice's copy restarts the two-buffer staging pipeline,
-    // so slices much smaller than that lose copy bandwidth.
-    const size_t kSliceBytes = (size_t)env_double("LSAMD_SLICE_BYTES", (double)(size_t(2) << 30));
+    // periodogram of slice s is copied back, slice s+1 is swept, so the
+    // end-to-end time approaches the longer of the two.  A slice in pinned memory
+    // holds an eighth of the periodogram, 8 to 32 MiB, one in device memory 2 GiB
+    // (at least 1 object; LSAMD_SLICE_BYTES overrides): each slice's copy through
+    // the staging buffers restarts their pipeline.
+    const size_t eighth = std::min(kRingSlice, std::max(size_t(8) << 20, (size_t)K * per_obj / 8));
+    const size_t most = ring_call ? kRingSlice : size_t(2) << 30;
+    const size_t kSliceBytes =
+        std::min(most, (size_t)env_double("LSAMD_SLICE_BYTES", ring_call ? (double)eighth : (double)most));
     const uint32_t objs_per_slice =
         per_obj > 0 ? (uint32_t)std::max<size_t>(1, std::min<size_t>(objs_per_batch, kSliceBytes / per_obj))
                     : objs_per_batch;
@@ -353,20 +436,58 @@ int lsamd_batch_host(int variant, int dtype, int form, int normalize, int precen
             return off[s0 + a + 1] - off[s0 + a] > off[s0 + b + 1] - off[s0 + b];
         });
     }
-    HIP_OK(hipMemcpyAsync(c.order.p, order.data(), (size_t)K * 4, hipMemcpyHostToDevice,
-                          c.stream));
 
+    // inputs, once: one device buffer, each part on a 256-byte boundary
+    size_t in_bytes = 0;
+    auto part = [](size_t &at, size_t bytes) {
+        const size_t o = at;
+        at += (bytes + 255) & ~size_t(255);
+        return o;
+    };
+    const size_t in_t = part(in_bytes, n * rsz), in_y = part(in_bytes, n * rsz);
+    const size_t in_dy = part(in_bytes, variant == LSAMD_GENERALIZED ? n * rsz : 0);
+    const size_t in_off = part(in_bytes, ((size_t)K + 1) * 8), in_order = part(in_bytes, (size_t)K * 4);
+    rc = ensure(c.in, in_bytes);
+    if (rc) return rc;
+    char *const in = static_cast<char *>(c.in.p);
+    const bool packed = in_bytes <= kIoIn;
+    auto upload = [&](size_t at, const void *from, size_t bytes) -> int {
+        if (packed) std::memcpy(c.io + at, from, bytes);
+        else HIP_OK(hipMemcpyAsync(in + at, from, bytes, hipMemcpyHostToDevice, c.stream));
+        return LSAMD_OK;
+    };
+    rc = upload(in_t, t, n * rsz);
+    if (!rc) rc = upload(in_y, y, n * rsz);
+    if (!rc && variant == LSAMD_GENERALIZED) rc = upload(in_dy, dy, n * rsz);
+    if (!rc) rc = upload(in_off, off.data(), ((size_t)K + 1) * 8);
+    if (!rc) rc = upload(in_order, order.data(), (size_t)K * 4);
+    if (rc) return rc;
+    if (packed) HIP_OK(hipMemcpyAsync(in, c.io, in_bytes, hipMemcpyHostToDevice, c.stream));
+
+    // Fresh memory is touched for the first time by the copy-back: with pages of
+    // 2 MiB where the system has them.
+    if (pgram && (size_t)K * per_obj >= (size_t(8) << 20)) {
+        const uintptr_t page = (uintptr_t)2 << 20, p0 = reinterpret_cast<uintptr_t>(pgram);
+        const uintptr_t lo = (p0 + page - 1) & ~(page - 1), hi = (p0 + (size_t)K * per_obj) & ~(page - 1);
+        if (hi > lo) (void)madvise(reinterpret_cast<void *>(lo), hi - lo, MADV_HUGEPAGE);
+    }
+
+    // outputs: the peaks, and behind them the periodogram of a small call, in one
+    // run of pinned memory; a larger periodogram in the ring or a device buffer
     const uint32_t tk = top_k;
-    if (tk) {
-        rc = ensure(c.pidx, (size_t)K * tk * 4);
-        if (!rc) rc = ensure(c.ppow, (size_t)K * tk * rsz);
-        if (!rc) rc = ensure(c.pper, (size_t)K * tk * rsz);
-        if (rc) return rc;
-    }
-    if (pgram) {
-        rc = ensure(c.pgram, (size_t)objs_per_batch * per_obj);
-        if (rc) return rc;
-    }
+    size_t out_bytes = 0;
+    const size_t out_idx = part(out_bytes, (size_t)K * tk * 4), out_pow = part(out_bytes, (size_t)K * tk * rsz);
+    const size_t out_per = part(out_bytes, (size_t)K * tk * rsz), peak_bytes = out_bytes;
+    const size_t out_pg = part(out_bytes, (size_t)K * per_obj);
+    const bool small = out_bytes <= kIoOut && slice_start.size() == 1;
+    const bool ring = ring_call && !small;
+    const bool peaks_pinned = peak_bytes <= kIoOut;
+    char *const io_out = c.io + kIoIn;
+    if (!peaks_pinned) rc = ensure(c.peaks, peak_bytes);
+    if (!rc && ring) rc = ensure_ring(c, (size_t)objs_per_slice * per_obj);
+    if (!rc && pgram && !ring && !small) rc = ensure(c.pgram, (size_t)objs_per_batch * per_obj);
+    if (rc) return rc;
+    char *const peaks = peaks_pinned ? io_out : static_cast<char *>(c.peaks.p);
 
     // slice i covers objects [s0, s1) and, inside its batch, periodogram rows
     // from (s0 - batch start); a slice never spans two batches
@@ -390,19 +511,22 @@ int lsamd_batch_host(int variant, int dtype, int form, int normalize, int precen
         a.num_obs = n;
         a.min_freq = fmin;
         a.max_freq = fmax;
-        a.offsets = static_cast<const uint64_t *>(c.off.p) + s0;
-        a.order = static_cast<const uint32_t *>(c.order.p) + s0;
-        a.t = c.t.p;
-        a.y = c.y.p;
-        a.dy = variant == LSAMD_GENERALIZED ? c.dy.p : nullptr;
-        a.pgram = pgram ? static_cast<char *>(c.pgram.p) + batch_row(s0) * per_obj : nullptr;
+        a.offsets = reinterpret_cast<const uint64_t *>(in + in_off) + s0;
+        a.order = reinterpret_cast<const uint32_t *>(in + in_order) + s0;
+        a.t = in + in_t;
+        a.y = in + in_y;
+        a.dy = variant == LSAMD_GENERALIZED ? in + in_dy : nullptr;
+        a.pgram = !pgram  ? nullptr
+                  : small ? io_out + out_pg
+                  : ring  ? c.ring[i % kAhead]
+                          : static_cast<char *>(c.pgram.p) + batch_row(s0) * per_obj;
         // a call of one object may slice its observations; sub-sweeps of a
         // larger call never do, so batching cannot change any result
         a.obs_slices = K == 1 ? 0 : 1;
         if (tk) {
-            a.peak_index = static_cast<uint32_t *>(c.pidx.p) + (size_t)s0 * tk;
-            a.peak_power = static_cast<char *>(c.ppow.p) + (size_t)s0 * tk * rsz;
-            a.peak_period = static_cast<char *>(c.pper.p) + (size_t)s0 * tk * rsz;
+            a.peak_index = reinterpret_cast<uint32_t *>(peaks + out_idx) + (size_t)s0 * tk;
+            a.peak_power = peaks + out_pow + (size_t)s0 * tk * rsz;
+            a.peak_period = peaks + out_per + (size_t)s0 * tk * rsz;
         }
         const size_t wsb = sweep_part_bytes(&a, K);
         int r = LSAMD_OK;
@@ -414,52 +538,68 @@ int lsamd_batch_host(int variant, int dtype, int form, int normalize, int precen
         }
         r = sweep_part(&a, K, c.ws.p, c.ws.cap, c.stream);
         if (r) return r;
-        HIP_OK(hipEventRecord(c.slice[i & 1], c.stream));
+        if (!small) HIP_OK(hipEventRecord(c.slice[i % kAhead], c.stream));
         return LSAMD_OK;
     };
     auto copy_slice = [&](size_t i) -> int {
         const uint32_t s0 = slice_start[i], s1 = slice_end(i);
-        HIP_OK(hipStreamWaitEvent(c.copy_stream, c.slice[i & 1], 0));
-        return copy_to_host(c, static_cast<char *>(pgram) + (size_t)s0 * per_obj,
-                            static_cast<char *>(c.pgram.p) + batch_row(s0) * per_obj,
-                            (size_t)(s1 - s0) * per_obj);
+        char *const to = static_cast<char *>(pgram) + (size_t)s0 * per_obj;
+        const size_t bytes = (size_t)(s1 - s0) * per_obj;
+        if (ring) {
+            HIP_OK(hipEventSynchronize(c.slice[i % kAhead]));
+            host_copy(to, c.ring[i % kAhead], bytes);
+            return LSAMD_OK;
+        }
+        HIP_OK(hipStreamWaitEvent(c.copy_stream, c.slice[i % kAhead], 0));
+        return copy_to_host(c, to, static_cast<char *>(c.pgram.p) + batch_row(s0) * per_obj, bytes);
     };
-    const size_t ns = slice_start.size();
-    rc = sweep_slice(0);
-    if (rc) return rc;
-    for (size_t i = 1; i <= ns; ++i) {
-        // Within a batch, slice i writes other device rows than slice i-1, so
-        // it is swept while slice i-1 is copied back.  The first slice of a
-        // new batch reuses rows from 0, which the still-pending last slice of
-        // the previous batch may occupy: that slice is copied back first
-        // (copy_slice returns once the data is in host memory).
-        const bool next = i < ns;
-        const bool new_batch = next && slice_start[i] % objs_per_batch == 0;
-        if (next && !new_batch) {
-            rc = sweep_slice(i);
+    // Within a batch the slices' rows are apart: the next sweeps are enqueued (as
+    // many as the ring holds, else one) while a slice is copied back.  A new
+    // batch reuses the rows, and is enqueued when the last slice before it is in
+    // host memory (copy_slice returns then).
+    const size_t ns = slice_start.size(), ahead = ring ? kAhead : 2;
+    for (size_t i = 0, queued = 0; i < ns; ++i) {
+        for (; queued < ns && queued < i + ahead &&
+               slice_start[queued] / objs_per_batch == slice_start[i] / objs_per_batch;
+             ++queued) {
+            rc = sweep_slice(queued);
             if (rc) return rc;
         }
-        if (pgram) {
-            rc = copy_slice(i - 1);
-            if (rc) return rc;
-        }
-        if (new_batch) {
-            rc = sweep_slice(i);
+        if (pgram && !small) {
+            rc = copy_slice(i);
             if (rc) return rc;
         }
     }
+    // the peaks (and a small call's periodogram), then into the caller's arrays
+    auto fetch = [&](void *to, size_t at, size_t bytes) -> int {
+        if (to && !peaks_pinned) HIP_OK(hipMemcpyAsync(to, peaks + at, bytes, hipMemcpyDeviceToHost, c.stream));
+        return LSAMD_OK;
+    };
     if (tk) {
-        if (peak_index)
-            HIP_OK(hipMemcpyAsync(peak_index, c.pidx.p, (size_t)K * tk * 4, hipMemcpyDeviceToHost,
-                                  c.stream));
-        if (peak_power)
-            HIP_OK(hipMemcpyAsync(peak_power, c.ppow.p, (size_t)K * tk * rsz,
-                                  hipMemcpyDeviceToHost, c.stream));
-        if (peak_period)
-            HIP_OK(hipMemcpyAsync(peak_period, c.pper.p, (size_t)K * tk * rsz,
-                                  hipMemcpyDeviceToHost, c.stream));
+        rc = fetch(peak_index, out_idx, (size_t)K * tk * 4);
+        if (!rc) rc = fetch(peak_power, out_pow, (size_t)K * tk * rsz);
+        if (!rc) rc = fetch(peak_period, out_per, (size_t)K * tk * rsz);
+        if (rc) return rc;
     }
     HIP_OK(hipStreamSynchronize(c.stream));
+    if (tk && peaks_pinned) {
+        if (peak_index) host_copy(reinterpret_cast<char *>(peak_index), io_out + out_idx, (size_t)K * tk * 4);
+        if (peak_power) host_copy(static_cast<char *>(peak_power), io_out + out_pow, (size_t)K * tk * rsz);
+        if (peak_period) host_copy(static_cast<char *>(peak_period), io_out + out_per, (size_t)K * tk * rsz);
+    }
+    if (pgram && small) host_copy(static_cast<char *>(pgram), io_out + out_pg, (size_t)K * per_obj);
+    c.busy = false;
+    return LSAMD_OK;
+}
+
+// numpy.argmax along the rows of a rows x cols array.
+int lsamd_row_argmax(int dtype, const void *data, uint64_t rows, uint64_t cols, uint64_t *index) {
+    if (!data || !index || cols == 0 || (dtype != LSAMD_F32 && dtype != LSAMD_F64))
+        return set_error(LSAMD_ERR_INVALID, "lsamd_row_argmax: bad arguments");
+#pragma omp parallel for num_threads(8) schedule(static) if (rows > 1 && rows * cols > 100000)
+    for (long long r = 0; r < (long long)rows; ++r)
+        index[r] = dtype == LSAMD_F64 ? row_argmax(static_cast<const double *>(data) + (uint64_t)r * cols, cols)
+                                      : row_argmax(static_cast<const float *>(data) + (uint64_t)r * cols, cols);
     return LSAMD_OK;
 }
 

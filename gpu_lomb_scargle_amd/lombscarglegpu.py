@@ -150,7 +150,10 @@ def lombscarglemain(objId, timeX, magY, minFreq, maxFreq, error, mode, magDY=Non
     if isinstance(freqToTest, str) and freqToTest == "auto":
         freqToTest = computeNumFreqAuto(objId, timeX, minFreqStandard, maxFreqStandard)
 
-    numObjects = np.size(np.unique(objId))
+    start, end, uniqueIdsOrdered = computeIndexRangesForEachObject(objId)
+    # one run of equal ids is one object; several runs hold several ids, but for NaN ones
+    several = start.size > 1 and not (np.asarray(objId).dtype.kind == "f" and np.size(np.unique(objId)) == 1)
+    numObjects = 2 if several else min(start.size, 1)
     if mode == "GPU" and numObjects > 1:
         setmode = 1
     elif mode == "GPU" and numObjects == 1:
@@ -166,7 +169,6 @@ def lombscarglemain(objId, timeX, magY, minFreq, maxFreq, error, mode, magDY=Non
         print("[Python] Error: No input error array, but the error mode is True. Set error mode to False.")
         sys.exit(0)
 
-    start, end, uniqueIdsOrdered = computeIndexRangesForEachObject(objId)
     objId = enumerateObjects(start, end)
 
     if dtype not in ("float", "double"):
@@ -197,7 +199,7 @@ def lombscarglemain(objId, timeX, magY, minFreq, maxFreq, error, mode, magDY=Non
     c_magDY = convert_type(magDY, ctype)
 
     dfstandard = (maxFreqStandard - minFreqStandard) / freqToTest * 1.0
-    uniqueObjects = np.size(np.unique(objId))
+    uniqueObjects = start.size
     print("[Python] Unique objects: %d" % uniqueObjects)
     ret_pgram = np.zeros(uniqueObjects * freqToTest, dtype=ctype)
     print("[Python] Size of pgram in elems: %d (%f GiB)" %
@@ -212,9 +214,12 @@ def lombscarglemain(objId, timeX, magY, minFreq, maxFreq, error, mode, magDY=Non
         raise RuntimeError("LombScarglePy failed (%d): %s" % (rc, lib.lsamd_last_error().decode()))
 
     ret_pgram = ret_pgram.reshape([uniqueObjects, freqToTest])
+    best = np.zeros(uniqueObjects, dtype=np.uint64)
+    _native.check(lib, lib.lsamd_row_argmax(_native.F32 if dtype == "float" else _native.F64, ret_pgram.ctypes.data,
+                                            uniqueObjects, freqToTest, best.ctypes.data))
     ret_periods = np.zeros(uniqueObjects)
     for x in range(uniqueObjects):
-        ret_periods[x] = 1.0 / (minFreqStandard + (dfstandard * np.argmax(ret_pgram[x])))
+        ret_periods[x] = 1.0 / (minFreqStandard + (dfstandard * int(best[x])))
 
     if uniqueObjects > 1:
         print("[Python] Sum of all periods: %f" % np.sum(ret_periods))

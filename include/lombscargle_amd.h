@@ -261,6 +261,10 @@ int lsamd_cpu_single(int variant, int dtype, int normalize, const void *t, void 
                      const void *dy, uint64_t n, double min_freq, double max_freq,
                      uint32_t num_freqs, void *pgram, int nthreads);
 
+/* Best bin of every row of a rows x cols periodogram in host memory, as
+ * numpy.argmax has it: the first NaN of the row, else its first maximum. */
+int lsamd_row_argmax(int dtype, const void *data, uint64_t rows, uint64_t cols, uint64_t *index);
+
 /* Number of runs of equal ids (objects) in objectId[n]. */
 uint32_t lsamd_count_objects(const uint32_t *objectId, uint64_t n);
 /* Fill offsets[K+1] (row ranges) and ids[K] (may be NULL) of the runs. */
