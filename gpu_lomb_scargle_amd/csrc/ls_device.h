@@ -364,17 +364,31 @@ __device__ __forceinline__ void sincos_near(double x, double *so, double *co) {
     *co = __longlong_as_double(__double_as_longlong(c0) ^ cs);
 }
 
-// NEAR: |x| < kTrigFar (or not finite) is known.
+// NEAR: |x| < kTrigFar (or not finite) is known.  The device library's sincos
+// is called, not inlined: its reduction of large arguments holds ~100 registers,
+// which would cost every sweep its second and third wavefront per SIMD.
+struct SinCos {
+    double s, c;
+};
+__device__ __attribute__((noinline)) SinCos sincos_far(double x) {
+    SinCos r;
+    sincos(x, &r.s, &r.c);
+    return r;
+}
 template <bool NEAR, bool CARRIED>
 __device__ __forceinline__ void sincos_r(double x, double *s, double *c) {
-    if constexpr (NEAR) sincos_near<CARRIED>(x, s, c);
-    else sincos(x, s, c);
+    if constexpr (NEAR) {
+        sincos_near<CARRIED>(x, s, c);
+    } else {
+        const SinCos r = sincos_far(x);
+        *s = r.s;
+        *c = r.c;
+    }
 }
 template <bool NEAR, bool CARRIED>
 __device__ __forceinline__ void sincos_r(float x, float *s, float *c) {
     double sd, cd;
-    if constexpr (NEAR) sincos_near<false>((double)x, &sd, &cd);
-    else sincos((double)x, &sd, &cd);
+    sincos_r<NEAR, false>((double)x, &sd, &cd);
     *s = (float)sd;
     *c = (float)cd;
 }

@@ -15,7 +15,8 @@ namespace {
 // objects (17,200 observations) x 100,003 bins 7.47 -> 3.38 ms (5.1e11
 // terms/s); generalized (two sines and cosines per term) FP64, 3555
 // observations x 200,000 bins 9.0 -> 5.7 ms, FP32, 136 objects (7,200
-// observations) x 100,000 bins 7.1 -> 3.5 ms.
+// observations) x 100,000 bins 7.1 -> 3.5 ms.  The stepped FP64 sweeps below
+// form most of them from their neighbours'.
 //
 // A bound of |omega| over the bins below k_end, and whether omega t may leave
 // the range of sincos_near (2^30, half the range its reduction holds for, so
@@ -175,6 +176,13 @@ __device__ __forceinline__ double direct_std_power(const SweepArgs &a, uint64_t 
     return plain_std_power(omega, xc, xs, cc, ss, cs, scale);
 }
 
+// (c, s) turned by (ec, es), corrected by the rotation r.
+__device__ __forceinline__ void turn_step(double &c, double &s, double ec, double es, double r) {
+    const double rc = fma(-r, es, ec), rs = fma(r, ec, es), c0 = c;
+    c = fma(c, rc, -(s * rs));
+    s = fma(c0, rs, s * rc);
+}
+
 template <int T, int M>
 __global__ __launch_bounds__(T) void k_sweep_plain_step(SweepArgs a) {
 #pragma clang fp contract(off)
@@ -214,7 +222,7 @@ __global__ __launch_bounds__(T) void k_sweep_plain_step(SweepArgs a) {
                 const double t = gt[b0 + tid], d = step * t;
                 double s, c;
                 far = om_most * fabs(t) >= kStepFar;
-                sincos_near<true>(far ? 0.0 : d, &s, &c);
+                sincos_near<false>(far ? 0.0 : d, &s, &c);
                 s_ty[tid] = make_double2(t, gy[b0 + tid]);
                 s_step[tid] = make_double2(c, s);
                 s_d[tid] = d;
@@ -230,12 +238,6 @@ __global__ __launch_bounds__(T) void k_sweep_plain_step(SweepArgs a) {
                     cc[m] = fma(c, c, cc[m]);
                     cs[m] = fma(c, s, cs[m]);
                 };
-                // (c, s) turned by (ec, es), corrected by the rotation r
-                auto turn = [](double &c, double &s, double ec, double es, double r) {
-                    const double rc = fma(-r, es, ec), rs = fma(r, ec, es), c0 = c;
-                    c = fma(c, rc, -(s * rs));
-                    s = fma(c0, rs, s * rc);
-                };
                 const double xm = om[kMid] * ty.x;
                 double cm, sm;
                 sincos_near<false>(xm, &sm, &cm);
@@ -244,7 +246,7 @@ __global__ __launch_bounds__(T) void k_sweep_plain_step(SweepArgs a) {
 #pragma unroll
                 for (int m = kMid + 1; m < M; ++m) {
                     const double xn = om[m] * ty.x;
-                    turn(c, s, e.x, e.y, (xn - x) - d);
+                    turn_step(c, s, e.x, e.y, (xn - x) - d);
                     x = xn;
                     add(m, c, s);
                 }
@@ -254,7 +256,7 @@ __global__ __launch_bounds__(T) void k_sweep_plain_step(SweepArgs a) {
 #pragma unroll
                 for (int m = kMid - 1; m >= 0; --m) {
                     const double xn = om[m] * ty.x;
-                    turn(c, s, e.x, -e.y, (xn - x) + d);
+                    turn_step(c, s, e.x, -e.y, (xn - x) + d);
                     x = xn;
                     add(m, c, s);
                 }
@@ -271,6 +273,7 @@ __global__ __launch_bounds__(T) void k_sweep_plain_step(SweepArgs a) {
             const bool low = crosses || !(fabs(om[m]) >= step);
             if ((direct || ill || low) && k0 + 64u * (uint32_t)m < a.nf) flags |= 1u << m;
             P[m] = direct ? 0.0 : plain_std_power(om[m], xc[m], xs[m], cc[m], ss, cs[m], scale);
+            __builtin_amdgcn_sched_barrier(0);  // one bin's temporaries at a time
         }
         // bin m of all lanes at once, where a lane needs it
         for (int m = 0; m < M; ++m) {
@@ -298,11 +301,144 @@ __global__ __launch_bounds__(T) void k_sweep_plain_step(SweepArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// The generalized FP64 second pass, stepped.  Its phases fl(om_m fl(t - tau_m))
+// differ from bin to bin by D - (T_m - T_{m-1}), T_m = om_m tau_m, and by their
+// roundings, so with u_m = e^{i (x_m + T_m - T_mid)}
+//   u_m = u_{m-1} e^{i D} (1 + i r),  r = (x_m - x_{m-1}) - D + (T_m - T_{m-1}),
+// as in the standard sweep, every phase the reference's own; the sums are turned
+// back by T_m - T_mid at the end.  (The first pass keeps a sine and cosine per
+// phase: the roundings of t - tau hang on the last bit of tau.)  A wavefront
+// takes a quarter of the observations and all 256 bins of the workgroup, four per
+// lane: ~33 instructions per term instead of ~105.  The quarters' sums meet in
+// LDS, and thread tid ends with those of its bin.  3555 observations x 200,000
+// bins 5.61 -> 3.41 ms, 100 objects of 165 x 100,003 8.84 -> 5.53 (two wavefronts per SIMD;
+// unbounded it takes 266 registers and one, 4.3 and 8.1 ms, three spill, 3.6 and
+// 6.2).
+// ---------------------------------------------------------------------------
+template <typename R>
+struct TauSums {  // weighted sums of y, y y, c, s, y c, y s, c c, and s s
+    R Y, YY, C, S, YC, YS, CC, SS;
+};
+constexpr uint32_t kStepGenLeastObs = 32;
+
+// The sums at thread tid's bin, with c s in the place of s s, turned by T - T_mid;
+// false, and no sums, if a phase is past kStepFar.  tau: of that bin, finite.  All
+// threads of the workgroup call it.
+template <int T>
+__device__ __forceinline__ bool stepped_tau_sums(const double *gt, const double *gy, const double *gw, uint64_t beg,
+                                                 uint64_t end, double fmin_r, double fstep_r, uint32_t kbase,
+                                                 double tau, TauSums<double> &out) {
+#pragma clang fp contract(off)
+    static_assert(T == 256, "four wavefronts");
+    constexpr int M = T / 64, kMid = M / 2, NS = 6;
+    __shared__ double2 s_t[T], s_w[T], s_e[T];  // t, D; w, w y; cos D, sin D
+    __shared__ double s_yy[T];                  // w y y
+    __shared__ double s_tau[T], s_y[M][2];
+    double *const s_sum = reinterpret_cast<double *>(s_t);  // [M][T], when the observations are done with
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
+    const double step = 64.0 * fstep_r;
+    const double om_most = fmax(fabs(fmin_r + fstep_r * (double)kbase),
+                                fabs(fmin_r + fstep_r * ((double)kbase + (double)T)));
+    s_tau[tid] = tau;
+    __syncthreads();
+    double om[M], tm[M], dT[M], acc[NS][M], Y = 0.0, YY = 0.0;
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+        om[m] = fmin_r + (fstep_r * (double)(kbase + 64u * (uint32_t)m + lane));
+        tm[m] = s_tau[64 * m + (int)lane];
+        dT[m] = m == 0 ? 0.0 : om[m] * tm[m] - om[m - 1] * tm[m - 1];
+#pragma unroll
+        for (int q = 0; q < NS; ++q) acc[q][m] = 0.0;
+    }
+    for (uint64_t b0 = beg; b0 < end; b0 += T) {
+        const uint32_t cnt = (uint32_t)((end - b0) < (uint64_t)T ? (end - b0) : (uint64_t)T);
+        __syncthreads();
+        bool far = false;
+        if (tid < cnt) {
+            const double t = gt[b0 + tid], w = gw[b0 + tid], d = step * t;
+            double s, c;
+            far = om_most * fabs(t) >= kStepFar;
+            sincos_near<false>(far ? 0.0 : d, &s, &c);
+            s_t[tid] = make_double2(t, d);
+            const double y = gy[b0 + tid], wy = w * y;
+            s_w[tid] = make_double2(w, wy);
+            s_yy[tid] = wy * y;
+            s_e[tid] = make_double2(c, s);
+        }
+        if (__syncthreads_or(far)) return false;
+        for (uint32_t j = wave; j < cnt; j += M) {
+            const double2 td = s_t[j], ww = s_w[j], e = s_e[j];
+            Y += ww.y;
+            YY += s_yy[j];
+            auto add = [&](int m, double c, double s) {
+                const double wc = ww.x * c;
+                acc[0][m] += wc;
+                acc[1][m] = fma(ww.x, s, acc[1][m]);
+                acc[2][m] = fma(ww.y, c, acc[2][m]);
+                acc[3][m] = fma(ww.y, s, acc[3][m]);
+                acc[4][m] = fma(wc, c, acc[4][m]);
+                acc[5][m] = fma(wc, s, acc[5][m]);
+            };
+            const double xm = om[kMid] * (td.x - tm[kMid]);
+            double cm, sm;
+            sincos_near<false>(xm, &sm, &cm);
+            add(kMid, cm, sm);
+            double c = cm, s = sm, x = xm;
+#pragma unroll
+            for (int m = kMid + 1; m < M; ++m) {
+                const double xn = om[m] * (td.x - tm[m]);
+                turn_step(c, s, e.x, e.y, ((xn - x) - td.y) + dT[m]);
+                x = xn;
+                add(m, c, s);
+            }
+            c = cm;
+            s = sm;
+            x = xm;
+#pragma unroll
+            for (int m = kMid - 1; m >= 0; --m) {
+                const double xn = om[m] * (td.x - tm[m]);
+                turn_step(c, s, e.x, -e.y, ((xn - x) + td.y) - dT[m + 1]);
+                x = xn;
+                add(m, c, s);
+            }
+        }
+    }
+    double sum[NS];
+    if (lane == 0) {
+        s_y[wave][0] = Y;
+        s_y[wave][1] = YY;
+    }
+#pragma unroll
+    for (int q = 0; q < NS; ++q) {
+        __syncthreads();
+#pragma unroll
+        for (int m = 0; m < M; ++m) s_sum[wave * T + 64u * (uint32_t)m + lane] = acc[q][m];
+        __syncthreads();
+        sum[q] = 0.0;
+#pragma unroll
+        for (int w = 0; w < M; ++w) sum[q] += s_sum[(uint32_t)w * T + tid];
+    }
+    out.Y = out.YY = 0.0;
+#pragma unroll
+    for (int w = 0; w < M; ++w) {
+        out.Y += s_y[w][0];
+        out.YY += s_y[w][1];
+    }
+    out.C = sum[0];
+    out.S = sum[1];
+    out.YC = sum[2];
+    out.YS = sum[3];
+    out.CC = sum[4];
+    out.SS = sum[5];
+    return true;
+}
+
+// ---------------------------------------------------------------------------
 // Plain form, generalized variant: two passes, tau then the tau-shifted sums
 // (lombscarglecpuinnerloopAstroPy, main.cu:1701-1777).
 // ---------------------------------------------------------------------------
 template <typename R, int T, int M>
-__global__ __launch_bounds__(T) void k_sweep_plain_gen(SweepArgs a) {
+__global__ __launch_bounds__(T, 2) void k_sweep_plain_gen(SweepArgs a) {
 #pragma clang fp contract(off)
     __shared__ R s_t[T], s_y[T], s_w[T];
     __shared__ double s_pp[T / 64][kPeaks];
@@ -365,41 +501,80 @@ __global__ __launch_bounds__(T) void k_sweep_plain_gen(SweepArgs a) {
             C2[m] -= (C[m] * C[m] - S[m] * S[m]);
             tau[m] = (R)(0.5 * (double)atan2_r(S2[m], C2[m]) / (double)om[m]);
         }
-        // pass 2: the tau-shifted sums
-        R Y[M], YY[M], Ct[M], St[M], YC[M], YS[M], CC[M], SS[M];
-    #pragma unroll
-        for (int m = 0; m < M; ++m) Y[m] = YY[m] = Ct[m] = St[m] = YC[m] = YS[m] = CC[m] = SS[m] = (R)0;
-        for (uint64_t b0 = beg; b0 < end; b0 += T) {
-            const uint32_t cnt = (uint32_t)((end - b0) < (uint64_t)T ? (end - b0) : (uint64_t)T);
-            __syncthreads();
-            bool far = false;
-            if (tid < cnt) {
-                const R t = gt[b0 + tid];
-                s_t[tid] = t;
-                s_y[tid] = gy[b0 + tid];
-                s_w[tid] = gw[b0 + tid];
-                far = far_phase(om_most, (double)t);
+        // pass 2: the tau-shifted sums.  FP64: stepped, but for objects of few
+        // observations, chunks that reach below the step (see
+        // k_sweep_plain_step), bins that amplify the steps' error (ccv ssv below
+        // 1 / (4 kStepCond)) and a tau that is not finite.
+        TauSums<R> q[M];
+        bool again = true;  // this thread's sums are still to be formed, phase by phase
+        if constexpr (std::is_same_v<R, double>) {
+            static_assert(M == 1, "a bin per thread");
+            const double tf = __builtin_isfinite(tau[0]) ? tau[0] : 0.0;
+            TauSums<double> u;
+            const double least = 64.0 * fstep, lo = fmin + fstep * (double)kbase, hi = lo + fstep * (double)(T - 1);
+            const bool apart = ::fmin(fabs(lo), fabs(hi)) >= least && (lo < 0.0) == (hi < 0.0);
+            if (apart && end - beg >= (uint64_t)kStepGenLeastObs &&
+                stepped_tau_sums<T>(gt, gy, gw, beg, end, fmin, fstep, kbase, tf, u)) {
+                s_t[tid] = om[0] * tf;
+                __syncthreads();
+                double sa, ca;
+                sincos_near<true>(s_t[tid] - s_t[128u + (tid & 63u)], &sa, &ca);
+                const double ss = wsum[0] - u.CC, w2 = 2.0 * ca * sa;
+                q[0].Y = u.Y;
+                q[0].YY = u.YY;
+                q[0].C = fma(u.C, ca, u.S * sa);
+                q[0].S = fma(u.S, ca, -(u.C * sa));
+                q[0].YC = fma(u.YC, ca, u.YS * sa);
+                q[0].YS = fma(u.YS, ca, -(u.YC * sa));
+                q[0].CC = fma(ca * ca, u.CC, fma(w2, u.SS, sa * sa * ss));  // (u.SS: the sum of c s)
+                q[0].SS = fma(ca * ca, ss, fma(-w2, u.SS, sa * sa * u.CC));
+                const double ct = q[0].C / wsum[0], st = q[0].S / wsum[0];
+                const double ccv = q[0].CC / wsum[0] - ct * ct, ssv = q[0].SS / wsum[0] - st * st;
+                again = tf != tau[0] || !(ccv * ssv * (4.0 * kStepCond) >= 1.0);
             }
-            auto sums = [&](auto near) {
-                for (uint32_t j = 0; j < cnt; ++j) {
-                    const R tj = s_t[j], yj = s_y[j], w = s_w[j];
+        }
+        if (__syncthreads_or(again)) {
+            TauSums<R> d[M];
     #pragma unroll
-                    for (int m = 0; m < M; ++m) {
-                        R s, c;  // |omega tau| <= pi/4 beside omega t
-                        sincos_r<decltype(near)::value, true>(om[m] * (tj - tau[m]), &s, &c);
-                        Y[m] += w * yj;
-                        YY[m] += w * yj * yj;
-                        Ct[m] += w * c;
-                        St[m] += w * s;
-                        YC[m] += w * yj * c;
-                        YS[m] += w * yj * s;
-                        CC[m] += w * c * c;
-                        SS[m] += w * s * s;
-                    }
+            for (int m = 0; m < M; ++m) d[m] = TauSums<R>{};
+            const bool wave_any = __ballot(again) != 0u;
+            for (uint64_t b0 = beg; b0 < end; b0 += T) {
+                const uint32_t cnt = (uint32_t)((end - b0) < (uint64_t)T ? (end - b0) : (uint64_t)T);
+                __syncthreads();
+                bool far = false;
+                if (tid < cnt) {
+                    const R t = gt[b0 + tid];
+                    s_t[tid] = t;
+                    s_y[tid] = gy[b0 + tid];
+                    s_w[tid] = gw[b0 + tid];
+                    far = far_phase(om_most, (double)t);
                 }
-            };
-            if (__syncthreads_or(far)) sums(std::false_type{});
-            else sums(std::true_type{});
+                auto sums = [&](auto near) {
+                    for (uint32_t j = 0; j < cnt; ++j) {
+                        const R tj = s_t[j], yj = s_y[j], w = s_w[j];
+    #pragma unroll
+                        for (int m = 0; m < M; ++m) {
+                            R s, c;  // |omega tau| <= pi/4 beside omega t
+                            sincos_r<decltype(near)::value, true>(om[m] * (tj - tau[m]), &s, &c);
+                            d[m].Y += w * yj;
+                            d[m].YY += w * yj * yj;
+                            d[m].C += w * c;
+                            d[m].S += w * s;
+                            d[m].YC += w * yj * c;
+                            d[m].YS += w * yj * s;
+                            d[m].CC += w * c * c;
+                            d[m].SS += w * s * s;
+                        }
+                    }
+                };
+                const bool some_far = __syncthreads_or(far) != 0;
+                if (!wave_any) continue;
+                if (some_far) sums(std::false_type{});
+                else sums(std::true_type{});
+            }
+    #pragma unroll
+            for (int m = 0; m < M; ++m)
+                if (again) q[m] = d[m];
         }
         R *pg = static_cast<R *>(a.pgram);
         Peaks L;
@@ -408,8 +583,8 @@ __global__ __launch_bounds__(T) void k_sweep_plain_gen(SweepArgs a) {
         for (int m = 0; m < M; ++m) {
             const uint32_t kf = kbase + m * T + tid;
             const R ws = wsum[m];
-            R y_ = Y[m] / ws, yy = YY[m] / ws, ct = Ct[m] / ws, st = St[m] / ws;
-            R yc = YC[m] / ws, ys = YS[m] / ws, ccv = CC[m] / ws, ssv = SS[m] / ws;
+            R y_ = q[m].Y / ws, yy = q[m].YY / ws, ct = q[m].C / ws, st = q[m].S / ws;
+            R yc = q[m].YC / ws, ys = q[m].YS / ws, ccv = q[m].CC / ws, ssv = q[m].SS / ws;
             yc -= y_ * ct;
             ys -= y_ * st;
             ccv -= ct * ct;

@@ -91,3 +91,33 @@ def test_parts_of_a_host_call(monkeypatch):
     monkeypatch.setenv("LSAMD_SLICE_BYTES", str(2 * 20011 * 8))
     parts = _native.batch_host(*args)
     assert np.array_equal(whole["pgram"], parts["pgram"]) and np.array_equal(whole["index"], parts["index"])
+
+
+@pytest.mark.parametrize("t0,lo,hi", [(0.0, synth.OMEGA_MIN, synth.OMEGA_MAX), (51075.0, 0.63, 62.8), (0.0, 0.3, 60.0),
+                                      (0.0, -60.0, -1.0)])
+def test_generalized_against_the_oracle(t0, lo, hi):
+    """The second pass of the generalized sweep, stepped from 32 observations on,
+    around the staged blocks.  A last-bit difference of tau moves the rounding of
+    t - tau (test_gpu_plain_phase_range.py): 1e-9 on bins of at least 1e-3 Pmax."""
+    counts = [5, 31, 32, 33, 64, 255, 256, 257, 700]
+    o, t, y = _curves(counts, t0=t0)
+    dy = np.random.default_rng(6).uniform(0.05, 0.3, len(t))
+    r = _native.batch_host(o, t, 17.0 + y, dy, lo, hi, 5003, _native.GENERALIZED, F64, _native.FORM_PLAIN)
+    ref = oracle.batch(o, t, 17.0 + y, dy, lo, hi, 5003, True, F64, nthreads=8)[0]
+    assert np.array_equal(np.isnan(r["pgram"]), np.isnan(ref))
+    assert_close(r["pgram"], ref, 1e-9, 1e-3, 1e-9)
+
+
+def test_generalized_grid_over_zero():
+    """tau is 0/0 at frequency 0: NaN there and nowhere else; a NaN time gives an
+    object of NaN.  (5003 bins from -20 to 30, and from 0.)"""
+    o, t, y = _curves([40, 300, 300])
+    dy = np.random.default_rng(6).uniform(0.05, 0.3, len(t))
+    t[400] = np.nan
+    for lo, hi in ((0.0, 30.0), (-20.0, 30.02)):
+        r = _native.batch_host(o, t, y.copy(), dy, lo, hi, 5003, _native.GENERALIZED, F64, _native.FORM_PLAIN)["pgram"]
+        ref = oracle.batch(o, t, y.copy(), dy, lo, hi, 5003, True, F64, nthreads=8)[0]
+        assert np.array_equal(np.isnan(r), np.isnan(ref))
+        far = np.abs(lo + (hi - lo) / 5003 * np.arange(5003)) > 0.1
+        for k in (0, 1):  # (object 2 holds the NaN)
+            assert_close(r[k][far], ref[k][far], 1e-9, 1e-3, 1e-9)
