@@ -43,6 +43,8 @@ __host__ __device__ constexpr double ip_beta(bool screen) {
 }
 constexpr uint32_t kIpLeastBins = 255 * 32, kIpLeastBinsScreen = 192 * 30;  // bins per workgroup, smallest mode
 constexpr uint32_t kIpGroup = 4;  // consecutive items of an object per workgroup, at most
+// The generalized sums' workgroups take one (the loop costs them 4%).
+__host__ __device__ constexpr bool ip_grouped(bool screen, bool gen) { return screen || !gen; }
 // Objects up to here keep the direct sums, those of at most 16 observations
 // their FP64 ones: with 18 observations and weights over a factor of 400 the
 // worst bin reached 1.4e-5 (direct 1.0e-5).  Peaks alone, generalized: with

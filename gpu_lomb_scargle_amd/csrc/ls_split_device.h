@@ -368,7 +368,8 @@ __device__ __forceinline__ void load_cols(const uint4 *cf, half8_t (&col)[NF]) {
 // objects).  The others take the groups of the objects in direct mode, in the
 // grid schedule's order; the launch has a workgroup for every group that there
 // could be, and those past the list's end, which only the device knows, leave
-// at once.  (In their place, where all objects are direct, 4000 x 100,000 bins,
+// at once; or, with a queue, as many workgroups as fill the chip drain it.  (In
+// the grid's place, where all objects are direct, standard, 4000 x 100,000 bins,
 // 4.53 ms with the plain grid: workgroups that stay on the chip and stride over
 // the groups 5.9, the persistent queues 4.9, groups of eight items 4.8.)
 __device__ __forceinline__ uint64_t cand_item(const SweepArgs &a, uint32_t obj, uint32_t from, uint32_t skip) {
@@ -387,6 +388,7 @@ __device__ __forceinline__ uint64_t direct_first(SweepArgs &a, uint64_t *s_item)
         a.cand = nullptr;
         a.order = a.direct_list;
         a.total_items = (uint64_t)*a.direct_count * a.chunks;
+        if (a.queue) return fetch_item(a, s_item, true);
         const uint64_t groups = (a.total_items + a.group - 1u) / a.group, w = a.item_base + blockIdx.x - a.marked_groups;
         if (w >= groups) return ~0ull;
         a.item_base = 0;
@@ -397,6 +399,7 @@ __device__ __forceinline__ uint64_t direct_first(SweepArgs &a, uint64_t *s_item)
     if (pos >= a.K) return ~0ull;
     const uint32_t obj = a.order ? a.order[pos] : pos;
     a.order = nullptr;  // the items name the object itself
+    a.queue = nullptr;
     return a.obj_ip[obj].mode ? cand_item(a, obj, 0u, r) : ~0ull;
 }
 __device__ __forceinline__ uint64_t direct_next(const SweepArgs &a, uint64_t *s_item, uint64_t item) {

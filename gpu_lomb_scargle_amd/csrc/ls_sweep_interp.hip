@@ -17,8 +17,8 @@
 //
 // FP32 periodograms, measured (top-1, ms of the whole sweep, direct -> coarse):
 // 1000 objects (164,000 observations) x 10^6 bins, standard, 23 bins per
-// resolution element, h = 10: 10.5 -> 2.84; 250 objects (42,700) x 429,119,
-// generalized, ten bins, h = 4: 2.0 -> 0.68.  k_sweep_interp takes 2.6 ms of
+// resolution element, h = 10: 10.5 -> 2.75; 250 objects (42,700) x 429,119,
+// generalized, ten bins, h = 4: 2.0 -> 0.68.  k_sweep_interp takes 2.55 ms of
 // the first: a third the coarse points, the rest the interpolation and the
 // FP64 powers (22 FP64 instructions per bin; VALU 58% and matrix cores 16% of
 // the SIMD cycles at 2.0 GHz), the stores 0.2 and the bins past the condition
@@ -33,9 +33,9 @@
 // (17 observations of uneven weight), 1e-3 typically, against a margin of
 // 1/8.  The results are the direct sums', bit for bit.  Measured: 8000 uneven
 // objects x 200,000 bins, top-3, standard FP64, 4.7 bins per resolution
-// element, h = 3: 13.1 -> 5.2 ms (screen 3.1, the marked chunks and the objects
-// of at most 16 observations 1.6, tables 0.45); 1000 objects x 500,000,
-// generalized, 10.5 bins, h = 8: 11.2 -> 1.4 ms.
+// element, h = 3: 13.1 -> 4.8 ms (screen 3.0, the marked chunks and the objects
+// of at most 16 observations 1.45, tables 0.35); 1000 objects x 500,000,
+// generalized, 10.5 bins, h = 8: 11.2 -> 1.2 ms.
 #include <type_traits>
 
 #include "ls_split_device.h"
@@ -132,6 +132,7 @@ __device__ void list_direct(const SweepArgs &a) {
         }
     }
     if (lane == 0) *a.direct_count = count;
+    if (lane < kQueues) a.queue[lane * kQueueStride] = 0ull;
 }
 
 // The first workgroups list the objects in direct mode (blockIdx.x = 0) and
@@ -356,8 +357,8 @@ __global__ __launch_bounds__(256, SCREEN ? 3 : 2) void k_sweep_interp(SweepArgs 
     const R rsw = uniform((R)sw), rhsw = uniform((R)hsw), rybu = uniform((R)ybu), rkg = uniform((R)kg);
     const R rhn = uniform((R)hn), rhn2 = uniform((R)hn2), rdmin = uniform((R)dmin), rkp = uniform((R)kp);
     const R rcond = (R)kCondMax;
-    // screen: a.group workgroups' worths of bins in turn, the object's constants
-    // and addresses stay (its workgroups are short)
+    // a.group workgroups' worths of bins in turn (ip_grouped), the object's
+    // constants and addresses stay
     auto sweep_item = [&](const uint32_t it, const uint32_t l) {
     const uint32_t rc = l & 31u, kh = l >> 5;
     const uint32_t kbase = it * (rows * rb);
@@ -626,8 +627,9 @@ __global__ __launch_bounds__(256, SCREEN ? 3 : 2) void k_sweep_interp(SweepArgs 
         }
     }
     };
-    if constexpr (SCREEN) {
+    if constexpr (ip_grouped(SCREEN, GEN)) {
         for (uint32_t it = it0; it < it0 + a.group && (uint64_t)it * (rows * rb) < a.nf; ++it) {
+            if (!SCREEN && it != it0) __syncthreads();  // the last tiles' points are read
             uint32_t lane = l;  // opaque: nothing derived from it is worth registers across items
             asm volatile("" : "+v"(lane));
             sweep_item(it, lane);
