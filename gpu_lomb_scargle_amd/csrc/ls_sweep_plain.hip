@@ -138,9 +138,10 @@ __global__ __launch_bounds__(T) void k_sweep_plain_std(SweepArgs a) {
 // amplifies the phasors' error (condition number above kStepCond), frequencies
 // below the step (or of both signs in a thread), phases past kStepFar, objects of fewer than
 // kStepLeastObs observations, most of whose bins are ill-conditioned.
-// 100 objects (17,200 observations) x 100,003 bins: 3.38 -> 1.31 ms (M = 8, 132 registers)
-// and 1.06 (M = 16); M = 6, 10, 12 lay between, four wavefronts per SIMD of M = 8
-// spill (2.8 ms).
+// 100 objects (17,200 observations) x 100,003 bins: 3.38 -> 1.31 ms (M = 8) and
+// 0.96 (M = 16, two wavefronts per SIMD by 18 spilled registers, mostly outside
+// the loop; 1.06 with one and none).  M = 10, 12 and 14 lie between (1.03, 1.14 and
+// 1.07 where M = 16 has 0.98), four wavefronts of M = 8 spill to 2.8 ms.
 // ---------------------------------------------------------------------------
 constexpr double kStepFar = 268435456.0;  // 2^28
 constexpr double kStepCond = 16.0;
@@ -184,7 +185,7 @@ __device__ __forceinline__ void turn_step(double &c, double &s, double ec, doubl
 }
 
 template <int T, int M>
-__global__ __launch_bounds__(T) void k_sweep_plain_step(SweepArgs a) {
+__global__ __launch_bounds__(T, 2) void k_sweep_plain_step(SweepArgs a) {
 #pragma clang fp contract(off)
     __shared__ double2 s_ty[T], s_step[T];  // t, y; cos D, sin D
     __shared__ double s_d[T];               // D
