@@ -12,8 +12,10 @@
 // share a hardware queue, where a copy waits for every sweep enqueued before it.
 // Larger outputs go through device memory and staging buffers as before.
 // Whole call, us: one star of 29 observations, 1188 bins, 204 -> 99; 136 stars
-// x 100,000 bins, generalized FP32 (54 MB), 7678 -> 4840 (the sweep alone 3530; with
-// slices copied on a second stream 5400, or 8700 beside another library).
+// x 100,000 bins, generalized FP32 (54 MB), 7678 -> 4770 (the sweep alone 2750 into device
+// memory, ~3800 into pinned memory, coherent or not, where a copy kernel after it
+// would take the difference; with slices copied on a second stream 5400, or 8700
+// beside another library).
 //
 // Replaces the reference's GPU host path: computeObjectRanges
 // (source/main.cu:468-510), computeNumBatches (main.cu:423-466),
