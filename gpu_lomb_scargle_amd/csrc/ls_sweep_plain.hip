@@ -332,10 +332,14 @@ __device__ __forceinline__ bool stepped_tau_sums(const double *gt, const double 
 #pragma clang fp contract(off)
     static_assert(T == 256, "four wavefronts");
     constexpr int M = T / 64, kMid = M / 2, NS = 6;
-    __shared__ double2 s_t[T], s_w[T], s_e[T];  // t, D; w, w y; cos D, sin D
-    __shared__ double s_yy[T];                  // w y y
+    // the staged observations, and when they are done with a sum of every
+    // wavefront and bin, [M][T]
+    __shared__ double2 s_obs[3][T];
+    double2 *const s_t = s_obs[0], *const s_w = s_obs[1], *const s_e = s_obs[2];  // t, D; w, w y; cos D, sin D
+    double *const s_sum = reinterpret_cast<double *>(s_obs);
+    static_assert(sizeof(s_obs) >= M * T * sizeof(double), "s_sum lies within s_obs");
+    __shared__ double s_yy[T];  // w y y
     __shared__ double s_tau[T], s_y[M][2];
-    double *const s_sum = reinterpret_cast<double *>(s_t);  // [M][T], when the observations are done with
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const double step = 64.0 * fstep_r;
     const double om_most = fmax(fabs(fmin_r + fstep_r * (double)kbase),
