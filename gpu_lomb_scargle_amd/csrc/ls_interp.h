@@ -38,6 +38,26 @@ __host__ __device__ constexpr int ip_rows(int mode) {
     return mode == 1 ? 192 : mode == 2 ? 255 : mode == 3 ? 320 : mode == 4 ? 408 : mode == 5 ? 510 : mode == 6 ? 672 : 1020;
 }
 __host__ __device__ constexpr int ip_taps(bool screen) { return screen ? 6 : 8; }
+// Points in LDS of a sum at f and of the sum at 2 f, the zeros behind the last ones included.
+constexpr uint32_t kIpPoints = 2048 + 32, kIpPoints2 = 4096 + 32;
+// Result row whose points lane row rc of tile t reads: its own, or the last one
+// (rows are no multiple of 32 in every mode; the results of those past it are dropped).
+__host__ __device__ constexpr uint32_t ip_operand_row(uint32_t rows, uint32_t t, uint32_t rc) {
+    const uint32_t s = 32u * t + rc;
+    return s < rows ? s : rows - 1u;
+}
+// A row's window at 2 f reaches past 16 points.
+__host__ __device__ constexpr bool ip_wide(bool screen, int mode) { return 2 * ip_per_row(mode) - 1 + ip_taps(screen) > 16; }
+constexpr bool ip_reads_fit() {
+    for (int screen = 0; screen < 2; ++screen)
+        for (int mode = 1; mode <= kIpModes; ++mode) {
+            const uint32_t m = (uint32_t)ip_per_row(mode), rows = (uint32_t)ip_rows(mode);
+            const uint32_t last = ip_operand_row(rows, (rows - 1) / 32, 31);
+            if (m * last + 16u > kIpPoints || 2u * m * last + (ip_wide(screen, mode) ? 32u : 16u) > kIpPoints2) return false;
+        }
+    return true;
+}
+static_assert(ip_reads_fit(), "operand reads stay within the points");
 __host__ __device__ constexpr double ip_beta(bool screen) {
     return 3.14159265358979323846 * ip_taps(screen) * (1.0 - 1.0 / (2.0 * (screen ? kIpSigmaScreen : kIpSigma)));
 }

@@ -311,7 +311,7 @@ __global__ __launch_bounds__(256, SCREEN ? 3 : 2) void k_sweep_interp(SweepArgs 
     constexpr int NC = SCREEN ? 1 : 2, FR = ip_frags(SCREEN);
     constexpr int NW = 4, NZ = GEN ? 2 : 1;
     constexpr uint32_t kFoldObs = 256;
-    constexpr int kZ = 2048 + 32, kX = 4096 + 32;  // points and zeros read past them
+    constexpr int kZ = (int)kIpPoints, kX = (int)kIpPoints2;
     __shared__ float2 s_u0[NW][64];
     __shared__ __align__(16) _Float16 s_z[NZ][2][NC][kZ];  // [sum][re, im][head, tail]
     __shared__ __align__(16) _Float16 s_x[2][NC][kX];
@@ -335,7 +335,7 @@ __global__ __launch_bounds__(256, SCREEN ? 3 : 2) void k_sweep_interp(SweepArgs 
     // |G| <= n max(1/Phi) 2^10 < n 2^12: into FP16's range
     const float gs = ldexpf(1.0f, 3 - (32 - __clz((int)n)));
     const bool at2f = wave >= (uint32_t)NZ;
-    const bool wide = 2u * m - 1u + (uint32_t)W > 16u;
+    const bool wide = ip_wide(SCREEN, mode);
     const double un = 1.0 / ((double)kFacScale * 1024.0 * (double)gs);  // power of two
     const double uy = un / (double)ys, uw = un / (double)ws;
     const double scale = a.obj_scale[obj];
@@ -506,7 +506,7 @@ __global__ __launch_bounds__(256, SCREEN ? 3 : 2) void k_sweep_interp(SweepArgs 
     const auto out = __builtin_amdgcn_make_buffer_rsrc(pg, 0, (int)(bin_end * 4u), 0x00027000);
 
     for (uint32_t tile = wave; 32u * tile < rows_here; tile += NW) {
-        const uint32_t s = 32u * tile + rc;  // this lane's row of the A operand
+        const uint32_t s = ip_operand_row(rows, tile, rc);  // this lane's row of the A operand
         f32x16_t z[2 * NZ], x[2];
         auto product = [&](const _Float16 *gh, const _Float16 *gt, const half8_t &th, const half8_t &tt, f32x16_t &acc) {
             half8_t ah, at;
