@@ -61,6 +61,14 @@ static_assert(ip_reads_fit(), "operand reads stay within the points");
 __host__ __device__ constexpr double ip_beta(bool screen) {
     return 3.14159265358979323846 * ip_taps(screen) * (1.0 - 1.0 / (2.0 * (screen ? kIpSigmaScreen : kIpSigma)));
 }
+// Largest 1/Phi at the ends of the span (ip_inv_window), rounded up: 2.95 and 9.94.
+__host__ __device__ constexpr double ip_window_most(bool screen) { return screen ? 10.0 : 3.0; }
+// The points' scale is 2^ip_point_shift / 2^bits, n < 2^bits: with the factors'
+// 2^10 and n observations in phase, at most 1 each, they end below FP16's 65504.
+__host__ __device__ constexpr int ip_point_shift(bool screen) { return screen ? 2 : 3; }
+static_assert(ip_window_most(false) * (1024 << ip_point_shift(false)) < 65504.0 &&
+                  ip_window_most(true) * (1024 << ip_point_shift(true)) < 65504.0,
+              "points within FP16's range");
 constexpr uint32_t kIpLeastBins = 255 * 32, kIpLeastBinsScreen = 192 * 30;  // bins per workgroup, smallest mode
 constexpr uint32_t kIpGroup = 4;  // consecutive items of an object per workgroup, at most
 // The generalized sums' workgroups take one (the loop costs them 4%).

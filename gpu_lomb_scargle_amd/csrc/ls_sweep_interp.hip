@@ -332,8 +332,8 @@ __global__ __launch_bounds__(256, SCREEN ? 3 : 2) void k_sweep_interp(SweepArgs 
     const uint64_t obeg = a.offsets[obj], oend = a.offsets[obj + 1];
     const uint32_t n = (uint32_t)(oend - obeg);
     const float ys = a.obj_ys[2 * obj], ws = a.obj_ys[2 * obj + 1];
-    // |G| <= n max(1/Phi) 2^10 < n 2^12: into FP16's range
-    const float gs = ldexpf(1.0f, 3 - (32 - __clz((int)n)));
+    // |G| <= n max(1/Phi) 2^10 into FP16's range
+    const float gs = ldexpf(1.0f, ip_point_shift(SCREEN) - (32 - __clz((int)n)));
     const bool at2f = wave >= (uint32_t)NZ;
     const bool wide = ip_wide(SCREEN, mode);
     const double un = 1.0 / ((double)kFacScale * 1024.0 * (double)gs);  // power of two
