@@ -109,6 +109,19 @@ __device__ __forceinline__ double ip_inv_window(bool screen, double xi) {
     return s / beta * exp(beta - s);
 }
 
+// Scale of the points of an object of n observations.
+__device__ __forceinline__ float ip_point_scale(bool screen, uint32_t n) {
+    return ldexpf(1.0f, ip_point_shift(screen) - (32 - __clz((int)n)));
+}
+// Unit of the screen's standard powers before the object's scale: the screen
+// only ranks an object's bins, and powers in this unit are of one order for
+// every unit of y (in FP32 the powers themselves leave the range for |y| below
+// 1e-20 or above 1e18).  A power of two.
+__device__ __forceinline__ double ip_rank_unit(double ys, double ws, uint32_t n) {
+    const double un = 1.0 / (1024.0 * 1024.0 * (double)ip_point_scale(true, n));
+    return un / ys * (ws / ys);
+}
+
 }  // namespace
 
 // Kernels of the coarse-grid sweep, [screen][variant][dtype] (sums: FP32 only).

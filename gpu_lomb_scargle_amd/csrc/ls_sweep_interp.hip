@@ -333,7 +333,7 @@ __global__ __launch_bounds__(256, SCREEN ? 3 : 2) void k_sweep_interp(SweepArgs 
     const uint32_t n = (uint32_t)(oend - obeg);
     const float ys = a.obj_ys[2 * obj], ws = a.obj_ys[2 * obj + 1];
     // |G| <= n max(1/Phi) 2^10 into FP16's range
-    const float gs = ldexpf(1.0f, ip_point_shift(SCREEN) - (32 - __clz((int)n)));
+    const float gs = ip_point_scale(SCREEN, n);
     const bool at2f = wave >= (uint32_t)NZ;
     const bool wide = ip_wide(SCREEN, mode);
     const double un = 1.0 / ((double)kFacScale * 1024.0 * (double)gs);  // power of two
@@ -342,9 +342,11 @@ __global__ __launch_bounds__(256, SCREEN ? 3 : 2) void k_sweep_interp(SweepArgs 
     // The powers from the unscaled results.  Standard, with c + i s = X / 2 and
     // CC = N/2 + c, SS = N/2 - c, CS = s:
     //   P = (N/2 |Z|^2 - c Re Z^2 - s Im Z^2) / (2 (N^2/4 - c^2 - s^2)),
-    // all in units of X's result (u = uw / 2): N/2 = hn u, P scaled by kp.
+    // all in units of X's result (u = uw / 2): N/2 = hn u, P scaled by kp (the
+    // screen's ranks: in units of ip_rank_unit = uy^2 / (2 u)).
     const double nobs = (double)n, u = 0.5 * uw, hn = 0.5 * nobs / u, hn2 = hn * hn;
-    const double dmin = nobs * nobs / (4.0 * kCondMax) / (u * u), kp = 0.5 * uy * uy / u * scale;
+    const double dmin = nobs * nobs / (4.0 * kCondMax) / (u * u), kp = SCREEN ? 1.0 : 0.5 * uy * uy / u * scale;
+    const double ke = SCREEN && !GEN ? 1.0 / ip_rank_unit((double)ys, (double)ws, n) : scale;  // of the powers computed again
     double Wf = 1.0, Yb = 0.0, YY = 1.0;
     if constexpr (GEN) {
         Wf = a.obj_gen[kGen * obj + 5];
@@ -558,7 +560,8 @@ __global__ __launch_bounds__(256, SCREEN ? 3 : 2) void k_sweep_interp(SweepArgs 
                 D = fm(-c, c, fm(-sn, sn, rhn2));
                 ill = !(D >= rdmin);
                 const R q = XC * XC;
-                num = rkp * fm(rhn, fm(XS, XS, q), -fm(c, fm(-XS, XS, q), (sn + sn) * (XC * XS)));
+                num = fm(rhn, fm(XS, XS, q), -fm(c, fm(-XS, XS, q), (sn + sn) * (XC * XS)));
+                if constexpr (!SCREEN) num *= rkp;
             }
             if constexpr (SCREEN) return num * __builtin_amdgcn_rcpf(D);
             else {
@@ -605,7 +608,7 @@ __global__ __launch_bounds__(256, SCREEN ? 3 : 2) void k_sweep_interp(SweepArgs 
             const uint32_t kf = kbase + rb * (32u * tile + 4u * (src >> 5) + 8u * (v / 4u) + v % 4u) + (src & 31u);
             const double pe = exact_power<GEN, IN>(a, obj, kf);
             if (l == src) {
-                const float pw = (float)(pe * scale);
+                const float pw = (float)(pe * ke);
                 if constexpr (!SCREEN) pg[kf] = pw;
                 best = fmaxf(best, pw);
                 flags &= flags - 1u;

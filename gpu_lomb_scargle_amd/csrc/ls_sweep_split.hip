@@ -657,9 +657,12 @@ __global__ __launch_bounds__(T) void k_sweep_split64(SweepArgs a) {
 // overlap a result tile whose best power reaches the top_k-th best of the
 // tiles' lane maxima (a lower bound of the top_k-th best power) less
 // a.ip_margin.  The direct tile computes them again, so that peaks come from the
-// same arithmetic whichever way the rest of the grid was formed.  One
-// wavefront per object; bit c % 64 of word c / 64.
+// same arithmetic whichever way the rest of the grid was formed.  All chunks
+// where the outputs cannot tell such powers apart (infinite or denormal ones: the
+// first of equal powers counts then).  One wavefront per object; bit c % 64 of
+// word c / 64.
 // ---------------------------------------------------------------------------
+template <bool GEN, typename OUT>
 __device__ void mark_chunks(const SweepArgs &a, uint32_t obj) {
     const uint32_t lane = threadIdx.x;
     const int mode = (int)a.obj_ip[obj].mode;
@@ -693,11 +696,18 @@ __device__ void mark_chunks(const SweepArgs &a, uint32_t obj) {
         }
     }
     const float least = tau * (1.0f - a.ip_margin);
+    double power = (double)tau;
+    if constexpr (!GEN)
+        if (!a.pgram)  // the screen's ranks
+            power *= ip_rank_unit((double)a.obj_ys[2 * obj], (double)a.obj_ys[2 * obj + 1],
+                                  (uint32_t)(a.offsets[obj + 1] - a.offsets[obj])) * a.obj_scale[obj];
+    constexpr double kLow = sizeof(OUT) == 4 ? 0x1p-100 : 0x1p-1000, kHigh = sizeof(OUT) == 4 ? 0x1p+120 : 0x1p+1000;
+    const bool all = tau > 0.0f && !(power >= kLow && power <= kHigh);
     uint64_t *bits = a.cand + (uint64_t)obj * a.cand_words;
     for (uint32_t w = 0; w < a.cand_words; ++w) {
         const uint32_t c = 64u * w + lane;
-        bool yes = false;
-        if (c < a.chunks) {
+        bool yes = all && c < a.chunks;
+        if (c < a.chunks && !all) {
             const uint32_t last = 1024u * c + 1023u < a.nf ? 1024u * c + 1023u : a.nf - 1u;
             const uint32_t end = tile_of_bin(last);
             for (uint32_t t = tile_of_bin(1024u * c); t <= end; ++t) {
@@ -717,7 +727,7 @@ __device__ void mark_chunks(const SweepArgs &a, uint32_t obj) {
 template <bool GEN, typename IN>
 __global__ __launch_bounds__(64) void k_colfac(SweepArgs a) {
     const uint32_t marks = a.cand ? a.K : 0u;
-    if (blockIdx.x < marks) return mark_chunks(a, blockIdx.x);
+    if (blockIdx.x < marks) return mark_chunks<GEN, IN>(a, blockIdx.x);
     uint32_t obj, block;
     if (!slot_block(a, blockIdx.x - marks, obj, block)) return;
     if (a.obj_ip && a.obj_ip[obj].mode == 0u) return;

@@ -57,3 +57,25 @@ def test_two_epochs(h, n, gen):
         ys.append(0.9999 - 1e-4 * (k + 1) * rng.uniform(0, 1, n))
         ds.append(rng.uniform(0.9, 1.0, n))
     check(ts, ys, ds if gen else None, nf, 3, F64)
+
+
+@pytest.mark.parametrize("dtype", [F32, F64])
+@pytest.mark.parametrize("normalize", [False, True])
+@pytest.mark.parametrize("unit", [1e-37, 1e-30, 1e-26, 1e-20, 1.0, 1e15, 1e24, 1e37])
+def test_units_of_the_magnitudes(unit, normalize, dtype):
+    """Flux densities in any unit, powers with and without their normalisation;
+    where FP32 powers are denormal or infinite, the first of the equal ones is
+    the peak.  The same objects in units of 1 have their peaks in the same bins
+    (FP64: the unit is a power of two, so that only exponents differ)."""
+    rng = np.random.default_rng(17)
+    nf, K, n = 400009, 40, 90
+    two = 2.0 ** np.round(np.log2(unit))
+    ts = [np.sort(rng.uniform(0.0, 1500.0, n)) for _ in range(K)]
+    ys = [np.sin(2 * np.pi * rng.uniform(0.3, 20.0) * t) + rng.normal(0, 0.3, n) for t in ts]
+    ys[3] = np.zeros(n)
+    ys[4] = np.full(n, 3.0)
+    r = check(ts, [two * y for y in ys], None, nf, 3, dtype, normalize=normalize)
+    if dtype == F64:
+        ref = check(ts, ys, None, nf, 3, dtype, normalize=normalize)
+        assert np.array_equal(r["index"], ref["index"])
+        assert (r["index"][5:, 0] > 0).all() and (r["power"][5:, 0] > 0).all()
