@@ -12,11 +12,13 @@
 
 namespace lsamd {
 
-// Coarse-grid sweep, per object: the mode (0: direct) and the centre of its
-// time span.
+// Coarse-grid sweep, per object: the mode (0: direct), the centre of its time
+// span, and the sum of the squares of its y (generalized: of (w/W) (y - ybar)),
+// times its y scale.
 struct InterpObj {
     double tc;
-    uint32_t mode, unused;
+    uint32_t mode;
+    float energy;
 };
 
 struct SweepArgs {

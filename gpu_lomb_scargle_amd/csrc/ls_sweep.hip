@@ -283,9 +283,10 @@ __global__ __launch_bounds__(T) void k_obj_stats_split(StatsArgs a) {
     if (!a.rec_t) return;
     // the object's 16-observation slots, up to the next object's first
     for (uint64_t s = (b >> 4) + k + tid; s < (e >> 4) + k + 1; s += T) a.slot_obj[s] = k;
+    double energy = 0.0;
     {  // largest |y| (generalized: (w/W) |y - ybar|) and weight, as powers of two
         const double iW = 1.0 / W;
-        double my = 0.0, mw = a.split_gen ? 0.0 : 1.0;
+        double my = 0.0, mw = a.split_gen ? 0.0 : 1.0, my2 = 0.0;
         each([&](uint64_t, double yi, double di, double) {
             double yv = yi;
             if (a.split_gen) {
@@ -294,12 +295,14 @@ __global__ __launch_bounds__(T) void k_obj_stats_split(StatsArgs a) {
                 mw = fmax(mw, w);
             }
             my = fmax(my, fabs(yv));
+            my2 += yv * yv;
         });
         my = most(my);
         mw = most(mw);
         int ey = 0, ew = 0;
         (void)frexp(my, &ey);  // my = f 2^ey, f in [0.5, 1)
         (void)frexp(mw, &ew);
+        if (a.obj_ip) energy = ldexp(sum(my2), -2 * ey);
         if (tid == 0) {
             a.obj_ys[2 * k] = (float)(my > 0.0 ? ldexp(1.0, -ey) : 1.0);
             a.obj_ys[2 * k + 1] = (float)(mw > 0.0 ? ldexp(1.0, -ew) : 1.0);
@@ -324,7 +327,7 @@ __global__ __launch_bounds__(T) void k_obj_stats_split(StatsArgs a) {
             InterpObj o;
             o.tc = tc;
             o.mode = mode;
-            o.unused = 0;
+            o.energy = (float)energy;
             a.obj_ip[k] = o;
         }
     }

@@ -659,8 +659,13 @@ __global__ __launch_bounds__(T) void k_sweep_split64(SweepArgs a) {
 // a.ip_margin.  The direct tile computes them again, so that peaks come from the
 // same arithmetic whichever way the rest of the grid was formed.  All chunks
 // where the outputs cannot tell such powers apart (infinite or denormal ones: the
-// first of equal powers counts then).  One wavefront per object; bit c % 64 of
-// word c / 64.
+// first of equal powers counts then), and where the sums are no longer good to
+// the margin: their error is some 5e-4 (FP32 periodograms: 3e-7) of
+// sqrt(sum y^2), and 3.5 times that at the worst of 10^5 bins, so the peak's
+// |sum y e^{2 pi i f t}| has to reach 1/16 of it.  Noise reaches 3.5; what does not
+// is the leakage of an uncentred mean or a smooth signal in evenly sampled
+// data (65,000 fluxes around 1 searched at 20 cycles per day: 1/250, and another
+// bin won).  One wavefront per object; bit c % 64 of word c / 64.
 // ---------------------------------------------------------------------------
 template <bool GEN, typename OUT>
 __device__ void mark_chunks(const SweepArgs &a, uint32_t obj) {
@@ -696,13 +701,20 @@ __device__ void mark_chunks(const SweepArgs &a, uint32_t obj) {
         }
     }
     const float least = tau * (1.0f - a.ip_margin);
-    double power = (double)tau;
-    if constexpr (!GEN)
+    // power of tau, and of a sum of 1/16 sqrt(sum y^2) (P = |Z|^2 scale / N, or
+    // 2 |Z|^2 / YY)
+    const double ys = (double)a.obj_ys[2 * obj], energy = (double)a.obj_ip[obj].energy;
+    double power = (double)tau, floor = energy / (ys * ys) / 256.0;
+    if constexpr (GEN) {
+        floor *= 2.0 / a.obj_gen[kGen * obj + 7];
+    } else {
+        const uint32_t n = (uint32_t)(a.offsets[obj + 1] - a.offsets[obj]);
+        floor *= a.obj_scale[obj] / (double)n;
         if (!a.pgram)  // the screen's ranks
-            power *= ip_rank_unit((double)a.obj_ys[2 * obj], (double)a.obj_ys[2 * obj + 1],
-                                  (uint32_t)(a.offsets[obj + 1] - a.offsets[obj])) * a.obj_scale[obj];
+            power *= ip_rank_unit(ys, (double)a.obj_ys[2 * obj + 1], n) * a.obj_scale[obj];
+    }
     constexpr double kLow = sizeof(OUT) == 4 ? 0x1p-100 : 0x1p-1000, kHigh = sizeof(OUT) == 4 ? 0x1p+120 : 0x1p+1000;
-    const bool all = tau > 0.0f && !(power >= kLow && power <= kHigh);
+    const bool all = energy > 0.0 && !(power >= kLow && power <= kHigh && power >= floor);
     uint64_t *bits = a.cand + (uint64_t)obj * a.cand_words;
     for (uint32_t w = 0; w < a.cand_words; ++w) {
         const uint32_t c = 64u * w + lane;

@@ -79,3 +79,29 @@ def test_units_of_the_magnitudes(unit, normalize, dtype):
         ref = check(ts, ys, None, nf, 3, dtype, normalize=normalize)
         assert np.array_equal(r["index"], ref["index"])
         assert (r["index"][5:, 0] > 0).all() and (r["power"][5:, 0] > 0).all()
+
+
+@pytest.mark.parametrize("gen", [False, True], ids=["standard", "generalized"])
+@pytest.mark.parametrize("n,nf", [(4001, 60011), (20011, 40009), (65003, 12007)])
+@pytest.mark.parametrize("top_k", [1, 3])
+def test_evenly_sampled_light_curves(n, nf, top_k, gen):
+    """Fluxes every half hour around 1, not centred (standard), with signals of
+    0, 10^-4 and 10^-3 of that, or a smooth one without noise, searched where the window's and the signal's
+    sidelobes are small: peaks of 10^-5 and less of the magnitudes' own power,
+    where the screen's rounding shows."""
+    rng = np.random.default_rng(n)
+    t = 100.0 + np.arange(n) / 48.0
+    T = t[-1] - t[0]
+    K = max(2, int(np.ceil(1.05e9 / (n * nf))))
+    df = 0.97 / (1.3 * 3 * T)
+    lo = 2 * np.pi * 20.0
+    ts, ys, ds = [], [], []
+    for k in range(K):
+        amp = (0.0, 1e-4, 1e-3)[k % 3]
+        y = 1.0 + amp * np.sin(2 * np.pi * (20.0 + rng.uniform(0.1, 0.9) * nf * df) * t + k) + 1e-4 * rng.normal(0, 1, n)
+        if k % 4 == 3:
+            y = 1.0 + 0.01 * np.sin(2 * np.pi * 1.3 * t)
+        ts.append(t)
+        ys.append(y)
+        ds.append(np.full(n, 1e-4))
+    check(ts, ys, ds if gen else None, nf, top_k, F64, lo=lo, hi=lo + 2 * np.pi * nf * df)
