@@ -35,7 +35,7 @@ EXPORTED = [
     "lsamd_sweep_workspace_size", "lsamd_sweep", "lsamd_batch_host", "lsamd_cpu_batch",
     "lsamd_cpu_single", "lsamd_row_argmax", "lsamd_count_objects", "lsamd_object_offsets", "lsamd_last_error_code",
     "lsamd_last_error", "lsamd_clear_error", "lsamd_device_count", "lsamd_set_timing",
-    "lsamd_last_sweep_kernel_ms", "lsamd_set_tile", "lsamd_get_tile", "lsamd_version",
+    "lsamd_last_sweep_kernel_ms", "lsamd_set_tile", "lsamd_get_tile", "lsamd_sweep_tile", "lsamd_version",
     "lsamd_graph_create", "lsamd_graph_launch", "lsamd_graph_destroy", "lsamd_autotune",
     "lsamd_autotune_workspace_size", "lsamd_power_grad", "lsamd_refine_peaks", "lsamd_read_table",
     "lsamd_write_periods", "lsamd_segment_workspace_size", "lsamd_segment", "lsamd_sweep_static",
@@ -107,6 +107,8 @@ def _declare(L):
     L.lsamd_set_tile.argtypes = [c_int, c_int, c_int, c_int]
     L.lsamd_set_tile.restype = c_int
     L.lsamd_get_tile.argtypes = [c_int, c_int, c_int, POINTER(c_int), POINTER(c_int)]
+    L.lsamd_sweep_tile.argtypes = [POINTER(SweepArgs), POINTER(c_int), POINTER(c_int)]
+    L.lsamd_sweep_tile.restype = None
     L.lsamd_version.restype = c_int
     L.lsamd_graph_create.argtypes = [POINTER(SweepArgs), c_void_p, c_size_t, c_void_p, POINTER(c_void_p)]
     L.lsamd_graph_create.restype = c_int

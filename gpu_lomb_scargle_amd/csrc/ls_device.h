@@ -79,7 +79,6 @@ struct TileEntry {
 };
 extern const TileEntry kPlainTiles[];  // ls_sweep_plain.hip
 extern const int kPlainTileCount;
-extern const TileEntry kPlainStep[2];  // standard FP64, chosen by the call's size (plan_workspace)
 extern const TileEntry kSplitTiles[];  // ls_sweep_split.hip
 extern const int kSplitTileCount;
 

@@ -530,7 +530,7 @@ int lsamd_batch_host(int variant, int dtype, int form, int normalize, int precen
             a.peak_power = peaks + out_pow + (size_t)s0 * tk * rsz;
             a.peak_period = peaks + out_per + (size_t)s0 * tk * rsz;
         }
-        const size_t wsb = sweep_part_bytes(&a, K);
+        const size_t wsb = lsamd_sweep_workspace_size(&a);
         int r = LSAMD_OK;
         if (c.ws.cap < wsb) {
             // growing the workspace frees it: wait for the sweeps using it
@@ -538,7 +538,7 @@ int lsamd_batch_host(int variant, int dtype, int form, int normalize, int precen
             r = ensure(c.ws, wsb);
             if (r) return r;
         }
-        r = sweep_part(&a, K, c.ws.p, c.ws.cap, c.stream);
+        r = lsamd_sweep(&a, c.ws.p, c.ws.cap, c.stream);
         if (r) return r;
         if (!small) HIP_OK(hipEventRecord(c.slice[i % kAhead], c.stream));
         return LSAMD_OK;

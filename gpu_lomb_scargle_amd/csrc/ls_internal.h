@@ -60,15 +60,8 @@ struct Workspace {
     uint32_t chunks = 0;
     uint32_t slices = 1;    // observation slices per (object, chunk)
     Tile tile{};
-    int step = 0;           // plain standard FP64: 1 + index of kPlainStep, not a tile of the registry
 };
-// call_objects: objects of the whole call that this sweep is a part of (0: it is
-// the whole call, or may not look at their number when obs_slices is 1).
-int plan_workspace(const lsamd_sweep_args *a, Workspace *w, uint32_t call_objects = 0);
-// lsamd_sweep and lsamd_sweep_workspace_size for a part of a call
-int sweep_part(const lsamd_sweep_args *a, uint32_t call_objects, void *workspace, size_t workspace_bytes,
-               void *stream);
-size_t sweep_part_bytes(const lsamd_sweep_args *a, uint32_t call_objects);
+int plan_workspace(const lsamd_sweep_args *a, Workspace *w);
 
 // ---- CPU path (ls_cpu.cpp) -------------------------------------------------
 int cpu_batch(int variant, int dtype, int normalize, const uint32_t *objectId, const void *t,

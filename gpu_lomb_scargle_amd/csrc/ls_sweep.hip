@@ -493,12 +493,16 @@ Tile default_tile(int form, int variant) {
     return Tile{256, 1};
 }
 
-// Bins of all objects from which the stepped plain sweep is chosen, with 8 and
-// with 16 bins per thread.  Measured (165 observations each, us, one bin per
-// thread / 8 / 16): 1 object x 131,072 bins 88 / 92; 4 x 40,000 109 / 95; 1 x
-// 262,143 137 / 95 / 132; 20 x 50,000 - / 165 / 233; 1 x 1,000,000 - / 159 / 137;
-// 4 x 500,000 - / 282 / 231; 100 x 100,003 3380 / 1309 / 1063.
-constexpr uint64_t kStepMinBins = 9u << 14, kStepWideBins = 1u << 21;
+// Bins from which the stepped plain sweep is chosen: of each object, of an
+// object alone; bins of all objects from which it is with whole chains.  Whole
+// sweep, us, 165 observations each (one bin per thread / half chains / whole):
+// 1 object x 65,536 bins 49 / 79 / 111, x 131,072 73 / 79 / 111, x 262,143
+// 123 / 80 / 110, x 1,000,000 386 / 133 / 117; 4 x 8192 44 / 108 / 141, x 16,384
+// 47 / 79 / 111; 20 x 8192 88 / 110 / 143, x 16,384 135 / 82 / 113; 100 x 8192
+// 289 / 166 / 149, x 100,003 3041 / 1072 / 882; 1000 x 8192 2494 / 1001 / 783.  A
+// line on the bins of all objects would spare the few small objects their 65 us,
+// but an object's powers would depend on how many others there are.
+constexpr uint64_t kStepMinFreqs = 1u << 13, kStepAloneFreqs = 9u << 14, kStepWideBins = 1u << 21;
 
 // Kernel timing, per host thread: the events bracketing this thread's last
 // timed sweep (created on the device of that sweep's stream).
@@ -549,8 +553,18 @@ Tile current_tile(int form, int variant, int dtype) {
     return default_tile(form, variant);
 }
 
+// The tile of a sweep: the caller's, the process default, or the built-in one.
+// Built-in for plain standard FP64: bins of a thread stepped from one another
+// where the grid is long enough.  The number of bins per object alone decides
+// that, so that an object's powers do not depend on what is swept beside it
+// (obs_slices = 0: an object swept by itself has a line of its own, as it has its
+// observation slices in the split forms); how many of them a thread takes, with
+// the same bits, follows the call's size.
 Tile tile_of(const lsamd_sweep_args *a) {
     if (a->tile_threads > 0 && a->tile_fpt > 0) return Tile{a->tile_threads, a->tile_fpt};
+    if (a->form == LSAMD_FORM_PLAIN && a->variant == LSAMD_STANDARD && a->dtype == LSAMD_F64 &&
+        a->num_freqs >= (a->num_objects == 1 && a->obs_slices == 0 ? kStepAloneFreqs : kStepMinFreqs) && g_default_tile[a->form][a->variant].load(std::memory_order_relaxed) == 0u)
+        return Tile{256, (uint64_t)a->num_objects * a->num_freqs >= kStepWideBins ? 16 : 8};
     return current_tile(a->form, a->variant, a->dtype);
 }
 
@@ -559,22 +573,9 @@ bool tile_supported(int form, int variant, int threads, int fpt) {
            find_tile(form, variant, LSAMD_F64, threads, fpt) != nullptr;
 }
 
-int plan_workspace(const lsamd_sweep_args *a, Workspace *w, uint32_t call_objects) {
+int plan_workspace(const lsamd_sweep_args *a, Workspace *w) {
     *w = Workspace{};
-    // The plain standard FP64 sweep: where the tile is the built-in one, bins of
-    // a thread are stepped from one another, unless the call is so small that
-    // one bin per thread, with eight times the wavefronts, is sooner done.  The
-    // parts of a call follow the whole call, and with obs_slices = 1 otherwise
-    // only the grid counts, so that an object's result does not depend on what
-    // is swept beside it.
-    Tile tile = tile_of(a);
-    if (a->form == LSAMD_FORM_PLAIN && a->variant == LSAMD_STANDARD && a->dtype == LSAMD_F64 &&
-        tile.threads == 256 && tile.fpt == 1) {
-        const uint64_t bins = (uint64_t)(call_objects ? call_objects : a->num_objects) * a->num_freqs;
-        if (a->obs_slices == 1 && !call_objects) w->step = a->num_freqs >= kStepMinBins ? 1 : 0;
-        else w->step = bins >= kStepWideBins ? 2 : bins >= kStepMinBins ? 1 : 0;
-        if (w->step) tile = Tile{kPlainStep[w->step - 1].T, kPlainStep[w->step - 1].M};
-    }
+    const Tile tile = tile_of(a);
     w->tile = tile;
     const uint64_t per_chunk = (uint64_t)tile.threads * tile.fpt;
     w->chunks = (uint32_t)((a->num_freqs + per_chunk - 1) / per_chunk);
@@ -687,6 +688,12 @@ size_t lsamd_sweep_workspace_size(const lsamd_sweep_args *a) {
     return w.bytes;
 }
 
+void lsamd_sweep_tile(const lsamd_sweep_args *a, int *threads, int *fpt) {
+    const Tile t = a && a->form >= 0 && a->form < kForms && a->variant >= 0 && a->variant <= 1 ? tile_of(a) : Tile{0, 0};
+    if (threads) *threads = t.threads;
+    if (fpt) *fpt = t.fpt;
+}
+
 int lsamd_set_tile(int form, int variant, int threads, int fpt) {
     if (form < 0 || form >= kForms || variant < 0 || variant > 1)
         return set_error(LSAMD_ERR_INVALID, "lsamd_set_tile: bad form/variant");
@@ -730,7 +737,7 @@ double lsamd_last_sweep_kernel_ms(void) {
 // device array of lsamd_sweep_static (no kernel timing, which would create
 // events).
 static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspace_bytes, void *stream_v,
-                      bool from_scratch, uint32_t call_objects) {
+                      bool from_scratch) {
     if (!a) return set_error(LSAMD_ERR_INVALID, "lsamd_sweep: null args");
     if (a->variant != LSAMD_STANDARD && a->variant != LSAMD_GENERALIZED)
         return set_error(LSAMD_ERR_INVALID, "lsamd_sweep: bad variant");
@@ -760,7 +767,7 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
         return set_error(LSAMD_ERR_INVALID, "lsamd_sweep: tile shape " + std::to_string(a->tile_threads) +
                                                 "x" + std::to_string(a->tile_fpt) + " not compiled");
     Workspace w;
-    plan_workspace(a, &w, call_objects);
+    plan_workspace(a, &w);
     if (from_scratch && w.bytes > workspace_bytes)
         return set_error(LSAMD_ERR_INVALID, "lsamd_sweep_static: these arguments need " +
                                                 std::to_string(w.bytes) + " bytes of workspace, more than the " +
@@ -769,7 +776,7 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
     if (!workspace || workspace_bytes < w.bytes)
         return set_error(LSAMD_ERR_INVALID, "lsamd_sweep: workspace too small (need " +
                                                 std::to_string(w.bytes) + " bytes)");
-    const TileEntry *te = w.step ? &kPlainStep[w.step - 1] : find_tile(a->form, a->variant, a->dtype, w.tile.threads, w.tile.fpt);
+    const TileEntry *te = find_tile(a->form, a->variant, a->dtype, w.tile.threads, w.tile.fpt);
     if (!te) return set_error(LSAMD_ERR_INVALID, "lsamd_sweep: no kernel for this tile");
 
     hipStream_t st = static_cast<hipStream_t>(stream_v);
@@ -1043,7 +1050,7 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
 }
 
 int lsamd_sweep(const lsamd_sweep_args *a, void *workspace, size_t workspace_bytes, void *stream_v) {
-    return sweep_into(a, workspace, workspace_bytes, stream_v, false, 0);
+    return sweep_into(a, workspace, workspace_bytes, stream_v, false);
 }
 
 int lsamd_sweep_static(const lsamd_sweep_args *a, void *stream_v) {
@@ -1063,7 +1070,7 @@ int lsamd_sweep_static(const lsamd_sweep_args *a, void *stream_v) {
                                                 hipGetErrorString(e));
         g_scratch_ptr[dev].store(ptr, std::memory_order_release);
     }
-    return sweep_into(a, ptr, kStaticScratchBytes, stream_v, true, 0);
+    return sweep_into(a, ptr, kStaticScratchBytes, stream_v, true);
 }
 
 struct lsamd_graph {
@@ -1219,18 +1226,3 @@ int lsamd_autotune(const lsamd_sweep_args *a, void *workspace, size_t workspace_
 }
 
 }  // extern "C"
-
-namespace lsamd {
-
-int sweep_part(const lsamd_sweep_args *a, uint32_t call_objects, void *workspace, size_t workspace_bytes,
-               void *stream) {
-    return sweep_into(a, workspace, workspace_bytes, stream, false, call_objects);
-}
-
-size_t sweep_part_bytes(const lsamd_sweep_args *a, uint32_t call_objects) {
-    Workspace w;
-    plan_workspace(a, &w, call_objects);
-    return w.bytes;
-}
-
-}  // namespace lsamd

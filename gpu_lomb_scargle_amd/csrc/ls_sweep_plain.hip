@@ -119,18 +119,21 @@ __global__ __launch_bounds__(T) void k_sweep_plain_std(SweepArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Standard FP64 variant, M bins per thread from one sine and cosine.  A sine
+// Standard FP64 variant, 16 bins from one sine and cosine.  A sine
 // and cosine of every phase is 59 of the 70 instructions per term above, though
 // the phases of a thread's bins, x_m = fl(om_m t), lie one common step
 // D = 64 df t apart up to their roundings.  So the phasor of the middle bin is
-// evaluated and the others follow from it,
+// (the ninth of 16) is evaluated and the others follow from it,
 //   e^{i x_m} = e^{i x_{m-1}} e^{i D} (1 + i r),  r = (x_m - x_{m-1}) - D,
 // where r holds the roundings of om_m and of the products: both differences
 // are exact (|x_{m-1}| >= D, see `low`), so each phase is the reference's own,
 // rounding included.  |r| <= 2 ulp of a phase, so that the 1 + r^2/2 of the last
 // factor stays within 2e-14 for phases below kStepFar (typically 1e-15).
-// 13 instructions per term and 59 / M for the middle bin; four (M = 8) or eight
-// (M = 16) steps each way add 2e-16 to 3e-16 to a phasor.  Against the CPU path over the test light
+// 13 instructions per term and 59 / 16 for the middle bin; the eight
+// steps each way add 2e-16 to 3e-16 to a phasor.  M = 16: a thread forms all 16
+// bins.  M = 8: the upper or the lower eight of them (by wavefront), from the same middle bin
+// in the same steps, so both give the same bits; twice the wavefronts, for
+// calls that would leave SIMDs idle.  Against the CPU path over the test light
 // curves (14 to 3555 observations) 2.3e-13 on bins of at least 1e-6 of the
 // peak, with a stride of 256 bins instead of 64 1.1e-11 at the lowest bins
 // (the differences are not exact there).
@@ -138,14 +141,14 @@ __global__ __launch_bounds__(T) void k_sweep_plain_std(SweepArgs a) {
 // amplifies the phasors' error (condition number above kStepCond), frequencies
 // below the step (or of both signs in a thread), phases past kStepFar, objects of fewer than
 // kStepLeastObs observations, most of whose bins are ill-conditioned.
-// 100 objects (17,200 observations) x 100,003 bins: 3.38 -> 1.31 ms (M = 8) and
-// 0.96 (M = 16, two wavefronts per SIMD by 18 spilled registers, mostly outside
-// the loop; 1.06 with one and none).  M = 10, 12 and 14 lie between (1.03, 1.14 and
-// 1.07 where M = 16 has 0.98), four wavefronts of M = 8 spill to 2.8 ms.
+// 100 objects (17,200 observations) x 100,003 bins: 3.38 -> 0.96 ms (M = 16, two wavefronts per SIMD by 18 spilled registers, mostly outside
+// the loop; 1.06 with one and none).  Chains of 8, 10, 12 and 14 bins: 1.31, 1.03, 1.14 and
+// 1.07 where 16 has 0.98; four wavefronts of 8 spill to 2.8 ms.
 // ---------------------------------------------------------------------------
 constexpr double kStepFar = 268435456.0;  // 2^28
 constexpr double kStepCond = 16.0;
 constexpr uint32_t kStepLeastObs = 16;
+constexpr int kStepRun = 16, kStepMid = 8;  // bins of a chain, its middle bin
 
 // Power at omega from a sine and cosine per observation, as k_sweep_plain_std
 // gives it (256 observations at a time near or far); the observations'
@@ -192,7 +195,8 @@ __global__ __launch_bounds__(T, 2) void k_sweep_plain_step(SweepArgs a) {
     __shared__ double s_pp[T / 64][kPeaks];
     __shared__ uint32_t s_pi[T / 64][kPeaks];
     __shared__ uint64_t s_item;
-    constexpr int kMid = M / 2;
+    static_assert(T == 256 && (M == kStepRun || M == kStepMid), "chains of whole wavefronts, or halves");
+    constexpr bool kHalf = M != kStepRun;
     for (uint64_t item = first_item(a, &s_item); item < a.total_items;
          item = next_item(a, &s_item, item)) {
         uint32_t obj, chunk;
@@ -202,18 +206,27 @@ __global__ __launch_bounds__(T, 2) void k_sweep_plain_step(SweepArgs a) {
         const double *gy = static_cast<const double *>(a.y);
         const uint32_t tid = threadIdx.x;
         const uint32_t kbase = chunk * (uint32_t)(T * M);
-        // a wavefront's bins are consecutive: bin m of a lane is k0 + 64 m
-        const uint32_t k0 = kbase + (tid >> 6) * (uint32_t)(64 * M) + (tid & 63u);
+        // The bins of a wavefront's chains are consecutive: bin b of a lane's chain
+        // is k0 + 64 b.  Entry m of a thread is bin m, or with half chains bin 8 + m
+        // (upper) or 7 - m: the steps lead away from the middle.
+        const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+        const uint32_t k0 = kbase + (kHalf ? wave >> 1 : wave) * (uint32_t)(64 * kStepRun) + (tid & 63u);
+        const bool upper = (wave & 1u) != 0u;
+        auto chain_bin = [&](int m) { return (uint32_t)(!kHalf ? m : upper ? kStepMid + m : kStepMid - 1 - m); };
+        auto bin_omega = [&](uint32_t b) { return a.fmin_r + (a.fstep_r * (double)(k0 + 64u * b)); };
         const double step = 64.0 * a.fstep_r;
         double om[M], xc[M], xs[M], cc[M], cs[M];
 #pragma unroll
         for (int m = 0; m < M; ++m) {
-            om[m] = a.fmin_r + (a.fstep_r * (double)(k0 + 64u * (uint32_t)m));
+            om[m] = bin_omega(chain_bin(m));
             xc[m] = xs[m] = cc[m] = cs[m] = 0.0;
         }
-        const double om_a = a.fmin_r + a.fstep_r * (double)kbase, om_b = om_a + a.fstep_r * (double)(T * M);
+        const double om_mid = bin_omega((uint32_t)kStepMid);
+        // over the 4096 bins that whole chains of the workgroup would have
+        const double om_a = a.fmin_r + a.fstep_r * (double)(kbase & ~(uint32_t)(T * kStepRun - 1));
+        const double om_b = om_a + a.fstep_r * (double)(T * kStepRun);
         const double om_most = fmax(fabs(om_a), fabs(om_b));
-        const bool crosses = (om[0] < 0.0) != (om[M - 1] < 0.0);
+        const bool crosses = (bin_omega(0u) < 0.0) != (bin_omega((uint32_t)(kStepRun - 1)) < 0.0);
         bool direct = end - beg < (uint64_t)kStepLeastObs;
         for (uint64_t b0 = beg; b0 < end && !direct; b0 += T) {
             const uint32_t cnt = (uint32_t)((end - b0) < (uint64_t)T ? (end - b0) : (uint64_t)T);
@@ -239,13 +252,26 @@ __global__ __launch_bounds__(T, 2) void k_sweep_plain_step(SweepArgs a) {
                     cc[m] = fma(c, c, cc[m]);
                     cs[m] = fma(c, s, cs[m]);
                 };
-                const double xm = om[kMid] * ty.x;
+                const double xm = om_mid * ty.x;
                 double cm, sm;
                 sincos_near<false>(xm, &sm, &cm);
-                add(kMid, cm, sm);
                 double c = cm, s = sm, x = xm;
+                if constexpr (kHalf) {
+                    const double es = upper ? e.y : -e.y, ds = upper ? d : -d;
 #pragma unroll
-                for (int m = kMid + 1; m < M; ++m) {
+                    for (int m = 0; m < M; ++m) {
+                        if (m > 0 || !upper) {  // (the middle bin itself is the first upper one)
+                            const double xn = om[m] * ty.x;
+                            turn_step(c, s, e.x, es, (xn - x) - ds);
+                            x = xn;
+                        }
+                        add(m, c, s);
+                    }
+                    continue;
+                }
+                add(kStepMid, cm, sm);
+#pragma unroll
+                for (int m = kStepMid + 1; m < M; ++m) {
                     const double xn = om[m] * ty.x;
                     turn_step(c, s, e.x, e.y, (xn - x) - d);
                     x = xn;
@@ -255,7 +281,7 @@ __global__ __launch_bounds__(T, 2) void k_sweep_plain_step(SweepArgs a) {
                 s = sm;
                 x = xm;
 #pragma unroll
-                for (int m = kMid - 1; m >= 0; --m) {
+                for (int m = kStepMid - 1; m >= 0; --m) {
                     const double xn = om[m] * ty.x;
                     turn_step(c, s, e.x, -e.y, (xn - x) + d);
                     x = xn;
@@ -272,7 +298,7 @@ __global__ __launch_bounds__(T, 2) void k_sweep_plain_step(SweepArgs a) {
             const double ss = nobs - cc[m];
             const bool ill = !(fma(cc[m], ss, -(cs[m] * cs[m])) >= least);
             const bool low = crosses || !(fabs(om[m]) >= step);
-            if ((direct || ill || low) && k0 + 64u * (uint32_t)m < a.nf) flags |= 1u << m;
+            if ((direct || ill || low) && k0 + 64u * chain_bin(m) < a.nf) flags |= 1u << m;
             P[m] = direct ? 0.0 : plain_std_power(om[m], xc[m], xs[m], cc[m], ss, cs[m], scale);
             __builtin_amdgcn_sched_barrier(0);  // one bin's temporaries at a time
         }
@@ -280,8 +306,8 @@ __global__ __launch_bounds__(T, 2) void k_sweep_plain_step(SweepArgs a) {
         for (int m = 0; m < M; ++m) {
             const bool mine = ((flags >> m) & 1u) != 0u;
             if (__ballot(mine) == 0u) continue;
-            const double omega = a.fmin_r + (a.fstep_r * (double)(k0 + 64u * (uint32_t)m));
-            const double most = chunk_omega_most(a, k0 - (tid & 63u) + 512u * (uint32_t)(m / 8 + 1));
+            const double omega = bin_omega(chain_bin(m));
+            const double most = chunk_omega_most(a, k0 - (tid & 63u) + 512u * (chain_bin(m) / 8u + 1u));
             const double p = direct_std_power(a, beg, end, omega, most, scale);
 #pragma unroll
             for (int q = 0; q < M; ++q) P[q] = mine && q == m ? p : P[q];
@@ -291,10 +317,11 @@ __global__ __launch_bounds__(T, 2) void k_sweep_plain_step(SweepArgs a) {
         peaks_init(L);
 #pragma unroll
         for (int m = 0; m < M; ++m) {
-            const uint32_t kf = k0 + 64u * (uint32_t)m;
+            const uint32_t kf = k0 + 64u * chain_bin(m);
             if (kf < a.nf) {
                 if (pg) pg[(uint64_t)obj * a.nf + kf] = P[m];
-                peaks_add(L, a.top_k, P[m], kf);
+                if constexpr (kHalf) peaks_merge(L, a.top_k, P[m], kf);  // (not in ascending order)
+                else peaks_add(L, a.top_k, P[m], kf);
             }
         }
         if (a.top_k) write_partial<double, T>(a, L, obj, chunk, s_pp, s_pi);
@@ -616,8 +643,6 @@ const TileEntry kPlainTiles[] = {
     LS_PLAIN_STD(float, LSAMD_F32, 256, 1), LS_PLAIN_STD(double, LSAMD_F64, 256, 1),
     LS_PLAIN_STD(float, LSAMD_F32, 256, 2), LS_PLAIN_STD(double, LSAMD_F64, 256, 2),
     LS_PLAIN_GEN(float, LSAMD_F32, 256, 1), LS_PLAIN_GEN(double, LSAMD_F64, 256, 1),
-};
-const TileEntry kPlainStep[2] = {
     {LSAMD_FORM_PLAIN, 0, LSAMD_F64, 256, 8, k_sweep_plain_step<256, 8>, nullptr},
     {LSAMD_FORM_PLAIN, 0, LSAMD_F64, 256, 16, k_sweep_plain_step<256, 16>, nullptr},
 };

@@ -44,7 +44,8 @@ class SweepPlan:
     by default objects are processed longest first.  obs_slices=1 keeps the
     way an object's sums are formed independent of what else the plan sweeps
     (0, the default, lets a single object's observations be spread over
-    workgroups and small float32 split32 sweeps keep the direct sums).  tile=(threads, freqs_per_thread)
+    workgroups, small float32 split32 sweeps keep the direct sums and a single
+    object's plain float64 sweep keep a sine and cosine per bin).  tile=(threads, freqs_per_thread)
     picks a compiled tile shape for this plan only (None: the process
     default); autotune() sets it to the fastest.
     """
@@ -105,11 +106,8 @@ class SweepPlan:
     def tile(self):
         """(threads, freqs_per_thread) of this plan's sweep kernel."""
         from ctypes import c_int
-        a = self.args
-        if a.tile_threads and a.tile_fpt:
-            return a.tile_threads, a.tile_fpt
         T, M = c_int(), c_int()
-        self.lib.lsamd_get_tile(a.form, a.variant, a.dtype, byref(T), byref(M))
+        self.lib.lsamd_sweep_tile(byref(self.args), byref(T), byref(M))
         return T.value, M.value
 
     def autotune(self, stream=None):

@@ -137,11 +137,14 @@ typedef struct lsamd_sweep_args {
     void *peak_power;        /* device, K*top_k, or NULL */
     void *peak_period;       /* device, K*top_k (days), or NULL */
     int32_t schedule;        /* enum lsamd_schedule */
-    int32_t obs_slices;      /* split forms, 0: a sweep of one object with many observations
-                              * spreads them over workgroups, and a small FP32 split32 sweep
+    int32_t obs_slices;      /* 0: a split-form sweep of one object with many observations
+                              * spreads them over workgroups, a small FP32 split32 sweep
                               * takes its sums at every bin where a larger one takes them on a
-                              * coarse grid (results then differ from the same object swept in
-                              * another batch by rounding only); 1: neither */
+                              * coarse grid, and a plain standard FP64 sweep of one object
+                              * takes a sine and cosine per bin up to 147,455 bins, one of
+                              * several objects up to 8,191 (results then differ from the same
+                              * object swept in another batch by rounding only); 1: none of
+                              * these, an object's result depends on itself and the grid alone */
     /* Tile shape of this sweep (threads per workgroup, frequencies per
      * thread), one of the shapes compiled for form/variant (lsamd_autotune
      * reports the fastest); 0, 0: the process default (lsamd_set_tile, else
@@ -329,8 +332,12 @@ double lsamd_last_sweep_kernel_ms(void);
  * reads it once, when it is planned.  Per-call tiles (the args fields) are
  * the way to run different shapes from several threads. */
 int lsamd_set_tile(int form, int variant, int threads, int freqs_per_thread);
-/* Tile shape lsamd_sweep uses for args that leave the tile at 0 (for reports). */
+/* Tile shape of sweeps whose args leave the tile at 0 (for reports; plain
+ * standard FP64 sweeps of long grids have another built-in one, see
+ * lsamd_sweep_tile). */
 void lsamd_get_tile(int form, int variant, int dtype, int *threads, int *freqs_per_thread);
+/* Tile shape that lsamd_sweep uses for these arguments. */
+void lsamd_sweep_tile(const lsamd_sweep_args *args, int *threads, int *freqs_per_thread);
 
 /* Library version (major*10000 + minor*100 + patch). */
 int lsamd_version(void);
