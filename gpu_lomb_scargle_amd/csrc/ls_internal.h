@@ -60,6 +60,7 @@ struct Workspace {
     uint32_t chunks = 0;
     uint32_t slices = 1;    // observation slices per (object, chunk)
     Tile tile{};
+    size_t spare = 0;       // bytes that lsamd_sweep_workspace_size adds to `bytes`
 };
 int plan_workspace(const lsamd_sweep_args *a, Workspace *w);
 

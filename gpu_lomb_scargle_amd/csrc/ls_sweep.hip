@@ -610,6 +610,15 @@ int plan_workspace(const lsamd_sweep_args *a, Workspace *w) {
     const size_t parts = (size_t)K * w->chunks * kPeaks;
     w->part_pow = take(8 * parts);
     w->part_idx = take(4 * parts);
+    // Where the plain tile follows the call's size, the size that callers ask for
+    // has the partials of its smallest chunks, so that a workspace also serves
+    // calls of fewer objects or bins.
+    if (a->form == LSAMD_FORM_PLAIN && !(a->tile_threads > 0 && a->tile_fpt > 0)) {
+        const uint64_t least = (uint64_t)current_tile(a->form, a->variant, a->dtype).threads *
+                               current_tile(a->form, a->variant, a->dtype).fpt;
+        const size_t most = (size_t)K * ((a->num_freqs + least - 1) / least) * kPeaks;
+        if (most > parts) w->spare = 12 * (most - parts) + 512;
+    }
     // Observation slices (split forms): a single object whose (object, chunk)
     // items are too few to fill the GPU has its observations split over
     // workgroups whose FP64 sums k_combine_slices adds up.  Only single-object
@@ -685,7 +694,7 @@ size_t lsamd_sweep_workspace_size(const lsamd_sweep_args *a) {
     if (!a) return 0;
     Workspace w;
     plan_workspace(a, &w);
-    return w.bytes;
+    return w.bytes + w.spare;
 }
 
 void lsamd_sweep_tile(const lsamd_sweep_args *a, int *threads, int *fpt) {

@@ -172,7 +172,7 @@ int lsamd_sweep(const lsamd_sweep_args *args, void *workspace, size_t workspace_
  * counterpart in the reference: for callers that cannot allocate device
  * memory (code under stream capture, tight serving loops, harnesses that
  * forbid hipMalloc).  Arguments as for lsamd_sweep; sweeps whose
- * lsamd_sweep_workspace_size() exceeds the array fail with
+ * workspace exceeds the array fail with
  * LSAMD_ERR_INVALID before anything is enqueued.  Every call on one GPU uses
  * that GPU's one array: calls that overlap on one GPU (two streams, two host
  * threads) race and must be serialised by the caller.  Kernel timing

@@ -20,6 +20,20 @@ def _args(K, nf, n, tile=(0, 0), obs_slices=0):
     return a
 
 
+def test_a_workspace_serves_smaller_calls():
+    """The workspace of a call is enough for every call of fewer objects, bins or
+    observations, whatever kernel those take."""
+    L = _native.core()
+    grids = [1, 255, 256, 257, 4096, 8191, 8192, 8193, 40000, 147455, 147456, 262144, 1000003]
+    counts = [1, 2, 3, 9, 10, 11, 200]
+    for obs_slices in (0, 1):
+        size = {(K, nf): L.lsamd_sweep_workspace_size(byref(_args(K, nf, 5000, obs_slices=obs_slices)))
+                for K in counts for nf in grids}
+        for (K, nf), s in size.items():
+            for (k, f), less in size.items():
+                assert k > K or f > nf or less <= s, (K, nf, k, f, obs_slices)
+
+
 def _tile(a):
     T, M = c_int(), c_int()
     _native.core().lsamd_sweep_tile(byref(a), byref(T), byref(M))
