@@ -62,7 +62,9 @@ struct Workspace {
     Tile tile{};
     size_t spare = 0;       // bytes that lsamd_sweep_workspace_size adds to `bytes`
 };
-int plan_workspace(const lsamd_sweep_args *a, Workspace *w);
+// route: the call whose way of forming the sums (coarse grid or direct) this one
+// takes, where it is a trial of it on fewer bins (null: its own).
+int plan_workspace(const lsamd_sweep_args *a, Workspace *w, const lsamd_sweep_args *route = nullptr);
 
 // ---- CPU path (ls_cpu.cpp) -------------------------------------------------
 int cpu_batch(int variant, int dtype, int normalize, const uint32_t *objectId, const void *t,

@@ -573,8 +573,9 @@ bool tile_supported(int form, int variant, int threads, int fpt) {
            find_tile(form, variant, LSAMD_F64, threads, fpt) != nullptr;
 }
 
-int plan_workspace(const lsamd_sweep_args *a, Workspace *w) {
+int plan_workspace(const lsamd_sweep_args *a, Workspace *w, const lsamd_sweep_args *route) {
     *w = Workspace{};
+    if (!route) route = a;
     const Tile tile = tile_of(a);
     w->tile = tile;
     const uint64_t per_chunk = (uint64_t)tile.threads * tile.fpt;
@@ -645,17 +646,17 @@ int plan_workspace(const lsamd_sweep_args *a, Workspace *w) {
     // call's type and grid alone, so that an object's result does not depend
     // on what else is swept with it; with 0 small sweeps, which the direct
     // sums' shorter chain of launches serves sooner, keep those.
-    const bool enough = a->obs_slices == 1 ? a->num_freqs >= kIpAloneFreqs
-                                           : a->num_freqs >= kIpMinFreqs &&
-                                                 (double)n * (double)a->num_freqs >= kIpMinTerms;
+    const uint32_t nf = route->num_freqs;
+    const bool enough = a->obs_slices == 1 ? nf >= kIpAloneFreqs
+                                           : nf >= kIpMinFreqs && (double)n * (double)nf >= kIpMinTerms;
     // (Its room does not depend on which outputs the arguments name.)
-    const bool room = te && te->prep && w->slices == 1 && enough && a->num_freqs < kIpMaxFreqs;
+    const bool room = te && te->prep && w->slices == 1 && enough && nf < kIpMaxFreqs;
     // Peaks without a periodogram, of either type: the coarse grid only finds
     // the chunks that can hold them, and the direct tile sweeps those, so that
     // the results are the direct sums' whatever the route.
-    const bool screen_room = te && te->prep && w->slices == 1 && a->num_freqs >= kIpMinFreqs &&
-                             a->num_freqs < kIpMaxFreqs && (double)n * (double)a->num_freqs >= kIpMinTermsScreen;
-    w->screen = screen_room && a->pgram == nullptr && a->top_k > 0;
+    const bool screen_room = te && te->prep && w->slices == 1 && nf >= kIpMinFreqs && nf < kIpMaxFreqs &&
+                             (double)n * (double)nf >= kIpMinTermsScreen;
+    w->screen = screen_room && route->pgram == nullptr && route->top_k > 0;
     w->interp = w->screen || (room && a->dtype == LSAMD_F32 && a->pgram != nullptr);
     if (room || screen_room) {
         w->obj_ip = take(sizeof(InterpObj) * K);
@@ -746,7 +747,7 @@ double lsamd_last_sweep_kernel_ms(void) {
 // device array of lsamd_sweep_static (no kernel timing, which would create
 // events).
 static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspace_bytes, void *stream_v,
-                      bool from_scratch) {
+                      bool from_scratch, const lsamd_sweep_args *route = nullptr) {
     if (!a) return set_error(LSAMD_ERR_INVALID, "lsamd_sweep: null args");
     if (a->variant != LSAMD_STANDARD && a->variant != LSAMD_GENERALIZED)
         return set_error(LSAMD_ERR_INVALID, "lsamd_sweep: bad variant");
@@ -776,7 +777,7 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
         return set_error(LSAMD_ERR_INVALID, "lsamd_sweep: tile shape " + std::to_string(a->tile_threads) +
                                                 "x" + std::to_string(a->tile_fpt) + " not compiled");
     Workspace w;
-    plan_workspace(a, &w);
+    plan_workspace(a, &w, route);
     if (from_scratch && w.bytes > workspace_bytes)
         return set_error(LSAMD_ERR_INVALID, "lsamd_sweep_static: these arguments need " +
                                                 std::to_string(w.bytes) + " bytes of workspace, more than the " +
@@ -1140,7 +1141,9 @@ void lsamd_graph_destroy(lsamd_graph *g) {
     delete g;
 }
 
-// The autotuner's trial sweeps: every object, at most 65536 bins, peaks only.
+// The autotuner's trial sweeps: every object, at most 65536 bins, peaks only, the
+// sums formed the way the whole call forms them.  The coarse-grid sums of FP32
+// periodograms need a periodogram: one of the trial's bins behind the workspace.
 static lsamd_sweep_args autotune_sample(const lsamd_sweep_args *a) {
     lsamd_sweep_args s = *a;
     s.num_freqs = std::min<uint32_t>(a->num_freqs, 65536u);
@@ -1151,6 +1154,19 @@ static lsamd_sweep_args autotune_sample(const lsamd_sweep_args *a) {
     s.peak_power = nullptr;
     s.peak_period = nullptr;
     return s;
+}
+
+// Workspace of a trial, its periodogram (from *pgram_at on) included where it has one.
+static size_t autotune_bytes(const lsamd_sweep_args &s, const lsamd_sweep_args *a, size_t *pgram_at = nullptr) {
+    Workspace whole, w;
+    lsamd_sweep_args c = *a;
+    c.tile_threads = s.tile_threads;
+    c.tile_fpt = s.tile_fpt;
+    plan_workspace(&c, &whole);
+    plan_workspace(&s, &w, a);
+    const bool pgram = whole.interp && !whole.screen;
+    if (pgram_at) *pgram_at = pgram ? align_up(w.bytes) : 0;
+    return pgram ? align_up(w.bytes) + (size_t)4 * s.num_objects * s.num_freqs : w.bytes;
 }
 
 size_t lsamd_autotune_workspace_size(const lsamd_sweep_args *a) {
@@ -1164,9 +1180,7 @@ size_t lsamd_autotune_workspace_size(const lsamd_sweep_args *a) {
         if (te.form != a->form || te.variant != a->variant || te.dtype != a->dtype) continue;
         s.tile_threads = te.T;
         s.tile_fpt = te.M;
-        Workspace w;
-        plan_workspace(&s, &w);
-        need = std::max(need, w.bytes);
+        need = std::max(need, autotune_bytes(s, a));
     }
     return need;
 }
@@ -1210,12 +1224,16 @@ int lsamd_autotune(const lsamd_sweep_args *a, void *workspace, size_t workspace_
         s.tile_threads = te.T;
         s.tile_fpt = te.M;
         Workspace w;
-        plan_workspace(&s, &w);
+        plan_workspace(&s, &w, a);
         if (w.bytes > workspace_bytes) continue;
-        int rc = lsamd_sweep(&s, workspace, workspace_bytes, stream_v);  // warm-up
+        size_t pgram_at = 0;  // without room for it, the direct sums stand in
+        const bool fits = autotune_bytes(s, a, &pgram_at) <= workspace_bytes;
+        s.pgram = fits && pgram_at ? static_cast<char *>(workspace) + pgram_at : nullptr;
+        const size_t room = s.pgram ? pgram_at : workspace_bytes;
+        int rc = sweep_into(&s, workspace, room, stream_v, false, a);  // warm-up
         if (rc) return rc;
         LS_HIP(hipEventRecord(ev.ev[0], st));
-        rc = lsamd_sweep(&s, workspace, workspace_bytes, stream_v);
+        rc = sweep_into(&s, workspace, room, stream_v, false, a);
         if (rc) return rc;
         LS_HIP(hipEventRecord(ev.ev[1], st));
         LS_HIP(hipEventSynchronize(ev.ev[1]));

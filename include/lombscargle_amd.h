@@ -190,7 +190,8 @@ int lsamd_graph_launch(lsamd_graph *graph, void *stream);
 void lsamd_graph_destroy(lsamd_graph *graph);
 
 /* Time every compiled tile shape of args->form/variant/dtype on these
- * arguments (reduced to at most 65536 frequency bins, peaks only) and report
+ * arguments (reduced to at most 65536 frequency bins, peaks only, the sums
+ * formed on the coarse grid or directly as the whole call does) and report
  * the fastest; the caller puts it into args->tile_threads / tile_fpt.  For
  * generalized split32 only the matrix-core tile is a candidate (the VALU
  * tiles reach 1.07e-5 relative on ill-sampled batches, above the form's
