@@ -3,15 +3,19 @@
 //
 // A mode has a coarse step of h bins and result rows of m coarse steps (h m
 // <= 32 bins, one lane each).  Two uses:
-//   sums   (FP32 periodograms) W = 8 taps at an oversampling of at least
-//     kIpSigma = 1.95 keep the aliasing at 2e-8 and leave the rounding, which
-//     at 1.95 is no larger than the direct sums': emulated over light curves
-//     of 30 to 700 observations, worst power 7.3e-6 (bins of at least 1e-3 of
-//     the peak) against 7.7e-6; W = 7 reaches 1.5e-5, an oversampling of 1.45
-//     with W = 10 2.5e-5 (the observations at the ends of the span carry
-//     weights 1/Phi of 18 there, 2.9 at 1.95).  The generalized power, from
-//     four interpolated sums, needs 2.4 (measured on 200 objects, h = 5 / 4:
-//     1.1e-5 / 8.0e-6, direct 7.6e-6).
+//   sums   (FP32 periodograms) W = 8 taps, the window for an oversampling of
+//     2.25, used from kIpSigma = 2.32 on: aliasing of at most 6e-8 of an
+//     observation (those at the ends of the span), 2e-8 in the mean, so that
+//     the rounding is what is left.  Error against 64 bits, coarse over direct
+//     sums, rms over bins of at least 1e-3 of the peak, at 2.32 to 3: 33 to 50
+//     observations 0.99 to 1.05, 64 0.97 to 1.00, 100 to 500 0.77 to 0.96,
+//     2,000 to 65,000 0.82 to 1.00 (worst bins alike, 8.1e-6).  Used at its own
+//     oversampling a window aliases ten times more: the one for 1.95, at
+//     1.95 (7.6e-7 at the ends), had 1.5 to 1.7 at 100 observations, 2.5 to 3.4
+//     at 30.  The generalized power, from four interpolated sums, takes 2.4: 33
+//     to 50 observations 0.98 to 1.05, 64 to 8,000 0.77 to 0.99; its direct sums
+//     fold y's in FP64, the coarse ones in FP32, which shows from there: 12,000
+//     1.06, 65,000 1.26.
 //   screen (peaks without a periodogram) FP16 heads alone, W = 6 taps at an
 //     oversampling of at least 1.3: aliasing 1.2e-4, powers near the peak
 //     good to ~1e-3, which only decide which chunks the direct tile sweeps.
@@ -24,7 +28,7 @@ namespace lsamd {
 namespace {
 
 constexpr int kIpModes = 7;           // h = 3 in the screen only
-constexpr double kIpSigma = 1.95, kIpSigmaGen = 2.4, kIpSigmaScreen = 1.3;
+constexpr double kIpSigma = 2.32, kIpSigmaGen = 2.4, kIpSigmaScreen = 1.3, kIpSigmaWindow = 2.25;
 __host__ __device__ constexpr int ip_frags(bool screen) { return screen ? 4 : 8; }  // column-factor fragments per 16 observations
 // Relative margin of the marked chunks below the top_k-th best power: ten
 // times the sums' error bound; the screen's: see k_sweep_interp.
@@ -59,9 +63,9 @@ constexpr bool ip_reads_fit() {
 }
 static_assert(ip_reads_fit(), "operand reads stay within the points");
 __host__ __device__ constexpr double ip_beta(bool screen) {
-    return 3.14159265358979323846 * ip_taps(screen) * (1.0 - 1.0 / (2.0 * (screen ? kIpSigmaScreen : kIpSigma)));
+    return 3.14159265358979323846 * ip_taps(screen) * (1.0 - 1.0 / (2.0 * (screen ? kIpSigmaScreen : kIpSigmaWindow)));
 }
-// Largest 1/Phi at the ends of the span (ip_inv_window), rounded up: 2.95 and 9.94.
+// Largest 1/Phi at the ends of the span (ip_inv_window), rounded up: 2.08 and 9.94.
 __host__ __device__ constexpr double ip_window_most(bool screen) { return screen ? 10.0 : 3.0; }
 // The points' scale is 2^ip_point_shift / 2^bits, n < 2^bits: with the factors'
 // 2^10 and n observations in phase, at most 1 each, they end below FP16's 65504.
@@ -74,12 +78,13 @@ constexpr uint32_t kIpGroup = 4;  // consecutive items of an object per workgrou
 // The generalized sums' workgroups take one (the loop costs them 4%).
 __host__ __device__ constexpr bool ip_grouped(bool screen, bool gen) { return screen || !gen; }
 // Objects up to here keep the direct sums, those of at most 16 observations
-// their FP64 ones: with 18 observations and weights over a factor of 400 the
-// worst bin reached 1.4e-5 (direct 1.0e-5).  Peaks alone, generalized: with
+// their FP64 ones: with 18
+// observations and weights over a factor of 400 the worst bin reached 1.4e-5
+// (direct 1.0e-5).  Peaks alone, generalized: with
 // few observations most chunks hold bins that either sweep computes again in
 // FP64, or powers near 1 (400 objects x 400,000 bins, direct / coarse, us: 20
 // observations 8420 / 13400, 30 2295 / 2517, 35 2004 / 930, 50 1939 / 405).
-constexpr uint32_t kIpLeastObs = 24, kIpLeastObsScreen = 16, kIpLeastObsScreenGen = 32;
+constexpr uint32_t kIpLeastObs = 32, kIpLeastObsScreen = 16, kIpLeastObsScreenGen = 32;
 // The screen computes a tile's ill-conditioned bins again when no more lanes
 // than this have one (1, 4, 16 lanes: 1394, 1227, 937 us at 35 observations,
 // 2485, 2517, 2654 at 30).
