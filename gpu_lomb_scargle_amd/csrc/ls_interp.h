@@ -77,14 +77,14 @@ constexpr uint32_t kIpLeastBins = 255 * 32, kIpLeastBinsScreen = 192 * 30;  // b
 constexpr uint32_t kIpGroup = 4;  // consecutive items of an object per workgroup, at most
 // The generalized sums' workgroups take one (the loop costs them 4%).
 __host__ __device__ constexpr bool ip_grouped(bool screen, bool gen) { return screen || !gen; }
-// Objects up to here keep the direct sums, those of at most 16 observations
-// their FP64 ones: with 18
+// Objects up to here (generalized ones also from kIpMostObsGen on) keep the
+// direct sums, those of at most 16 observations their FP64 ones: with 18
 // observations and weights over a factor of 400 the worst bin reached 1.4e-5
 // (direct 1.0e-5).  Peaks alone, generalized: with
 // few observations most chunks hold bins that either sweep computes again in
 // FP64, or powers near 1 (400 objects x 400,000 bins, direct / coarse, us: 20
 // observations 8420 / 13400, 30 2295 / 2517, 35 2004 / 930, 50 1939 / 405).
-constexpr uint32_t kIpLeastObs = 32, kIpLeastObsScreen = 16, kIpLeastObsScreenGen = 32;
+constexpr uint32_t kIpLeastObs = 32, kIpLeastObsScreen = 16, kIpLeastObsScreenGen = 32, kIpMostObsGen = 8192;
 // The screen computes a tile's ill-conditioned bins again when no more lanes
 // than this have one (1, 4, 16 lanes: 1394, 1227, 937 us at 35 observations,
 // 2485, 2517, 2654 at 30).

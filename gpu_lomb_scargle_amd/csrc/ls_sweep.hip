@@ -70,7 +70,8 @@ struct StatsArgs {
     InterpObj *obj_ip;
     double df_rev;
     double sigma;        // least oversampling of the coarse grid, observations an object needs
-    uint32_t least_obs;  // more than, and the first mode
+    uint32_t least_obs;  // more than, the most it may have, and the first mode
+    uint64_t most_obs;
     int first_mode, screen;
 };
 
@@ -319,7 +320,7 @@ __global__ __launch_bounds__(T) void k_obj_stats_split(StatsArgs a) {
         lo = -most(-lo);
         hi = most(hi);
         const double cycles = (hi - lo) * a.df_rev * a.sigma;
-        if (n > a.least_obs && cycles > 0.0)
+        if (n > a.least_obs && n <= a.most_obs && cycles > 0.0)
             for (int q = a.first_mode; q <= kIpModes; ++q)
                 if (cycles * (double)ip_step(q) <= 1.0) mode = (uint32_t)q;
         tc = 0.5 * (lo + hi);
@@ -813,7 +814,8 @@ static int sweep_into(const lsamd_sweep_args *a, void *workspace, size_t workspa
                  mfma ? reinterpret_cast<double2 *>(ws + w.rec_r) : nullptr,
                  mfma ? reinterpret_cast<uint32_t *>(ws + w.slot_obj) : nullptr, obj_ip, dw * kInv2Pi,
                  w.screen ? kIpSigmaScreen : gen ? kIpSigmaGen : kIpSigma,
-                 w.screen ? (gen ? kIpLeastObsScreenGen : kIpLeastObsScreen) : kIpLeastObs, w.screen ? 1 : 2, w.screen ? 1 : 0};
+                 w.screen ? (gen ? kIpLeastObsScreenGen : kIpLeastObsScreen) : kIpLeastObs,
+                 gen && !w.screen ? kIpMostObsGen : ~0ull, w.screen ? 1 : 2, w.screen ? 1 : 0};
     if (split) {
         const bool wide = w.slices > 1;  // one long object alone
         void (*fn)(StatsArgs) = wide ? (f64 ? k_obj_stats_split<double, 512> : k_obj_stats_split<float, 512>)

@@ -54,3 +54,17 @@ def test_error_against_the_direct_sums(sigma, h, n, gen):
     e = [torch.sqrt((((p - ref) / ref)[big] ** 2).mean()).item() for p in (coarse, direct)]
     print(f"coarse {e[0]:.2e} direct {e[1]:.2e}")
     assert e[0] <= 1.2 * e[1]
+
+
+@pytest.mark.parametrize("n,coarse", [(8192, True), (8193, False)])
+def test_generalized_objects_of_many_observations_keep_the_direct_sums(n, coarse):
+    """Their y sums are folded in FP64 there.  Five objects are under the terms of
+    the coarse grid, 24 are above."""
+    torch = pytest.importorskip("torch")
+    from gpu_lomb_scargle_amd import device
+    o, t, y, dy = _curves(n, 2.5 * 4, True, n)
+    kw = dict(min_freq=synth.OMEGA_MIN, max_freq=synth.OMEGA_MIN + (synth.OMEGA_MAX - synth.OMEGA_MIN) * 20001 / NF,
+              num_freqs=20001, form=_native.FORM_SPLIT32, variant=_native.GENERALIZED, top_k=1)
+    whole = device.sweep(*device.numpy_to_device(o, t, y, dy, F32), **kw)["pgram"]
+    few = device.sweep(*device.numpy_to_device(o[:5 * n], t[:5 * n], y[:5 * n], dy[:5 * n], F32), **kw)["pgram"]
+    assert torch.equal(whole[:5], few) == (not coarse)
