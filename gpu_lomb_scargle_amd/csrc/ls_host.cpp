@@ -24,8 +24,6 @@
 
 #include <hip/hip_runtime.h>
 
-#include <sys/mman.h>
-
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
@@ -465,14 +463,6 @@ int lsamd_batch_host(int variant, int dtype, int form, int normalize, int precen
     if (!rc) rc = upload(in_order, order.data(), (size_t)K * 4);
     if (rc) return rc;
     if (packed) HIP_OK(hipMemcpyAsync(in, c.io, in_bytes, hipMemcpyHostToDevice, c.stream));
-
-    // Fresh memory is touched for the first time by the copy-back: with pages of
-    // 2 MiB where the system has them.
-    if (pgram && (size_t)K * per_obj >= (size_t(8) << 20)) {
-        const uintptr_t page = (uintptr_t)2 << 20, p0 = reinterpret_cast<uintptr_t>(pgram);
-        const uintptr_t lo = (p0 + page - 1) & ~(page - 1), hi = (p0 + (size_t)K * per_obj) & ~(page - 1);
-        if (hi > lo) (void)madvise(reinterpret_cast<void *>(lo), hi - lo, MADV_HUGEPAGE);
-    }
 
     // outputs: the peaks, and behind them the periodogram of a small call, in one
     // run of pinned memory; a larger periodogram in the ring or a device buffer
