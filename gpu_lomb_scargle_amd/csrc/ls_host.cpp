@@ -120,12 +120,10 @@ struct Ctx {
     DevBuf in, ws, pgram, peaks;
     char *io = nullptr;                 // pinned: packed inputs, then small outputs
     bool busy = false;                  // a call is enqueued (or failed half-way)
-    void *pinned[2] = {nullptr, nullptr};
+    char *pinned = nullptr;             // staging buffers, or the slices under way (ring)
     size_t pinned_cap = 0;
     hipEvent_t ev[2] = {nullptr, nullptr};     // staging chunks (copy stream)
     hipEvent_t slice[kAhead] = {};             // sweep of a slice done (sweep stream)
-    char *ring[kAhead] = {};                   // pinned: periodograms of the slices under way
-    size_t ring_cap = 0;                       // bytes of each
 };
 
 // One context per device, for the device current on the calling thread.
@@ -196,6 +194,18 @@ int ensure(DevBuf &b, size_t bytes) {
 
 constexpr size_t kPinnedChunk = size_t(64) << 20;  // a staging buffer, at most
 
+// Pinned memory of a context: two staging buffers or kAhead slices, never both in
+// one call (128 MiB at most either way, kept for the next call).
+int ensure_pinned(Ctx &c, size_t bytes) {
+    if (c.pinned_cap >= bytes) return LSAMD_OK;
+    c.pinned_cap = 0;
+    if (c.pinned) HIP_OK(hipHostFree(c.pinned));
+    c.pinned = nullptr;
+    HIP_OK(hipHostMalloc(reinterpret_cast<void **>(&c.pinned), bytes, hipHostMallocCoherent));
+    c.pinned_cap = bytes;
+    return LSAMD_OK;
+}
+
 // Pinned to pageable memory: first touches of fresh pages dominate, which
 // threads share.
 void host_copy(char *to, const char *from, size_t len) {
@@ -217,29 +227,23 @@ void host_copy(char *to, const char *from, size_t len) {
 int copy_to_host(Ctx &c, void *dst, const void *src, size_t bytes) {
     if (bytes == 0) return LSAMD_OK;
     const size_t chunk = std::min(kPinnedChunk, std::max(size_t(2) << 20, (bytes / 4 + 4095) & ~size_t(4095)));
-    if (c.pinned_cap < chunk) {
-        c.pinned_cap = 0;
-        for (int i = 0; i < 2; ++i) {
-            if (c.pinned[i]) HIP_OK(hipHostFree(c.pinned[i]));
-            c.pinned[i] = nullptr;
-            HIP_OK(hipHostMalloc(&c.pinned[i], chunk, hipHostMallocDefault));
-        }
-        c.pinned_cap = chunk;
-    }
+    const int rc = ensure_pinned(c, 2 * chunk);
+    if (rc) return rc;
+    char *const stage[2] = {c.pinned, c.pinned + chunk};
     const size_t nch = (bytes + chunk - 1) / chunk;
     auto chunk_len = [&](size_t i) { return std::min(chunk, bytes - i * chunk); };
     const char *s = static_cast<const char *>(src);
     char *d = static_cast<char *>(dst);
-    HIP_OK(hipMemcpyAsync(c.pinned[0], s, chunk_len(0), hipMemcpyDeviceToHost, c.copy_stream));
+    HIP_OK(hipMemcpyAsync(stage[0], s, chunk_len(0), hipMemcpyDeviceToHost, c.copy_stream));
     HIP_OK(hipEventRecord(c.ev[0], c.copy_stream));
     for (size_t i = 1; i <= nch; ++i) {
         if (i < nch) {
-            HIP_OK(hipMemcpyAsync(c.pinned[i & 1], s + i * chunk, chunk_len(i), hipMemcpyDeviceToHost,
+            HIP_OK(hipMemcpyAsync(stage[i & 1], s + i * chunk, chunk_len(i), hipMemcpyDeviceToHost,
                                   c.copy_stream));
             HIP_OK(hipEventRecord(c.ev[i & 1], c.copy_stream));
         }
         HIP_OK(hipEventSynchronize(c.ev[(i - 1) & 1]));
-        host_copy(d + (i - 1) * chunk, static_cast<const char *>(c.pinned[(i - 1) & 1]), chunk_len(i - 1));
+        host_copy(d + (i - 1) * chunk, stage[(i - 1) & 1], chunk_len(i - 1));
     }
     return LSAMD_OK;
 }
@@ -279,18 +283,6 @@ uint64_t row_argmax(const R *x, uint64_t n) {
         }
     }
     return at;
-}
-
-int ensure_ring(Ctx &c, size_t bytes) {
-    if (c.ring_cap >= bytes) return LSAMD_OK;
-    c.ring_cap = 0;
-    for (char *&r : c.ring) {
-        if (r) HIP_OK(hipHostFree(r));
-        r = nullptr;
-        HIP_OK(hipHostMalloc(reinterpret_cast<void **>(&r), bytes, hipHostMallocCoherent));
-    }
-    c.ring_cap = bytes;
-    return LSAMD_OK;
 }
 
 double env_double(const char *name, double dflt) {
@@ -476,7 +468,9 @@ int lsamd_batch_host(int variant, int dtype, int form, int normalize, int precen
     const bool peaks_pinned = peak_bytes <= kIoOut;
     char *const io_out = c.io + kIoIn;
     if (!peaks_pinned) rc = ensure(c.peaks, peak_bytes);
-    if (!rc && ring) rc = ensure_ring(c, (size_t)objs_per_slice * per_obj);
+    // (slices of the ring start on page boundaries)
+    const size_t ring_step = ((size_t)objs_per_slice * per_obj + 4095) & ~size_t(4095);
+    if (!rc && ring) rc = ensure_pinned(c, kAhead * ring_step);
     if (!rc && pgram && !ring && !small) rc = ensure(c.pgram, (size_t)objs_per_batch * per_obj);
     if (rc) return rc;
     char *const peaks = peaks_pinned ? io_out : static_cast<char *>(c.peaks.p);
@@ -510,7 +504,7 @@ int lsamd_batch_host(int variant, int dtype, int form, int normalize, int precen
         a.dy = variant == LSAMD_GENERALIZED ? in + in_dy : nullptr;
         a.pgram = !pgram  ? nullptr
                   : small ? io_out + out_pg
-                  : ring  ? c.ring[i % kAhead]
+                  : ring  ? c.pinned + i % kAhead * ring_step
                           : static_cast<char *>(c.pgram.p) + batch_row(s0) * per_obj;
         // a call of one object may slice its observations; sub-sweeps of a
         // larger call never do, so batching cannot change any result
@@ -539,7 +533,7 @@ int lsamd_batch_host(int variant, int dtype, int form, int normalize, int precen
         const size_t bytes = (size_t)(s1 - s0) * per_obj;
         if (ring) {
             HIP_OK(hipEventSynchronize(c.slice[i % kAhead]));
-            host_copy(to, c.ring[i % kAhead], bytes);
+            host_copy(to, c.pinned + i % kAhead * ring_step, bytes);
             return LSAMD_OK;
         }
         HIP_OK(hipStreamWaitEvent(c.copy_stream, c.slice[i % kAhead], 0));
