@@ -219,7 +219,7 @@ def lombscarglemain(objId, timeX, magY, minFreq, maxFreq, error, mode, magDY=Non
                                             uniqueObjects, freqToTest, best.ctypes.data))
     ret_periods = np.zeros(uniqueObjects)
     for x in range(uniqueObjects):
-        ret_periods[x] = 1.0 / (minFreqStandard + (dfstandard * int(best[x])))
+        ret_periods[x] = 1.0 / (minFreqStandard + (dfstandard * np.int64(best[x])))
 
     if uniqueObjects > 1:
         print("[Python] Sum of all periods: %f" % np.sum(ret_periods))
