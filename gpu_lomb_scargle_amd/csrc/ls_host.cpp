@@ -407,9 +407,8 @@ int lsamd_batch_host(int variant, int dtype, int form, int normalize, int precen
     // (at least 1 object; LSAMD_SLICE_BYTES overrides): each slice's copy through
     // the staging buffers restarts their pipeline.
     const size_t eighth = std::min(kRingSlice, std::max(size_t(8) << 20, (size_t)K * per_obj / 8));
-    const size_t most = ring_call ? kRingSlice : size_t(2) << 30;
-    const size_t kSliceBytes =
-        std::min(most, (size_t)env_double("LSAMD_SLICE_BYTES", ring_call ? (double)eighth : (double)most));
+    size_t kSliceBytes = (size_t)env_double("LSAMD_SLICE_BYTES", ring_call ? (double)eighth : (double)(size_t(2) << 30));
+    if (ring_call) kSliceBytes = std::min(kRingSlice, kSliceBytes);
     const uint32_t objs_per_slice =
         per_obj > 0 ? (uint32_t)std::max<size_t>(1, std::min<size_t>(objs_per_batch, kSliceBytes / per_obj))
                     : objs_per_batch;
