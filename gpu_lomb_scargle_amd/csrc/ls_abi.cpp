@@ -137,7 +137,15 @@ extern "C" void LombScarglePy(unsigned int *objectId, real_t *timeX, real_t *mag
     if (env_flag("LSAMD_GPU_STATS", true)) {
         if (FILE *f = std::fopen("gpu_stats.txt", "a")) {
             int T = 0, M = 0;
-            lsamd_get_tile(form, kVariant, kDtype, &T, &M);
+            lsamd_sweep_args a{};
+            a.variant = kVariant;
+            a.dtype = kDtype;
+            a.form = form;
+            a.num_objects = MODE == 1 ? lsamd_count_objects(objectId, sizeData) : 1u;
+            a.num_freqs = freqToTest;
+            a.obs_slices = a.num_objects == 1 ? 0 : 1;  // as lsamd_batch_host has it
+            if (gpu) lsamd_sweep_tile(&a, &T, &M);
+            else lsamd_get_tile(form, kVariant, kDtype, &T, &M);
             std::fprintf(f,
                          "%g, Sum of periods: %g, Min/Max Freq: %g/%g,  Num tested freq: %u, MODE: %d, "
                          "ERROR/DTYPE/FORM/TILE: %d, %s, %s, %dx%d\n",

@@ -125,3 +125,14 @@ def test_a_named_tile_runs_its_kernel():
     o, t, y = _curves([90] * 20)
     a, b = (_sweep(o, t, y, 1.0, 60.0, 40013, tile=tile)[0] for tile in ((256, 1), (256, 2)))
     assert np.array_equal(a["pgram"], b["pgram"])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K,nf,tile", [(1, 100003, "256x1"), (1, 200003, "256x8"), (3, 5003, "256x1"), (3, 20011, "256x8")])
+def test_the_stats_record_names_the_tile(K, nf, tile, tmp_path, monkeypatch):
+    from gpu_lomb_scargle_amd import lombscarglegpu as ls
+    monkeypatch.chdir(tmp_path)
+    monkeypatch.setenv("LSAMD_GPU_STATS", "1")
+    o, t, y = _curves([40] * K)
+    ls.lombscargle(o, t, y, 0.1, 10.0, False, "GPU", None, nf, "double")
+    assert (tmp_path / "gpu_stats.txt").read_text().strip().endswith(tile)
