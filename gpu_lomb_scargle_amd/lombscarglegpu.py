@@ -214,12 +214,11 @@ def lombscarglemain(objId, timeX, magY, minFreq, maxFreq, error, mode, magDY=Non
         raise RuntimeError("LombScarglePy failed (%d): %s" % (rc, lib.lsamd_last_error().decode()))
 
     ret_pgram = ret_pgram.reshape([uniqueObjects, freqToTest])
-    best = np.zeros(uniqueObjects, dtype=np.uint64)
+    best = np.zeros(uniqueObjects, dtype=np.int64)
     _native.check(lib, lib.lsamd_row_argmax(_native.F32 if dtype == "float" else _native.F64, ret_pgram.ctypes.data,
                                             uniqueObjects, freqToTest, best.ctypes.data))
     ret_periods = np.zeros(uniqueObjects)
-    for x in range(uniqueObjects):
-        ret_periods[x] = 1.0 / (minFreqStandard + (dfstandard * np.int64(best[x])))
+    ret_periods[:] = 1.0 / (minFreqStandard + (dfstandard * best))
 
     if uniqueObjects > 1:
         print("[Python] Sum of all periods: %f" % np.sum(ret_periods))

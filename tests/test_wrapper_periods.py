@@ -19,3 +19,13 @@ def test_periods_are_formed_from_numpy_s_argmax(kind, nf):
     df = (hi - lo) / nf * 1.0
     want = [1.0 / (lo + (df * np.argmax(row))) for row in pgram]
     assert np.array_equal(periods, want)
+
+
+def test_a_peak_at_frequency_zero_has_an_infinite_period():
+    """0/0 at frequency 0 is numpy's argmax; the period is inf, with numpy's
+    warning, as the loop over numpy scalars had it."""
+    rng = np.random.default_rng(4)
+    t = np.sort(rng.uniform(0, 200, 60))
+    with pytest.warns(RuntimeWarning, match="divide by zero"):
+        _, periods, pgram = ls.lombscargle(np.zeros(60, int), t, np.sin(2.0 * t), 0.0, 3.0, False, "CPU", None, 2003, "double")
+    assert np.isnan(pgram[0, 0]) and np.isinf(periods[0])
