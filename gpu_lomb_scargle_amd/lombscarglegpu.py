@@ -217,8 +217,7 @@ def lombscarglemain(objId, timeX, magY, minFreq, maxFreq, error, mode, magDY=Non
     best = np.zeros(uniqueObjects, dtype=np.int64)
     _native.check(lib, lib.lsamd_row_argmax(_native.F32 if dtype == "float" else _native.F64, ret_pgram.ctypes.data,
                                             uniqueObjects, freqToTest, best.ctypes.data))
-    ret_periods = np.zeros(uniqueObjects)
-    ret_periods[:] = 1.0 / (minFreqStandard + (dfstandard * best))
+    ret_periods = np.asarray(1.0 / (minFreqStandard + (dfstandard * best)), dtype=np.float64)
 
     if uniqueObjects > 1:
         print("[Python] Sum of all periods: %f" % np.sum(ret_periods))
