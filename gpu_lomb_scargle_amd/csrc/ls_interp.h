@@ -95,7 +95,7 @@ constexpr int kIpScreenIll = 16;
 // 131 / 130; 100 x 200,000, 3.4e9: 252 / 177 and 440 / 235; 4 x 500,000, 0.3e9:
 // 56 / 75.  A call that may not look at how many objects it sweeps takes the
 // coarse grid from 2^18 bins on, where a few objects lose ~25 us by it.
-constexpr uint32_t kIpMinFreqs = 8192;  // bins a workgroup takes, smallest mode
+constexpr uint32_t kIpMinFreqs = 8192;  // about the bins that a workgroup takes (5760 screen, 8160 sums, or more)
 constexpr double kIpMinTerms = 1.5e9;
 // Peaks alone (FP64, top-3, direct / coarse): 10 objects x 300,000 bins, 0.5e9
 // terms, 82 / 76 standard and 127 / 110 generalized; 40 x 100,000, 0.7e9: 87 / 99

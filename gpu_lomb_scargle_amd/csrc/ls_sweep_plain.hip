@@ -136,7 +136,10 @@ __global__ __launch_bounds__(T) void k_sweep_plain_std(SweepArgs a) {
 // calls that would leave SIMDs idle.  Against the CPU path over the test light
 // curves (14 to 3555 observations) 2.3e-13 on bins of at least 1e-6 of the
 // peak, with a stride of 256 bins instead of 64 1.1e-11 at the lowest bins
-// (the differences are not exact there).
+// (the differences are not exact there).  Against powers of the exact phases in
+// 80 bits (40 to 3555 observations, times from 0, 51,075 and 2,458,652 days) the
+// errors are those of a sine and cosine per bin to three digits, 1e-11 to 3e-8:
+// the roundings of the phases, which both have.
 // The sums above serve, bin by bin, what this does not: bins whose 2x2 system
 // amplifies the phasors' error (condition number above kStepCond), frequencies
 // below the step (or of both signs in a thread), phases past kStepFar, objects of fewer than

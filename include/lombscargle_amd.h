@@ -68,7 +68,11 @@ enum lsamd_dtype { LSAMD_F32 = 0, LSAMD_F64 = 1 };
 enum lsamd_form {
     /* the reference's arithmetic: DTYPE phases omega*t, libm-accurate
      * sin/cos, sequential DTYPE sums, tau form; matches the reference CPU
-     * path of the same DTYPE */
+     * path of the same DTYPE.  FP64 standard sweeps of long grids (see
+     * obs_slices) and the second pass of FP64 generalized ones form the sine
+     * and cosine of those same phases from a neighbouring bin's and add with
+     * FMAs (generalized: four partial sums per bin): within 2.3e-13 of that
+     * path on bins of at least 1e-6 of the peak */
     LSAMD_FORM_PLAIN = 0,
     /* FP64 phase reduction, FP32 hardware sin/cos seeds with an FP64
      * residual correction and a unit-modulus Newton step, FP64 rotation and
@@ -87,7 +91,10 @@ enum lsamd_form {
      * at most 16 observations are computed in FP64.  Matrix-core tiles:
      * within 1e-5 of FP64 on every batch measured (7.9e-6 on a 1000-object
      * standard batch, 8.4e-6 generalized); the VALU generalized tiles reach
-     * 1.07e-5 on the generalized batch */
+     * 1.07e-5 on the generalized batch.  FP32 periodograms of grids finer
+     * than an object's resolution have these sums on a coarser grid and are
+     * interpolated, and peaks without a periodogram are looked for that way
+     * first and then computed directly */
     LSAMD_FORM_SPLIT32 = 2
 };
 enum lsamd_schedule {
